@@ -1,7 +1,11 @@
 import os
 import sys
 
-import pytest
+# The golden outputs are fp32 sums in the order of OpenBLAS's AVX2 kernels; the AVX-512 kernels that it picks on newer
+# CPUs add in another order (up to 2.4e-6 apart, the test allows 1e-6).  Read when numpy is loaded.
+os.environ.setdefault("OPENBLAS_CORETYPE", "Haswell")
+
+import pytest  # noqa: E402
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 if ROOT not in sys.path:
