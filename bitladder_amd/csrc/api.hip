@@ -80,21 +80,51 @@ int query_cus() {
     return n;
 }
 
-// A wave streams whole packed units (64 tokens at 4 bits, 128 at 2 bits) plus a share of the 16-token
-// fp16 tiles, and a workgroup has 16 or 12 waves.  Pick the number of splits so that the grid is about
-// one workgroup per CU (a second round of workgroups costs far more than idle waves) while a
-// workgroup still gets at least one unit for every second wave (or four fp16 tiles per unit when
-// nothing is packed); measured optimum over 4K-128K tokens, 1-128 (batch, kv-head) pairs.
+// Number of workgroups ("splits") a (batch, kv-head) pair is cut into.
+//
+// By the machine: a launch is as long as its busiest compute unit, and a unit that gets a second workgroup takes
+// twice as long as its neighbours.  So the grid holds at most one workgroup per unit: the largest n with n * pairs
+// <= units.  One split more (n rounded up instead of down: a grid of 264 for 24 pairs, 288 for 48) measured, us at
+// 8K tokens, 4 bits g128 | 2 bits g128 | 4 bits g32:
+//   24 pairs, 11 and 10 splits: 10.6 and 10.0 | 9.3 (10 splits) | 15.4 and 12.1      48 pairs (10K), 6 and 5: 19.4 and 16.5 | 21.7 and 12.7 | 29.5 and 19.3
+//   80 pairs,  4 and  3 splits: 22.8 and 18.6 | 23.1 and 15.6 | 34.4 and 23.7        160 pairs (4K), 2 and 1: 24.0 and 23.7 | 23.4 and 18.0 | 34.9 and 30.5
+// With more pairs than half the units, one workgroup each leaves units idle (or, above 256 pairs, most units with
+// one and some with two); two or three splits then even that out at 4 bits, where the waves of several workgroups
+// overlap on a unit, and from 4K tokens on, where the extra merges pay: 136 pairs of 8K tokens 41.3 us with one
+// split, 31.3 with three; 264 pairs of 4K 39.5 and 34.9; 384 pairs 44.1 and 41.0 with two.  At 2 bits (one
+// workgroup of 16 waves per unit) it never paid (136 pairs: 29.2 against 29.9 us).
+//
+// By the work: a workgroup wants a unit for every wave of the 8-wave kernels at 4 bits (a unit for each of 4 waves,
+// one per SIMD, at 2 bits, up to 16 splits: the merging wave takes 16 records per round trip, and a wave's time per unit
+// is bound by its SIMD's vector ALU; one sequence, 8 kv heads: 2K tokens 8.5 us with 2 splits, 8.0 with 4; 8K tokens
+// 8.8 with 8, 8.6 with 16).  Without packed tokens, four fp16 tiles count as a unit.
 int choose_splits(int b, int hk, int max_seqlen_k, int max_res_len, int num_cus, int bits, int gs) {
-    const int nw = bitdecode::decode_waves(bits, gs);
     const int packed_units = max_seqlen_k / bitdecode::unit_tokens(bits);
     const int tiles = (max_res_len + 15) / 16;
     const int units = packed_units > 0 ? packed_units : (tiles + 3) / 4;
     if (units <= 0) return 1;
-    const int heads = std::max(1, b * hk);
-    const int by_occupancy = std::max(1, (num_cus + heads - 1) / heads);
-    const int by_work = std::max(1, (2 * units + nw - 1) / nw);
-    int n = std::min(std::min(by_occupancy, by_work), 256);
+    const int64_t pairs = std::max<int64_t>(1, static_cast<int64_t>(b) * hk);
+    int by_machine = static_cast<int>(std::max<int64_t>(1, num_cus / pairs));
+    if (bits == 4 && 2 * pairs > num_cus && packed_units >= 64) {
+        // share of the machine's time that the busiest unit uses: ceil(n * pairs / units) / n, against pairs / units
+        double best = 0.0;
+        for (int n = 1; n <= 3; ++n) {
+            const int64_t wgs = n * pairs, rounds = (wgs + num_cus - 1) / num_cus;
+            const double fill = static_cast<double>(wgs) / static_cast<double>(rounds * num_cus);
+            if (fill > 1.1 * best) {
+                best = fill;
+                by_machine = n;
+            }
+        }
+    }
+    int by_work;
+    if (bits == 4) {
+        by_work = (units + bitdecode::kFewWaves - 1) / bitdecode::kFewWaves;
+    } else {
+        const int nw = bitdecode::decode_waves(bits, gs);
+        by_work = units <= 8 ? 1 : std::max(std::min((units + 3) / 4, 16), (2 * units + nw - 1) / nw);
+    }
+    int n = std::min(std::min(by_machine, std::max(1, by_work)), 256);
     // drop splits that would be empty: ceil(units / n) units per split
     const int ups = (units + n - 1) / n;
     n = (units + ups - 1) / ups;
@@ -118,14 +148,22 @@ bool use_few_waves(int bits, int gs, int max_s, int max_r, int nsplit, bool devi
 // unequal sequences is better served by twice as many workgroups of half the size: the two that share a unit
 // add up, and the kernel orders the sequences so that the longest shares with the shortest (decode.hip:
 // sequence_of_position).  16 sequences of 1.9K-8K tokens: 62 units on the busiest unit with one workgroup
-// per unit, 49.5 with two.  Only for batches that fill the machine with one or two splits: the host cannot tell a
+// per unit, 49.5 with two.  Only for batches that fill the machine with one to three splits: the host cannot tell a
 // ragged batch from an equal one, and equal sequences lose by the doubling what the extra splits cost
 // (32 x 8 heads: nothing; 16 x 8: 1.5 %; 8 x 8 and 4 x 8, where 4 and 8 splits would become 8 and 16: 9-12 %).
+// Lengths drawn from 1K-8K, 8 kv heads, 4 bits: 9 sequences 16.3 us with 3 splits, 15.4 with 7; 12 sequences 21.7 with
+// 2, 17.4 with 5.  Where the doubling does not apply, sequences that occupy more than half of the units are cut in two:
+// the short ones end early anyway (20 sequences: 35.4 us with one split, 27.7 with two; 2 bits 28.5 and 23.2).
 int choose_splits_for(int b, int hk, int max_s, int max_r, int num_cus, int bits, int gs, bool ragged) {
-    const int n1 = choose_splits(b, hk, max_s, max_r, num_cus, bits, gs);
-    if (!ragged || b < 2 || n1 > 2) return n1;
+    int n1 = choose_splits(b, hk, max_s, max_r, num_cus, bits, gs);
+    if (!ragged || b < 2 || n1 > 3) return n1;
+    const int64_t pairs = static_cast<int64_t>(b) * hk;
+    if (2 * pairs > num_cus) n1 = pairs < num_cus ? std::min(2, choose_splits(1, 1, max_s, max_r, num_cus, bits, gs)) : 1;
+    // (the 8-wave kernel of group size 32 takes 95 KB of LDS: one workgroup per unit, 20.0 us with 3 splits against 23.5
+    // with 7 for 9 sequences)
+    if (gs < 64) return n1;
     const int n2 = choose_splits(b, hk, max_s, max_r, 2 * num_cus, bits, gs);
-    if (n2 > n1 && static_cast<int64_t>(n2) * b * hk <= 2 * num_cus && use_few_waves(bits, gs, max_s, max_r, n2, true))
+    if (n2 > n1 && n2 * pairs <= 2 * num_cus && use_few_waves(bits, gs, max_s, max_r, n2, true))
         return n2;
     return n1;
 }
