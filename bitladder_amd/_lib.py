@@ -58,6 +58,14 @@ class FwdArgs(ctypes.Structure):
     ]
 
 
+class FwdRowsArgs(ctypes.Structure):
+    _fields_ = [
+        ("fwd", FwdArgs),
+        ("rows", _i32),
+        ("q_stride_row", _i64), ("out_stride_row", _i64),
+    ]
+
+
 class FwdAppendArgs(ctypes.Structure):
     _fields_ = [
         ("fwd", FwdArgs),
@@ -71,7 +79,8 @@ class FwdAppendArgs(ctypes.Structure):
 
 EXPORTS = ("bitdecode_abi_version", "bitdecode_last_error", "bitdecode_num_splits",
            "bitdecode_fwd_workspace_bytes", "bitdecode_num_splits_for", "bitdecode_qpack", "bitdecode_fwd",
-           "bitdecode_fwd_append", "bitdecode_fwd_append_workspace_bytes", "bitdecode_fwd_static")
+           "bitdecode_fwd_append", "bitdecode_fwd_append_workspace_bytes", "bitdecode_fwd_static",
+           "bitdecode_fwd_rows")
 
 _lib = None
 
@@ -108,6 +117,8 @@ def lib():
         L.bitdecode_fwd.argtypes = [ctypes.POINTER(FwdArgs), _vp]
         L.bitdecode_fwd_static.restype = ctypes.c_int
         L.bitdecode_fwd_static.argtypes = [ctypes.POINTER(FwdArgs), _vp]
+        L.bitdecode_fwd_rows.restype = ctypes.c_int
+        L.bitdecode_fwd_rows.argtypes = [ctypes.POINTER(FwdRowsArgs), _vp]
         L.bitdecode_fwd_append.restype = ctypes.c_int
         L.bitdecode_fwd_append.argtypes = [ctypes.POINTER(FwdAppendArgs), _vp]
         L.bitdecode_fwd_append_workspace_bytes.restype = ctypes.c_size_t

@@ -285,9 +285,9 @@ size_t bitdecode_fwd_append_workspace_bytes(int32_t b, int32_t h, int32_t num_sp
     return step_ticket_bytes(b) + bitdecode_fwd_workspace_bytes(b, h, num_splits);
 }
 
-// decode, or (step != null) decode step with append
+// decode, or (step != null) decode step with append, or (rows_args != null) decode of several query rows
 static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args* step, void* stream,
-                   unsigned char* static_scratch = nullptr) {
+                   unsigned char* static_scratch = nullptr, const bitdecode_fwd_rows_args* rows_args = nullptr) {
     using namespace bitdecode;
     if (!a) return fail(BITDECODE_EINVAL, "args is null");
     if (int rc = check_quant(a->bits, a->group_size, a->dtype, a->d)) return rc;
@@ -297,6 +297,12 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     const int g = a->h / a->h_k;
     if (g > kMaxGroupHeads)
         return fail(BITDECODE_EUNSUPPORTED, "%d query heads per kv head unsupported (at most %d)", g, kMaxGroupHeads);
+    const int rows = rows_args ? rows_args->rows : 1;
+    if (rows < 1 || rows > 4096) return fail(BITDECODE_EINVAL, "%d query rows per sequence (1 to 4096)", rows);
+    if (rows_args && rows_args->q_stride_row % 8)
+        return fail(BITDECODE_EINVAL, "q and residual strides must be multiples of 8 elements");
+    const int row_blocks = rows > 1 ? (rows * g + kMaxGroupHeads - 1) / kMaxGroupHeads : 1;
+    const int n_h = a->h * rows;        // workspace rows per sequence
     int max_s = a->seqlens_k ? a->max_seqlen_k : a->seqlen_k;
     int max_r = a->res_lens ? a->max_res_len : a->res_len;
     if (step) {
@@ -345,19 +351,19 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     if (nsplit > 512) return fail(BITDECODE_EINVAL, "num_splits %d is above the limit of 512", nsplit);
     const int cus = query_cus();
     if (nsplit == 0)
-        nsplit = choose_splits_for(a->b, a->h_k, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k && !step);
-    if (nsplit > 1 && slots_bytes(a->b, a->h, nsplit) >= (size_t(1) << 31))
-        return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d heads: partial outputs of 2 GiB or more", nsplit, a->b, a->h);
+        nsplit = choose_splits_for(a->b, a->h_k * row_blocks, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k && !step);
+    if (nsplit > 1 && slots_bytes(a->b, n_h, nsplit) >= (size_t(1) << 31))
+        return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d heads: partial outputs of 2 GiB or more", nsplit, a->b, n_h);
     // the kernel divides workgroup ids and unit counts by the split count and the head count with a
     // multiply (kernels.h: division_magic), exact while numerator x divisor stays below 2^32
     {
-        const uint64_t wgs = static_cast<uint64_t>(nsplit) * a->b * a->h_k;
+        const uint64_t wgs = static_cast<uint64_t>(nsplit) * a->b * a->h_k * row_blocks;
         // lengths read on the device are clamped to the capacity by the kernel, not to max_seqlen_k: that is the bound
         const uint64_t cap_tokens = a->block_table ? static_cast<uint64_t>(a->max_pages_per_seq) * a->cache_tokens
                                                    : static_cast<uint64_t>(a->cache_tokens);
         const uint64_t longest = (a->seqlens_k || step) ? std::max<uint64_t>(cap_tokens, max_s) : static_cast<uint64_t>(max_s);
         const uint64_t units = longest / 64 + static_cast<uint64_t>(nsplit);
-        if (wgs * std::max(nsplit, a->h_k) >= (1ull << 32) || units * nsplit >= (1ull << 32))
+        if (wgs * std::max(std::max(nsplit, a->h_k), row_blocks) >= (1ull << 32) || units * nsplit >= (1ull << 32))
             return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d kv heads: too many workgroups", nsplit, a->b, a->h_k);
     }
     if (static_scratch) {
@@ -369,7 +375,7 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
                         need, kStaticHeads, kStaticScratchBytes - kStaticCounterBytes);
     } else if (nsplit > 1 || step) {
         const size_t need = step ? bitdecode_fwd_append_workspace_bytes(a->b, a->h, nsplit)
-                                 : bitdecode_fwd_workspace_bytes(a->b, a->h, nsplit);
+                                 : bitdecode_fwd_workspace_bytes(a->b, n_h, nsplit);
         if (!a->workspace || a->workspace_bytes < need)
             return fail(BITDECODE_EWORKSPACE, "workspace of %zu bytes needed for %d splits, got %zu", need, nsplit,
                         a->workspace ? a->workspace_bytes : size_t(0));
@@ -398,7 +404,14 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     P.out = static_cast<uint16_t*>(a->out);
     P.out_sb = a->out_stride_b; P.out_sh = a->out_stride_h;
     P.lse = a->softmax_lse;
-    P.b = a->b; P.h = a->h; P.hk = a->h_k; P.g = g; P.nsplit = nsplit;
+    P.b = a->b; P.h = n_h; P.hk = a->h_k; P.g = g; P.nsplit = nsplit;
+    P.rows = rows; P.row_blocks = row_blocks;
+    P.row_blocks_magic = division_magic(static_cast<uint32_t>(row_blocks));
+    P.g_magic = division_magic(static_cast<uint32_t>(g));
+    if (rows_args) {
+        P.q_sr = rows_args->q_stride_row;
+        P.out_sr = rows_args->out_stride_row;
+    }
     P.scale = a->softmax_scale;
     P.scale_log2 = fabsf(a->softmax_scale) * 1.4426950408889634f;   // decode_api.cpp:128-142
     P.neg_scale = a->softmax_scale < 0.0f;
@@ -407,7 +420,8 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     // more than one workgroup per compute unit and lengths that differ: the kernel deals the sequences out so
     // that long ones share a unit with short ones (a pure permutation of the batch index, from the lengths
     // on the device; not in the step with append, whose launch itself advances the lengths)
-    P.seq_perm = a->seqlens_k && !step && a->b >= 2 && a->b <= 64 && static_cast<int64_t>(nsplit) * a->b * a->h_k > cus;
+    P.seq_perm = a->seqlens_k && !step && a->b >= 2 && a->b <= 64 &&
+                 static_cast<int64_t>(nsplit) * a->b * a->h_k * row_blocks > cus;
     P.nsplit_magic = division_magic(static_cast<uint32_t>(nsplit));
     P.hk_magic = division_magic(static_cast<uint32_t>(a->h_k));
     P.block_table = a->block_table; P.bt_stride = a->block_table_stride;
@@ -429,13 +443,13 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
         P.vnew_sb = step->vnew_stride_b; P.vnew_sh = step->vnew_stride_h;
     }
     if (nsplit > 1) {
-        const size_t records = static_cast<size_t>(nsplit) * a->b * a->h;
+        const size_t records = static_cast<size_t>(nsplit) * a->b * n_h;
         if (static_scratch) {
             P.tickets = reinterpret_cast<int*>(static_scratch);
             P.o_part = reinterpret_cast<uint32_t*>(static_scratch + kStaticCounterBytes);
         } else {
             P.tickets = reinterpret_cast<int*>(ws);
-            P.o_part = reinterpret_cast<uint32_t*>(ws + ticket_bytes(a->b, a->h));
+            P.o_part = reinterpret_cast<uint32_t*>(ws + ticket_bytes(a->b, n_h));
         }
         P.ml_part = reinterpret_cast<float*>(P.o_part + 2 * records * kPartialWords);
         if (static_scratch) {
@@ -464,6 +478,11 @@ int bitdecode_fwd_static(const bitdecode_fwd_args* a, void* stream) {
         g_scratch_ptr[dev].store(ptr, std::memory_order_release);
     }
     return run_fwd(a, nullptr, stream, ptr);
+}
+
+int bitdecode_fwd_rows(const bitdecode_fwd_rows_args* a, void* stream) {
+    if (!a) return fail(BITDECODE_EINVAL, "args is null");
+    return run_fwd(&a->fwd, nullptr, stream, nullptr, a);
 }
 
 int bitdecode_fwd_append(const bitdecode_fwd_append_args* a, void* stream) {

@@ -1397,7 +1397,7 @@ __device__ __forceinline__ int sequence_of_position(const FwdParams& P, int p, i
 }
 
 // ---------------------------------------------------------------------------------------------
-// split-KV kernel: 1-D grid of num_splits * h_k * b workgroups of UnitCfg::NW waves.
+// split-KV kernel: 1-D grid of num_splits * h_k * b (ROWS: * blocks of query rows) workgroups of UnitCfg::NW waves.
 // Split s of a (batch, kv-head) owns packed units [s*ups, (s+1)*ups) dealt round-robin to its
 // waves; the 16-token tiles of the fp16 window are dealt round-robin over ALL waves of the head.
 // With more than one split each head's wave writes its (O / sum in fp16, max, sum) and takes a ticket of the head;
@@ -1414,7 +1414,14 @@ constexpr int fwd_lds_bytes() {
     return C::NW * C::REGION + (kMaxGroupHeads + 1) * kQRowBytes + 2 * C::NW * kMaxGroupHeads * 4 + 16 + 2 * kMaxGroupHeads * 4;
 }
 
-template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW>
+// ROWS: several query rows per sequence.  The rows x heads (query row, query head) pairs of a kv head are numbered row
+// by row and cut into blocks of eight, one workgroup per block, so that every MFMA column but those of the last block
+// carries a query whatever the two counts are.  A pair takes the place of a query head: workspace rows, tickets and
+// waves of the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; they are
+// neighbours on one XCD, so all but the first find them in its L2.  (Before, the rows were folded into the head dimension
+// on the host, 8 / g rows per launch, the cache read once per launch: eight rows of 32 / 8 heads over 2 x 8K tokens took
+// four launches and eight copies, 112 us; one launch takes 15.3.)
+template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, bool ROWS>
 // (second bound: waves per SIMD the register count has to leave room for.  Two workgroups of the 8-wave kernels share
 // a compute unit when sequences differ in length, 4 waves per SIMD like the 16-wave kernels: 128 registers.  The
 // per-token-K kernel of group size 32 needs more and runs one workgroup per unit.)
@@ -1461,10 +1468,16 @@ void fwd_splitkv_kernel(FwdParams P) {
     asm volatile("" : : "s"(P.xcd_remap));
     PROF(11);
 #endif
-    int split, hk, bi;
+    int split, hk, bi, blk = 0;
     {
-        const int lin = blockIdx.x;
+        int lin = blockIdx.x;
         int bhid;
+        if constexpr (ROWS) {      // the block of query rows is the fastest index on an XCD
+            const int xcd = P.xcd_remap ? lin & 7 : 0, r = P.xcd_remap ? lin >> 3 : lin;
+            const int q = div_magic(r, P.row_blocks_magic);
+            blk = r - q * P.row_blocks;
+            lin = P.xcd_remap ? q * 8 + xcd : q;
+        }
         if (P.xcd_remap) {
             const int xcd = lin & 7, r = lin >> 3;
             const int q = div_magic(r, P.nsplit_magic);
@@ -1485,8 +1498,9 @@ void fwd_splitkv_kernel(FwdParams P) {
     const int col = lane & 15, kg = lane >> 4;
     const int head = col & 7;          // query head inside the GQA group
     const bool lo_part = col >= 8;     // columns 8-15 carry the lo halves of the split products
-    const int g = P.g;
-    const int64_t bh = static_cast<int64_t>(bi) * P.hk + hk;
+    // heads (ROWS: row and head pairs) of this workgroup, and the number of the first one
+    const int g = ROWS ? min(kMaxGroupHeads, P.g * P.rows - kMaxGroupHeads * blk) : P.g;
+    const int h0 = ROWS ? hk * P.g * P.rows + kMaxGroupHeads * blk : hk * P.g;
 
     int S, R, r_new = -1, step_len = 0;
     if constexpr (APPEND) {
@@ -1517,9 +1531,17 @@ void fwd_splitkv_kernel(FwdParams P) {
     u4 qa_raw, qb_raw, qa, qb;
     {
         const int hq = lane >> 4;                         // head within a row of four
-        const uint16_t* q0 = P.q + bi * P.q_sb + (hk * g) * P.q_sh + (lane & 15) * 8;
-        qa_raw = load_untracked(q0 + (hq < g ? hq : 0) * P.q_sh);
-        qb_raw = load_untracked(q0 + (hq + 4 < g ? hq + 4 : 0) * P.q_sh);
+        if constexpr (ROWS) {
+            const uint16_t* q0 = P.q + bi * P.q_sb + (hk * P.g) * P.q_sh + (lane & 15) * 8;
+            const int xa = kMaxGroupHeads * blk + (hq < g ? hq : 0), xb = kMaxGroupHeads * blk + (hq + 4 < g ? hq + 4 : 0);
+            const int ra = div_magic(xa, P.g_magic), rb = div_magic(xb, P.g_magic);
+            qa_raw = load_untracked(q0 + ra * P.q_sr + (xa - ra * P.g) * P.q_sh);
+            qb_raw = load_untracked(q0 + rb * P.q_sr + (xb - rb * P.g) * P.q_sh);
+        } else {
+            const uint16_t* q0 = P.q + bi * P.q_sb + (hk * g) * P.q_sh + (lane & 15) * 8;
+            qa_raw = load_untracked(q0 + (hq < g ? hq : 0) * P.q_sh);
+            qb_raw = load_untracked(q0 + (hq + 4 < g ? hq + 4 : 0) * P.q_sh);
+        }
     }
     PROF(13);
     UnitAddr<BITS, GS> A;
@@ -1542,9 +1564,9 @@ void fwd_splitkv_kernel(FwdParams P) {
         if constexpr (KT) {
             const kblock ob = karg_block<BLOCK_AT(o_part)>();       // o_part ... bits
             tk = BLOCK_PTR(const int*, ob, o_part, tickets) +
-                 (static_cast<int64_t>(bi) * BLOCK_I32(ob, o_part, h) + hk * g) * kTicketStride + kSlotWord;
+                 (static_cast<int64_t>(bi) * BLOCK_I32(ob, o_part, h) + h0) * kTicketStride + kSlotWord;
         } else {
-            tk = P.tickets + (static_cast<int64_t>(bi) * P.h + hk * g) * kTicketStride + kSlotWord;
+            tk = P.tickets + (static_cast<int64_t>(bi) * P.h + h0) * kTicketStride + kSlotWord;
         }
         const uint64_t heads = (1ull << g) - 1;
         uint64_t saved;
@@ -1712,13 +1734,20 @@ void fwd_splitkv_kernel(FwdParams P) {
     // trip is over by the time wave j needs it.  The ticket travels through LDS (s_tick).
     const bool helpers = NW >= 2 * g;
     if (split_run && helpers && wave >= g && wave < 2 * g && lane == 0) {
-        const int64_t hr = static_cast<int64_t>(bi) * n_h + hk * g + (wave - g);
+        const int64_t hr = static_cast<int64_t>(bi) * n_h + h0 + (wave - g);
         const int d = __hip_atomic_fetch_add(&tickets[hr * kTicketStride], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         __hip_atomic_store(&s_tick[wave - g], d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    const int hq = hk * g + wave;                                  // this wave's query head
+    const int hq = h0 + wave;                                      // this wave's query head
     const int64_t hrow = static_cast<int64_t>(bi) * n_h + hq;      // its row in [b][h] tables
-    uint16_t* const out_row = out + bi * out_sb + hq * out_sh;
+    uint16_t* out_row = out + bi * out_sb + hq * out_sh;
+    float* lse_row = lse_out ? lse_out + hrow : nullptr;
+    if constexpr (ROWS) {
+        const int x = kMaxGroupHeads * blk + wave, row = div_magic(x, P.g_magic);
+        const int head_of_row = hk * P.g + x - row * P.g;
+        out_row = out + bi * out_sb + row * P.out_sr + head_of_row * out_sh;
+        if (lse_out) lse_row = lse_out + (static_cast<int64_t>(bi) * P.rows + row) * (P.g * P.hk) + head_of_row;
+    }
     if (wave < g) {
         // weights of the waves: lane (any row, w) takes wave w; the row reductions give every lane the
         // head's maximum, the weights travel to all lanes as scalars
@@ -1738,7 +1767,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             O1 = __builtin_fmaf(a, v.y, O1);
         }
         if (!split_run) {
-            write_head<BF16>(out_row, lse_out ? lse_out + hrow : nullptr, lane, O0, O1, M, L, p_shift(BITS));
+            write_head<BF16>(out_row, lse_row, lane, O0, O1, M, L, p_shift(BITS));
         } else {
             const int par = __builtin_amdgcn_readfirstlane(s_cnt[wave]) & 1;
             const uint32_t mine_words = par ? slot_words : 0u, other_words = par ? 0u : slot_words;
@@ -1778,7 +1807,7 @@ void fwd_splitkv_kernel(FwdParams P) {
                 if (wave == 0) *s_last = last;
             } else if (last) {
                 merge_splits<kMergeLoads>(o_part, lo_words, ml_part, hrow, P.nsplit, lane, O0, O1, M, L, PROF_TS);
-                write_head<BF16>(out_row, lse_out ? lse_out + hrow : nullptr, lane, O0, O1, M, L, p_shift(BITS));
+                write_head<BF16>(out_row, lse_row, lane, O0, O1, M, L, p_shift(BITS));
             }
         }
     }
@@ -1793,7 +1822,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             if (appends) step_begin<NW>(bi, hk, step_len);
             if (wave < g && last) {
                 merge_splits<kMergeLoads>(o_part, lo_words, ml_part, hrow, P.nsplit, lane, O0, O1, M, L, PROF_TS);
-                write_head<BF16>(out_row, lse_out ? lse_out + hrow : nullptr, lane, O0, O1, M, L, p_shift(BITS));
+                write_head<BF16>(out_row, lse_row, lane, O0, O1, M, L, p_shift(BITS));
             }
         }
         if (appends) step_end<BITS, GS, BF16, KT>(lds, bi, hk, step_len);
@@ -1802,7 +1831,7 @@ void fwd_splitkv_kernel(FwdParams P) {
     PROF_FLUSH();
 }
 
-template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW>
+template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, bool ROWS>
 hipError_t launch_fwd_ttt(const FwdParams& P, hipStream_t stream) {
     constexpr int kLds = fwd_lds_bytes<BITS, GS, FEW>();
     // the dynamic-LDS limit is raised once per kernel and device (idempotent, so a race between
@@ -1811,12 +1840,12 @@ hipError_t launch_fwd_ttt(const FwdParams& P, hipStream_t stream) {
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
     if (dev < 0 || dev >= 64 || !configured[dev].load(std::memory_order_acquire)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW, ROWS>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) return e;
         if (dev >= 0 && dev < 64) configured[dev].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW>), dim3(P.nsplit * P.hk * P.b),
+    hipLaunchKernelGGL((fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW, ROWS>), dim3(P.nsplit * P.hk * P.b * (ROWS ? P.row_blocks : 1)),
                        dim3(UnitCfg<BITS, GS, FEW>::NW * 64), kLds, stream, P);
     return hipGetLastError();
 }
@@ -1827,32 +1856,31 @@ hipError_t launch_fwd_ttt(const FwdParams& P, hipStream_t stream) {
 // 128K tokens and from 1 to 16 sequences of equal length.  The 16 waves keep more bytes in flight per compute
 // unit, which only pays when a few workgroups are left streaming alone (ragged batches).  A 2-bit unit admits
 // only four rows in flight, and there the 8 waves lose 2-3 %: not built.
-template <int BITS, int GS, bool BF16, bool APPEND, bool KT = false>
+template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool ROWS>
 hipError_t launch_fwd_tt(const FwdParams& P, hipStream_t stream) {
     if constexpr (few_waves_variant(BITS, GS)) {
-        if (P.few_waves) return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, true>(P, stream);
+        if (P.few_waves) return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, true, ROWS>(P, stream);
     }
-    return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, false>(P, stream);
+    return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, false, ROWS>(P, stream);
+}
+
+template <int BITS, int GS, bool BF16, bool KT>
+hipError_t launch_fwd_b(const FwdParams& P, hipStream_t stream) {
+    if (P.lengths) return launch_fwd_tt<BITS, GS, BF16, true, KT, false>(P, stream);
+    return P.rows > 1 ? launch_fwd_tt<BITS, GS, BF16, false, KT, true>(P, stream)
+                      : launch_fwd_tt<BITS, GS, BF16, false, KT, false>(P, stream);
 }
 
 template <int BITS, int GS>
 hipError_t launch_fwd_t(const FwdParams& P, hipStream_t stream) {
     if (P.ktensor) {      // "k-tensor" mode: 4 bits
         if constexpr (BITS == 4) {
-            if (P.lengths) {
-                return P.bf16 ? launch_fwd_tt<BITS, GS, true, true, true>(P, stream)
-                              : launch_fwd_tt<BITS, GS, false, true, true>(P, stream);
-            }
-            return P.bf16 ? launch_fwd_tt<BITS, GS, true, false, true>(P, stream)
-                          : launch_fwd_tt<BITS, GS, false, false, true>(P, stream);
+            return P.bf16 ? launch_fwd_b<BITS, GS, true, true>(P, stream) : launch_fwd_b<BITS, GS, false, true>(P, stream);
         } else {
             return hipErrorInvalidValue;
         }
     }
-    if (P.lengths) {
-        return P.bf16 ? launch_fwd_tt<BITS, GS, true, true>(P, stream) : launch_fwd_tt<BITS, GS, false, true>(P, stream);
-    }
-    return P.bf16 ? launch_fwd_tt<BITS, GS, true, false>(P, stream) : launch_fwd_tt<BITS, GS, false, false>(P, stream);
+    return P.bf16 ? launch_fwd_b<BITS, GS, true, false>(P, stream) : launch_fwd_b<BITS, GS, false, false>(P, stream);
 }
 
 }  // namespace

@@ -207,21 +207,21 @@ def _run_kept(key, q, kwargs, make_plan):
         plan = make_plan(True)
         out, lse = plan.out, plan.lse
         # a kept plan must not keep the caller's tensors alive: it holds addresses, and its workspace
-        fwd = plan.args.fwd if isinstance(plan.args, _lib.FwdAppendArgs) else plan.args
+        fwd = plan.fwd
         plan._keep = plan._keep[-1:] if fwd.workspace else ()
         plan.out = plan.lse = None
         if len(cache) >= _MAX_PLANS:
             cache.pop(next(iter(cache)))
         cache[key] = plan
     else:
-        fwd = plan.args.fwd if isinstance(plan.args, _lib.FwdAppendArgs) else plan.args
+        fwd = plan.fwd
         out = kwargs.get("out")
         if out is None:         # a new output (and LSE) tensor per call, as the reference returns
             out = torch.empty_like(q)
             fwd.out = out.data_ptr()
         lse = None
         if return_lse:
-            lse = torch.empty((fwd.b, fwd.h), dtype=torch.float32, device=q.device)
+            lse = torch.empty(plan.lse_shape, dtype=torch.float32, device=q.device)
             fwd.softmax_lse = lse.data_ptr()
     with _on_device(plan.device):
         plan.run()
@@ -308,14 +308,21 @@ class DecodePlan:
 
     def __init__(self, args, out: torch.Tensor, lse: Optional[torch.Tensor],
                  keep: tuple, device: torch.device):
-        self.args = args            # FwdArgs, or FwdAppendArgs for a decode step with append
+        # FwdArgs, FwdRowsArgs (several query rows per sequence) or FwdAppendArgs (a decode step with append)
+        self.args = args
+        self.fwd = args if isinstance(args, _lib.FwdArgs) else args.fwd
         self.out = out
         self.lse = lse
         self._keep = keep
         self.device = device
-        step = isinstance(args, _lib.FwdAppendArgs)
-        self.num_splits = args.fwd.num_splits if step else args.num_splits
-        self._fn = _lib.lib().bitdecode_fwd_append if step else _lib.lib().bitdecode_fwd
+        self.num_splits = self.fwd.num_splits
+        self.lse_shape = (self.fwd.b, self.fwd.h)
+        self._fn = _lib.lib().bitdecode_fwd
+        if isinstance(args, _lib.FwdAppendArgs):
+            self._fn = _lib.lib().bitdecode_fwd_append
+        elif isinstance(args, _lib.FwdRowsArgs):
+            self._fn = _lib.lib().bitdecode_fwd_rows
+            self.lse_shape = (self.fwd.b, args.rows, self.fwd.h)
         self._ref = ctypes.byref(args)
 
     def run(self, stream: Optional[int] = None) -> torch.Tensor:
@@ -344,16 +351,17 @@ def plan_fwd_kvcache_int(q: torch.Tensor,
                          num_splits: int = 0,
                          out: Optional[torch.Tensor] = None,
                          return_lse: bool = False,
-                         _stream_ws: bool = False) -> DecodePlan:
+                         _stream_ws: bool = False,
+                         _rows: bool = False) -> DecodePlan:
     """Validates a decode call and returns a `DecodePlan`; see `fwd_kvcache_int`."""
     mode = _check_quant(quant_mode, group_size, num_bits)
-    if q.dim() != 4 or q.shape[1] != 1:
+    if q.dim() != 4 or (q.shape[1] != 1 and not _rows):
         raise RuntimeError("q must be [batch, 1, nheads, head_dim] (one query token per sequence)")
     if not q.is_cuda:
         raise RuntimeError("q must be on a GPU device")
     dtype = _dtype_code(q)
     device = q.device
-    b, _, h, d = q.shape
+    b, m, h, d = q.shape
     cb, S, h_k = _check_cache(k_pack, k_params, v_pack, v_params, num_bits, group_size, device, mode == _lib.K_TENSOR)
     paged = opt_block_table is not None
     if paged:      # page pools: cb pages of S tokens; a sequence holds up to max_pages_per_seq * S tokens
@@ -367,7 +375,8 @@ def plan_fwd_kvcache_int(q: torch.Tensor,
     if q.stride(3) != 1:
         raise RuntimeError("Input tensor must have contiguous last dimension")
 
-    a = _lib.FwdArgs()
+    args = _lib.FwdRowsArgs() if m > 1 else _lib.FwdArgs()
+    a = args.fwd if m > 1 else args
     keep = [q, k_pack, k_params, v_pack, v_params]
     a.q, a.q_stride_b, a.q_stride_h = q.data_ptr(), q.stride(0), q.stride(2)
     a.k_pack, a.k_params = k_pack.data_ptr(), k_params.data_ptr()
@@ -425,7 +434,7 @@ def plan_fwd_kvcache_int(q: torch.Tensor,
     a.out, a.out_stride_b, a.out_stride_h = out.data_ptr(), out.stride(0), out.stride(2)
     lse = None
     if return_lse:
-        lse = torch.empty((b, h), dtype=torch.float32, device=device)
+        lse = torch.empty((b, h) if m == 1 else (b, m, h), dtype=torch.float32, device=device)
         keep.append(lse)
         a.softmax_lse = lse.data_ptr()
     a.b, a.h, a.h_k, a.d = b, h, h_k, d
@@ -433,17 +442,21 @@ def plan_fwd_kvcache_int(q: torch.Tensor,
     a.quant_mode = mode
     a.softmax_scale = float(softmax_scale)
     with _on_device(device):
-        ns, nbytes = _split_plan(device.index, b, h, h_k, a.max_seqlen_k, a.max_res_len, seqlens_k is not None,
-                                 num_bits, group_size, int(num_splits))
+        # (several query rows: a workgroup per eight row and head pairs of a kv head, workspace rows by pairs)
+        blocks = 1 if m == 1 else (m * (h // h_k) + 7) // 8
+        ns, nbytes = _split_plan(device.index, b, h * m, h_k * blocks, a.max_seqlen_k, a.max_res_len,
+                                 seqlens_k is not None, num_bits, group_size, int(num_splits))
         a.num_splits = ns
         if nbytes:
             # zero-filled: the arrival counters at its head must be 0 before the first call
             # (every call leaves them at 0 again)
-            ws = (_stream_workspace(device, "fwd", b, h, ns, nbytes) if _stream_ws
+            ws = (_stream_workspace(device, "fwd", b, h * m, ns, nbytes) if _stream_ws
                   else torch.zeros(nbytes, dtype=torch.uint8, device=device))
             keep.append(ws)
             a.workspace, a.workspace_bytes = ws.data_ptr(), nbytes
-    return DecodePlan(a, out, lse, tuple(keep), device)
+    if m > 1:
+        args.rows, args.q_stride_row, args.out_stride_row = m, q.stride(1), out.stride(1)
+    return DecodePlan(args, out, lse, tuple(keep), device)
 
 
 def fwd_kvcache_int(q: torch.Tensor,
@@ -460,8 +473,8 @@ def fwd_kvcache_int(q: torch.Tensor,
 
     q [b, 1, h, 128] fp16/bf16; returns a new tensor of the same shape.  `softmax_scale`
     defaults to 1.0 as in the reference; callers pass 1/sqrt(d).  q [b, m, h, 128] with m > 1 rows per sequence is
-    accepted too (every row attends every key, as with the reference's fixed is_causal = False): see
-    _fwd_query_rows.
+    accepted too (the reference admits them, decode_api.cpp:341, 358-368: rows of the M tile; its interface fixes
+    is_causal = False, so every row attends every key): one launch for all rows, the LSE is then [b, m, h].
 
     Keyword-only extensions:
       seqlen_k          valid packed tokens (multiple of 128); default = capacity of the cache
@@ -485,31 +498,37 @@ def fwd_kvcache_int(q: torch.Tensor,
 
 def _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale, quant_mode, group_size,
                     num_bits, out=None, return_lse=False, **kwargs):
-    """Several query rows per sequence, q [b, m, h, 128] (the reference admits them, decode_api.cpp:341, 358-368:
-    rows of the M tile; its interface fixes is_causal = False, so every row attends every key).  The kernel's
-    16 columns hold up to eight (query head, row) pairs of a kv head: the rows are folded into the head dimension,
-    8 // (h / h_k) rows per launch, and unfolded again.  Returns [b, m, h, 128] (and lse [b, m, h])."""
+    """`fwd_kvcache_int` for q [b, m, h, 128] with m > 1: the kernel takes the rows as they are (bitdecode_fwd_rows).
+    Returns [b, m, h, 128] (and lse [b, m, h])."""
     b, m, h, d = q.shape
     h_k = v_pack.shape[2]
     if h_k <= 0 or h % h_k or h // h_k > 8:
         raise ValueError(f"q has {h} heads for {h_k} kv heads: need a multiple, at most 8 per kv head")
-    g = h // h_k
-    per = max(1, 8 // g)
-    res = out if out is not None else torch.empty_like(q)
-    if res.shape != q.shape or res.dtype != q.dtype or res.device != q.device:
+    if out is not None and (out.shape != q.shape or out.dtype != q.dtype or out.device != q.device):
         raise ValueError("out must match q in shape, dtype and device")
-    lse = torch.empty((b, m, h), dtype=torch.float32, device=q.device) if return_lse else None
-    for r0 in range(0, m, per):
-        mr = min(per, m - r0)
-        # (kv head, query head in the group, row) -> one head index
-        qv = q[:, r0:r0 + mr].reshape(b, mr, h_k, g, d).permute(0, 2, 3, 1, 4).reshape(b, 1, h_k * g * mr, d).contiguous()
-        got = fwd_kvcache_int(qv, k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale, quant_mode,
-                              group_size, num_bits, return_lse=return_lse, **kwargs)
-        ov, lv = got if return_lse else (got, None)
-        res[:, r0:r0 + mr] = ov.reshape(b, h_k, g, mr, d).permute(0, 3, 1, 2, 4).reshape(b, mr, h, d)
-        if return_lse:
-            lse[:, r0:r0 + mr] = lv.reshape(b, h_k, g, mr).permute(0, 3, 1, 2).reshape(b, mr, h)
-    return (res, lse) if return_lse else res
+    if q.stride(3) != 1 or q.data_ptr() % 16 or any(s % 8 for s in q.stride()[:3]):
+        q = q.contiguous()
+    # the workspace holds a record per row, head and split: many rows of a large batch go in several launches
+    per = max(1, 32768 // max(1, b * h))
+    if m > per or (out is not None and out.stride(3) != 1):
+        res = out if out is not None else torch.empty_like(q)
+        parts = []
+        for r0 in range(0, m, per):
+            got = fwd_kvcache_int(q[:, r0:r0 + per], k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale,
+                                  quant_mode, group_size, num_bits, return_lse=return_lse, **kwargs)
+            o, lse = got if return_lse else (got, None)
+            res[:, r0:r0 + per] = o
+            if return_lse:
+                parts.append(lse.reshape(b, -1, h))
+        return (res, torch.cat(parts, 1)) if return_lse else res
+    if out is not None:
+        kwargs["out"] = out
+    kwargs["return_lse"] = return_lse
+    key = _call_key((q, k_pack, k_params, v_pack, v_params, opt_block_table),
+                    (softmax_scale, quant_mode, group_size, num_bits), kwargs)
+    return _run_kept(key, q, kwargs, lambda shared: plan_fwd_kvcache_int(
+        q, k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale, quant_mode, group_size, num_bits,
+        _stream_ws=shared, _rows=True, **kwargs))
 
 
 def plan_fwd_kvcache_int_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor,

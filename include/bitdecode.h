@@ -136,6 +136,20 @@ int bitdecode_fwd(const bitdecode_fwd_args* args, void* stream);
  * the array's address (hipGetSymbolAddress): make it outside any stream capture. */
 int bitdecode_fwd_static(const bitdecode_fwd_args* args, void* stream);
 
+/* bitdecode_fwd for several query rows per sequence (the reference's host code admits them, decode_api.cpp:341,
+ * 358-368; its interface fixes is_causal = False, so every row attends every key).  In `fwd`: q and out are
+ * [b, rows, h, 128], softmax_lse is [b, rows, h]; the workspace is sized, and zeroed for another shape, as for
+ * rows * h heads: bitdecode_fwd_workspace_bytes(b, rows * h, num_splits).  The rows * (h / h_k) row and head pairs
+ * of a kv head run in blocks of eight, one workgroup each: bitdecode_num_splits(_for) wants h_k * ceil(that / 8). */
+typedef struct bitdecode_fwd_rows_args {
+    bitdecode_fwd_args fwd;
+    int32_t rows;              /* query rows per sequence, 1 to 4096                        */
+    int64_t q_stride_row;      /* elements, a multiple of 8                                 */
+    int64_t out_stride_row;
+} bitdecode_fwd_rows_args;
+
+int bitdecode_fwd_rows(const bitdecode_fwd_rows_args* args, void* stream);
+
 /* One decode step in one launch: attend the new token together with everything held, append it, and
  * quantize-pack the fp16 window when it fills.  This is the "residual kernel" the reference's figures
  * describe (imgs/overview.png, imgs/scheme.png) and its kernel traits still name

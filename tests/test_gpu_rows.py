@@ -1,0 +1,53 @@
+"""Several query rows per sequence in one launch: the (row, head) pairs of a kv head run in blocks of eight."""
+import math
+
+import pytest
+import torch
+
+from oracle import bitdecode_oracle as O
+from tests import helpers as H
+
+pytestmark = pytest.mark.gpu
+
+SCALE = 1.0 / math.sqrt(128)
+
+
+@pytest.mark.parametrize("h,h_k,m,bits,gs,mode,dtype,ns,paged", [
+    (6, 2, 5, 4, 128, "k-channel", "fp16", 3, False),      # 15 pairs: a row is cut by the block boundary, last block of 7
+    (3, 3, 9, 2, 64, "k-channel", "fp16", 2, False),       # 9 pairs: last block of 1
+    (16, 2, 2, 4, 32, "k-channel", "bf16", 1, True),       # 16 pairs, one block per row, one split
+    (8, 1, 3, 4, 64, "k-tensor", "fp16", 4, False),
+    (7, 1, 300, 2, 128, "k-channel", "fp16", 0, True),     # many blocks, more workgroups than compute units
+])
+def test_rows_equal_the_calls_for_each_row(device, h, h_k, m, bits, gs, mode, dtype, ns, paged):
+    """Every row of one launch equals a call with that row alone: both take the same scores and differ by the split
+    count at most, so by the rounding of the fp16 records and of the output (2^-11 of |out| < 2 each: 1e-3, and a bf16
+    output by its rounding, 2^-8 of |out|)."""
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
+    b, S, R = 3, 128 * 10, 53
+    _, k, v = O.make_inputs(b, h, h_k, S, R, seed=m, dtype=dtype)
+    tdt = H.torch_dtype(dtype)
+    kd, vd = H.to_dev(k, dtype, device), H.to_dev(v, dtype, device)
+    g = torch.Generator(device=device).manual_seed(m)
+    wide = torch.randn((b, h, m, 128), generator=g, device=device).to(tdt)
+    q = wide.transpose(1, 2)                                # rows are not the slowest index in memory
+    table = None
+    if paged:
+        table = torch.randperm(b * S // 256, generator=g, device=device).to(torch.int32).reshape(b, -1)
+        cache = H.alloc_cache(b * S // 256, 256, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
+    else:
+        cache = H.alloc_cache(b, S, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
+    kvcache_pack_int(kd[:, :S], cache[0], cache[1], vd[:, :S], cache[2], cache[3], table, None, S, mode, gs, bits)
+    lens = torch.tensor([S, 128 * 3, 0], dtype=torch.int32, device=device)
+    res = torch.tensor([R, 1, 17], dtype=torch.int32, device=device)
+    kw = dict(seqlens_k=lens, k_residual=kd[:, S:], v_residual=vd[:, S:], residual_len=res, return_lse=True)
+    args = (*cache, table, SCALE, mode, gs, bits)
+    given = torch.full((b, m, h, 128), float("nan"), dtype=tdt, device=device)
+    for _ in range(2):                                      # the second launch finds the workspace as the first left it
+        out, lse = fwd_kvcache_int(q, *args, num_splits=ns, out=given, **kw)
+    assert out is given and lse.shape == (b, m, h)
+    for r in sorted({0, 1, m // 2, m - 1}):
+        one, lse1 = fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args, num_splits=ns, **kw)
+        err = (out[:, r:r + 1].float() - one.float()).abs()
+        assert (err <= 1e-3 + (2 ** -8 * one.float().abs() if dtype == "bf16" else 0)).all(), (r, err.max().item())
+        assert (lse[:, r] - lse1).abs().max().item() < 1e-4, r
