@@ -645,8 +645,14 @@ __device__ __forceinline__ h8 q_load(const uint8_t* row, int j) {
 // a*b as an exact fp16 pair: hi columns get hi = round(a*b), lo columns get fma(a, b, -hi).
 // a_lo_only is a in the lo columns and 0 in the hi columns, so no lane select is needed.
 __device__ __forceinline__ h8 split_mul_masked(h8 a, h8 a_lo_only, h8 b) {
-    const h8 hi_in_lo_cols = a_lo_only * b;
-    return __builtin_elementwise_fma(a, b, -hi_in_lo_cols);
+    u4 hi_in_lo_cols = __builtin_bit_cast(u4, a_lo_only * b);
+    // (the product hidden from the optimizer, or it moves the sign to b, whose first register it then negates half by half
+    // with three instructions; a sign on the product is a modifier of the fma: 48 of 732 vector instructions per 2-bit
+    // unit at group 64, 24 of 636 at group 128, 48 of 493 per 4-bit unit at group 32; 128K tokens at 2 bits, group 64:
+    // 24.0 -> 23.5 us, 8 sequences of 64K at 2 bits 68.1 -> 67.3, 6 sequences of 10K at group 32 20.7 -> 20.3)
+#pragma unroll
+    for (int x = 0; x < 4; ++x) asm("" : "+v"(hi_in_lo_cols[x]));
+    return __builtin_elementwise_fma(a, b, -__builtin_bit_cast(h8, hi_in_lo_cols));
 }
 
 template <int BITS, bool BF16>
