@@ -77,10 +77,28 @@ class FwdAppendArgs(ctypes.Structure):
     ]
 
 
+class CacheArgs(ctypes.Structure):
+    _fields_ = [
+        ("k", _vp), ("v", _vp),
+        ("k_stride_b", _i64), ("k_stride_t", _i64), ("k_stride_h", _i64),
+        ("v_stride_b", _i64), ("v_stride_t", _i64), ("v_stride_h", _i64),
+        ("k_pack", _vp), ("k_params", _vp), ("v_pack", _vp), ("v_params", _vp),
+        ("k_res", _vp), ("v_res", _vp),
+        ("kres_stride_b", _i64), ("kres_stride_t", _i64), ("kres_stride_h", _i64),
+        ("vres_stride_b", _i64), ("vres_stride_t", _i64), ("vres_stride_h", _i64),
+        ("total", _vp), ("packed_lens", _vp), ("res_lens", _vp),
+        ("lengths", ctypes.POINTER(_i32)),
+        ("b", _i32), ("n_tokens", _i32), ("h_k", _i32), ("d", _i32),
+        ("cache_tokens", _i32),
+        ("bits", _i32), ("group_size", _i32), ("dtype", _i32),
+        ("quant_mode", _i32),
+    ]
+
+
 EXPORTS = ("bitdecode_abi_version", "bitdecode_last_error", "bitdecode_num_splits",
            "bitdecode_fwd_workspace_bytes", "bitdecode_num_splits_for", "bitdecode_qpack", "bitdecode_fwd",
            "bitdecode_fwd_append", "bitdecode_fwd_append_workspace_bytes", "bitdecode_fwd_static",
-           "bitdecode_fwd_rows")
+           "bitdecode_fwd_rows", "bitdecode_cache_prefill", "bitdecode_cache_append")
 
 _lib = None
 
@@ -121,6 +139,9 @@ def lib():
         L.bitdecode_fwd_rows.argtypes = [ctypes.POINTER(FwdRowsArgs), _vp]
         L.bitdecode_fwd_append.restype = ctypes.c_int
         L.bitdecode_fwd_append.argtypes = [ctypes.POINTER(FwdAppendArgs), _vp]
+        for fn in (L.bitdecode_cache_prefill, L.bitdecode_cache_append):
+            fn.restype = ctypes.c_int
+            fn.argtypes = [ctypes.POINTER(CacheArgs), _vp]
         L.bitdecode_fwd_append_workspace_bytes.restype = ctypes.c_size_t
         L.bitdecode_fwd_append_workspace_bytes.argtypes = [_i32] * 3
         if L.bitdecode_abi_version() != ABI_VERSION:

@@ -13,12 +13,15 @@ device.
 """
 from __future__ import annotations
 
+import ctypes
 import math
 from typing import Optional, Sequence
 
 import torch
 
-from .interface import fwd_kvcache_int, fwd_kvcache_int_append, kvcache_pack_int, plan_fwd_kvcache_int_append
+from . import _lib
+from .interface import (_check_cache, _dtype_code, _on_device, _stream_ptr, fwd_kvcache_int, fwd_kvcache_int_append,
+                        kvcache_pack_int, plan_fwd_kvcache_int_append)
 
 BLOCK = 128          # tokens per packed block = residual window size N_r
 
@@ -59,6 +62,8 @@ class BitKVCache:
         self.res_len = [0] * batch
         self.total = torch.zeros(batch, dtype=torch.int32, device=dev)     # tokens held, as `step` needs them
         self._rows = torch.arange(batch, device=dev)
+        # packed and window lengths on the device as the last `prefill` or `append` left them (_publish_lengths)
+        self._published = None
 
     # ------------------------------------------------------------------ lengths
     @property
@@ -69,6 +74,62 @@ class BitKVCache:
         return torch.tensor(list(values), dtype=torch.int32, device=self.device)
 
     # ------------------------------------------------------------------ writes
+    def _write(self, entry: str, k: torch.Tensor, v: torch.Tensor, lengths: list[int]) -> bool:
+        """`prefill` or `append` in one launch: tokens k / v [b, n, h_k, 128], lengths per sequence, to the packed cache,
+        the window, `total` and a new pair of device length arrays.  False if the tensors are not what the kernels take
+        (another element type than the cache's, unaligned or strided rows, a capture in progress, no GPU): the caller then
+        works with torch operations."""
+        kr, vr = self.k_res, self.v_res
+        if (not kr.is_cuda or self.b < 1 or k.dim() != 4 or k.shape != v.shape or k.shape[0] != self.b or
+                k.shape[2] != self.h_k or k.shape[3] != 128 or kr.shape != (self.b, BLOCK, self.h_k, 128) or
+                vr.shape != kr.shape or self.total.dtype != torch.int32 or self.total.shape != (self.b,) or
+                self.total.stride(0) != 1):
+            return False
+        device, dtype = kr.device, kr.dtype
+        args = (k, v, kr, vr)
+        for t in args:
+            st = t.stride()
+            if (t.dtype != dtype or t.device != device or st[3] != 1 or (st[0] | st[1] | st[2]) % 8 or
+                    t.data_ptr() % 16):
+                return False
+        if self.total.device != device or torch.cuda.is_current_stream_capturing():
+            return False
+        b, S, h_k = _check_cache(self.k_pack, self.k_params, self.v_pack, self.v_params, self.bits, self.gs, device,
+                                 self.quant_mode == "k-tensor")
+        if (b, S, h_k) != (self.b, self.capacity, self.h_k):
+            return False
+        a = _lib.CacheArgs()
+        a.k, a.v, a.k_res, a.v_res = (t.data_ptr() for t in args)
+        a.k_stride_b, a.k_stride_t, a.k_stride_h = k.stride()[:3]
+        a.v_stride_b, a.v_stride_t, a.v_stride_h = v.stride()[:3]
+        a.kres_stride_b, a.kres_stride_t, a.kres_stride_h = kr.stride()[:3]
+        a.vres_stride_b, a.vres_stride_t, a.vres_stride_h = vr.stride()[:3]
+        a.k_pack, a.k_params = self.k_pack.data_ptr(), self.k_params.data_ptr()
+        a.v_pack, a.v_params = self.v_pack.data_ptr(), self.v_params.data_ptr()
+        # new arrays with every call: an earlier `decode` may still be reading the old ones on another stream
+        packed = torch.empty(b, dtype=torch.int32, device=device)
+        res = torch.empty_like(packed)
+        a.total, a.packed_lens, a.res_lens = self.total.data_ptr(), packed.data_ptr(), res.data_ptr()
+        a.lengths = (ctypes.c_int32 * b)(*lengths)
+        a.b, a.n_tokens, a.h_k, a.d = b, k.shape[1], h_k, 128
+        a.cache_tokens = S
+        a.bits, a.group_size, a.dtype = self.bits, self.gs, _dtype_code(kr)
+        a.quant_mode = _lib.K_TENSOR if self.quant_mode == "k-tensor" else _lib.K_CHANNEL
+        with _on_device(device):
+            stream = _stream_ptr(device)
+            _lib.check(getattr(_lib.lib(), entry)(ctypes.byref(a), stream))
+        self._published = (packed, res, stream)      # (the caller adds the host's lengths)
+        return True
+
+    def _device_lengths(self):
+        """Packed and window lengths as device tensors: those the last write left if the host's lengths are still theirs
+        and the stream is the one that wrote them (their memory belongs to it), else uploaded."""
+        if self._published is not None:
+            packed, res, stream, host_packed, host_res = self._published
+            if host_packed == self.packed_len and host_res == self.res_len and _stream_ptr(packed.device) == stream:
+                return packed, res
+        return self._i32(self.packed_len), self._i32(self.res_len)
+
     def prefill(self, k: torch.Tensor, v: torch.Tensor, lengths: Optional[Sequence[int]] = None) -> None:
         """Start the cache from prompt K/V `[b, L, h_k, 128]` (`lengths[i] <= L` valid tokens per sequence,
         default L): whole 128-token blocks are quantize-packed in one launch, each sequence's last
@@ -81,6 +142,9 @@ class BitKVCache:
             raise ValueError(f"prefill: {max(lengths)} tokens exceed the capacity of {self.capacity}")
         self.packed_len = [x // BLOCK * BLOCK for x in lengths]
         self.res_len = [x - p for x, p in zip(lengths, self.packed_len)]
+        if self._write("bitdecode_cache_prefill", k, v, lengths):
+            self._published += (list(self.packed_len), list(self.res_len))
+            return
         n_pack = max(self.packed_len)
         if n_pack:
             # sequences shorter than n_pack get blocks of padding packed behind their prefix; decode never
@@ -97,10 +161,17 @@ class BitKVCache:
         """Append one token per sequence, `[b, 1, h_k, 128]` (or `[b, h_k, 128]`).  A window that reaches 128
         tokens is quantize-packed behind its sequence's prefix in the same call (one launch for all
         sequences that filled up; the others are skipped through a negative offset)."""
-        if k_new.dim() == 4:
-            k_new, v_new = k_new[:, 0], v_new[:, 0]
         if any(p + r + 1 > self.capacity for p, r in zip(self.packed_len, self.res_len)):
             raise ValueError("append: cache capacity exceeded")
+        if all(p % BLOCK == 0 and 0 <= r < BLOCK for p, r in zip(self.packed_len, self.res_len)):
+            k1, v1 = (k_new[:, :1], v_new[:, :1]) if k_new.dim() == 4 else (k_new[:, None], v_new[:, None])
+            if self._write("bitdecode_cache_append", k1, v1, self.lengths):
+                self.packed_len = [p + BLOCK if r == BLOCK - 1 else p for p, r in zip(self.packed_len, self.res_len)]
+                self.res_len = [(r + 1) % BLOCK for r in self.res_len]
+                self._published += (list(self.packed_len), list(self.res_len))
+                return
+        if k_new.dim() == 4:
+            k_new, v_new = k_new[:, 0], v_new[:, 0]
         pos = self._i32(self.res_len).long()
         self.k_res[self._rows, pos] = k_new.to(self.dtype)
         self.v_res[self._rows, pos] = v_new.to(self.dtype)
@@ -119,12 +190,13 @@ class BitKVCache:
         """Attention of one query token per sequence, `q [b, 1, h, 128]`, over everything appended so far."""
         if softmax_scale is None:
             softmax_scale = 1.0 / math.sqrt(q.shape[-1])
-        max_p, max_r = max(self.packed_len), max(self.res_len)
+        packed, res = self._device_lengths()
+        # (the window's bound is its size, not the longest window of the moment: the same grid, and one call all along a block)
         return fwd_kvcache_int(q, self.k_pack, self.k_params, self.v_pack, self.v_params, None, softmax_scale,
                                self.quant_mode, self.gs, self.bits,
-                               seqlens_k=self._i32(self.packed_len), max_seqlen_k=max_p,
+                               seqlens_k=packed, max_seqlen_k=max(self.packed_len),
                                k_residual=self.k_res, v_residual=self.v_res,
-                               residual_len=self._i32(self.res_len), max_residual_len=max_r, **kw)
+                               residual_len=res, max_residual_len=BLOCK, **kw)
 
     # ------------------------------------------------------------------ one launch per token
     def plan_step(self, q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor,

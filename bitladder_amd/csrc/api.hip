@@ -278,6 +278,79 @@ int bitdecode_qpack(const bitdecode_qpack_args* a, void* stream) {
     return BITDECODE_OK;
 }
 
+// BitKVCache's prefill (append = false) and append of a token (append = true)
+static int run_cache(const bitdecode_cache_args* a, bool append, void* stream) {
+    using namespace bitdecode;
+    if (!a) return fail(BITDECODE_EINVAL, "args is null");
+    if (int rc = check_quant(a->bits, a->group_size, a->dtype, a->d)) return rc;
+    if (int rc = check_mode(a->quant_mode, a->bits)) return rc;
+    if (a->b <= 0 || a->b > 65535 || a->h_k <= 0 || a->h_k > 65535 || a->n_tokens < 0)
+        return fail(BITDECODE_EINVAL, "batch %d, %d kv heads, %d tokens", a->b, a->h_k, a->n_tokens);
+    if (a->cache_tokens % kChunk || a->cache_tokens <= 0)
+        return fail(BITDECODE_EINVAL, "cache_tokens %d is not a positive multiple of 128", a->cache_tokens);
+    if (append && a->n_tokens != 1) return fail(BITDECODE_EINVAL, "append of %d tokens (one per sequence)", a->n_tokens);
+    if (!a->lengths || !a->total || !a->k_pack || !a->k_params || !a->v_pack || !a->v_params || !a->k_res || !a->v_res ||
+        (a->n_tokens > 0 && (!a->k || !a->v)) || !a->packed_lens != !a->res_lens)
+        return fail(BITDECODE_EINVAL, "null tensor pointer");
+    if (!aligned16(a->k) || !aligned16(a->v) || !aligned16(a->k_pack) || !aligned16(a->k_params) || !aligned16(a->v_pack) ||
+        !aligned16(a->v_params) || !aligned16(a->k_res) || !aligned16(a->v_res))
+        return fail(BITDECODE_EINVAL, "tensor pointers must be 16-byte aligned");
+    const int64_t strides[12] = {a->k_stride_b, a->k_stride_t, a->k_stride_h, a->v_stride_b, a->v_stride_t, a->v_stride_h,
+                                 a->kres_stride_b, a->kres_stride_t, a->kres_stride_h,
+                                 a->vres_stride_b, a->vres_stride_t, a->vres_stride_h};
+    for (int64_t s : strides)
+        if (s % 8) return fail(BITDECODE_EINVAL, "K/V strides must be multiples of 8 elements");
+    int longest = 0;
+    for (int i = 0; i < a->b; ++i) {
+        const int n = a->lengths[i];
+        longest = std::max(longest, n);
+        // append: a window that this token fills needs room for its chunk
+        const int64_t need = append && n % kChunk == kChunk - 1 ? static_cast<int64_t>(n) + 1 : n;
+        if (n < 0 || need > a->cache_tokens || (!append && n > a->n_tokens))
+            return fail(BITDECODE_EINVAL, "sequence %d: length %d (%d tokens given, capacity %d)", i, n, a->n_tokens,
+                        a->cache_tokens);
+    }
+    CacheParams P{};
+    P.k = static_cast<const uint16_t*>(a->k);
+    P.v = static_cast<const uint16_t*>(a->v);
+    P.k_sb = a->k_stride_b; P.k_st = a->k_stride_t; P.k_sh = a->k_stride_h;
+    P.v_sb = a->v_stride_b; P.v_st = a->v_stride_t; P.v_sh = a->v_stride_h;
+    P.k_pack = static_cast<uint8_t*>(a->k_pack);
+    P.k_params = static_cast<uint8_t*>(a->k_params);
+    P.v_pack = static_cast<uint8_t*>(a->v_pack);
+    P.v_params = static_cast<uint8_t*>(a->v_params);
+    P.kpack_bh = code_region_bytes(a->cache_tokens, a->bits);
+    P.vpack_bh = P.kpack_bh;
+    P.ktensor = a->quant_mode == BITDECODE_K_TENSOR;
+    P.kparams_bh = P.ktensor ? v_param_region_bytes(a->cache_tokens, a->group_size)
+                             : k_param_region_bytes(a->cache_tokens, a->group_size);
+    P.vparams_bh = v_param_region_bytes(a->cache_tokens, a->group_size);
+    P.k_res = static_cast<uint16_t*>(a->k_res);
+    P.v_res = static_cast<uint16_t*>(a->v_res);
+    P.kres_sb = a->kres_stride_b; P.kres_st = a->kres_stride_t; P.kres_sh = a->kres_stride_h;
+    P.vres_sb = a->vres_stride_b; P.vres_st = a->vres_stride_t; P.vres_sh = a->vres_stride_h;
+    P.total = a->total; P.packed_lens = a->packed_lens; P.res_lens = a->res_lens;
+    P.b = a->b; P.hk = a->h_k;
+    P.pack_chunks = longest / kChunk;
+    P.bits = a->bits; P.gs = a->group_size; P.bf16 = a->dtype == BITDECODE_BF16;
+    for (P.first = 0; P.first < a->b; P.first += kCacheSeqs) {
+        const int n = std::min(kCacheSeqs, a->b - P.first);
+        bool fills = false;
+        for (int i = 0; i < n; ++i) {
+            P.lengths[i] = a->lengths[P.first + i];
+            fills = fills || P.lengths[i] % kChunk == kChunk - 1;
+        }
+        hipError_t e = append ? launch_cache_append(P, n, fills, static_cast<hipStream_t>(stream))
+                              : launch_cache_prefill(P, n, static_cast<hipStream_t>(stream));
+        if (e != hipSuccess) return fail(BITDECODE_ELAUNCH, "cache launch failed: %s", hipGetErrorString(e));
+    }
+    return BITDECODE_OK;
+}
+
+int bitdecode_cache_prefill(const bitdecode_cache_args* a, void* stream) { return run_cache(a, false, stream); }
+
+int bitdecode_cache_append(const bitdecode_cache_args* a, void* stream) { return run_cache(a, true, stream); }
+
 // bytes of the per-sequence step counters that lead a step workspace
 static size_t step_ticket_bytes(int32_t b) { return static_cast<size_t>(b) * bitdecode::kTicketStride * sizeof(int); }
 

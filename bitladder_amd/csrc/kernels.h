@@ -32,6 +32,31 @@ struct QpackParams {
     int chunks_per_page;
 };
 
+// BitKVCache's prefill and append (qpack.hip).  Lengths come from the host and travel as kernel arguments: nothing is
+// copied to the device ahead of the launch (a copy of a few integers from pageable memory waits for the stream).
+constexpr int kCacheSeqs = 128;     // sequences per launch
+struct CacheParams {
+    const uint16_t* k;          // prefill: [b][n][hk][128]; append: the new token, n = 1
+    const uint16_t* v;
+    int64_t k_sb, k_st, k_sh, v_sb, v_st, v_sh;      // element strides
+    uint8_t* k_pack;
+    uint8_t* k_params;
+    uint8_t* v_pack;
+    uint8_t* v_params;
+    int64_t kpack_bh, kparams_bh, vpack_bh, vparams_bh;  // bytes per (batch, kv-head) region
+    uint16_t* k_res;            // fp16 window [b][>= 128][hk][128]
+    uint16_t* v_res;
+    int64_t kres_sb, kres_st, kres_sh, vres_sb, vres_st, vres_sh;
+    int* total;                 // device counters: tokens held, and (optional) packed and window tokens, after the call
+    int* packed_lens;
+    int* res_lens;
+    int b, hk;
+    int pack_chunks;            // prefill: whole chunks of the longest prompt (of all launches)
+    int first;                  // sequence of the launch's block 0
+    int bits, gs, bf16, ktensor;
+    int lengths[kCacheSeqs];    // of sequences first, first + 1, ...: prompt tokens (prefill), tokens held before (append)
+};
+
 // The decode kernel fetches its arguments in 64-byte blocks with scalar loads of its own (decode.hip): the first
 // three blocks, everything a workgroup needs up to its first loads of the stream, in one round at its entry;
 // k_res ... vres_sh and o_part ... bits where they are used.  Keep each group contiguous and in this order;
@@ -108,6 +133,10 @@ inline uint32_t division_magic(uint32_t d) { return d <= 1 ? 0u : static_cast<ui
 
 hipError_t launch_qpack(const QpackParams& p, hipStream_t stream);
 hipError_t launch_fwd(const FwdParams& p, hipStream_t stream);
+// `n` sequences from p.first on
+hipError_t launch_cache_prefill(const CacheParams& p, int n, hipStream_t stream);
+// fills: some sequence's window becomes full and is packed
+hipError_t launch_cache_append(const CacheParams& p, int n, bool fills, hipStream_t stream);
 #ifdef BITDECODE_PROF
 hipError_t set_prof_buffer(unsigned long long* p);   // per-wave timeline buffer (tuning builds only)
 #endif

@@ -181,6 +181,42 @@ typedef struct bitdecode_fwd_append_args {
 int bitdecode_fwd_append(const bitdecode_fwd_append_args* args, void* stream);
 size_t bitdecode_fwd_append_workspace_bytes(int32_t b, int32_t h, int32_t num_splits);
 
+/* The write side of a cache of packed prefixes and fp16 windows in one launch (per 128 sequences).  No counterpart in the
+ * reference, which ships no cache management.  Sequence i's tokens lie in the packed cache up to the last multiple of 128
+ * and behind that in rows 0.. of its window.  The lengths are read on the HOST during the call and travel as kernel
+ * arguments; the device arrays are written.
+ *   bitdecode_cache_prefill   starts sequence i from the first lengths[i] <= n_tokens tokens of k / v: whole chunks are
+ *                             packed, the rest goes to the window, total[i] = lengths[i] (chunks up to the longest
+ *                             sequence's last are packed for all; those behind a shorter one are padding);
+ *   bitdecode_cache_append    adds one token (n_tokens = 1) to a sequence that holds lengths[i]: stored in the window's
+ *                             next row, a window that it fills is packed behind the prefix, total[i] += 1.
+ * packed_lens / res_lens (both or neither) receive what bitdecode_fwd takes as seqlens_k / res_lens after the call. */
+typedef struct bitdecode_cache_args {
+    const void* k;             /* [b, n_tokens, h_k, 128] fp16/bf16, last dim contiguous    */
+    const void* v;
+    int64_t k_stride_b, k_stride_t, k_stride_h;
+    int64_t v_stride_b, v_stride_t, v_stride_h;
+    void* k_pack;              /* contiguous cache, as in bitdecode_qpack_args              */
+    void* k_params;
+    void* v_pack;
+    void* v_params;
+    void* k_res;               /* window [b, >= 128, h_k, 128], element type of k           */
+    void* v_res;
+    int64_t kres_stride_b, kres_stride_t, kres_stride_h;
+    int64_t vres_stride_b, vres_stride_t, vres_stride_h;
+    int32_t* total;            /* device int32[b]                                           */
+    int32_t* packed_lens;      /* optional device int32[b]                                  */
+    int32_t* res_lens;         /* optional device int32[b]                                  */
+    const int32_t* lengths;    /* HOST int32[b]                                             */
+    int32_t b, n_tokens, h_k, d;   /* d must be 128                                         */
+    int32_t cache_tokens;      /* capacity S of the packed tensors, multiple of 128         */
+    int32_t bits, group_size, dtype;
+    int32_t quant_mode;        /* BITDECODE_K_CHANNEL / BITDECODE_K_TENSOR                  */
+} bitdecode_cache_args;
+
+int bitdecode_cache_prefill(const bitdecode_cache_args* args, void* stream);
+int bitdecode_cache_append(const bitdecode_cache_args* args, void* stream);
+
 /* Split count the library would choose for this problem (host function, no GPU work);
  * replaces num_splits_heuristic (csrc/bit_decode/decode_api.cpp:234-268), retuned for 256 CUs.
  * num_cus <= 0 queries the current device; returns -1 for an unsupported (bits, group_size). */

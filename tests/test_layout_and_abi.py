@@ -345,3 +345,40 @@ def test_drop_in_package_name_and_signatures():
                                          "softmax_scale", "quant_mode", "group_size", "num_bits"]
     assert sig.parameters["softmax_scale"].default == 1.0       # bit_decode_interface.py:47
     assert bit_decode.__version__ == "1.0.0.post1"              # bit_decode/__init__.py:1
+
+
+def test_cache_entries_reject_bad_arguments_without_launching():
+    header = open(os.path.join(ROOT, "include", "bitdecode.h")).read()
+    body = re.search(r"typedef struct bitdecode_cache_args \{(.*?)\} bitdecode_cache_args;", header, re.S).group(1)
+    names = [re.findall(r"[A-Za-z_][A-Za-z_0-9]*", part)[-1]
+             for decl in re.sub(r"/\*.*?\*/", "", body, flags=re.S).split(";") if decl.strip() for part in decl.split(",")]
+    assert names == [f[0] for f in _lib.CacheArgs._fields_]
+
+    def args(lengths=(100,), **kw):
+        a = _lib.CacheArgs()
+        a.k = a.v = a.k_res = a.v_res = a.k_pack = a.k_params = a.v_pack = a.v_params = a.total = 0x1000
+        a.b, a.n_tokens, a.h_k, a.d = len(lengths), 1, 8, 128
+        a.cache_tokens = 256
+        a.bits, a.group_size = 4, 128
+        a.lengths = (ctypes.c_int32 * len(lengths))(*lengths)
+        for k, v in kw.items():
+            setattr(a, k, v)
+        return a
+
+    lib = _lib.lib()
+    for entry, a, code, text in ((lib.bitdecode_cache_append, args((-1,)), 1, "length"),
+                                 (lib.bitdecode_cache_append, args((300,)), 1, "length"),
+                                 (lib.bitdecode_cache_append, args((100, 383), cache_tokens=256), 1, "sequence 1"),
+                                 (lib.bitdecode_cache_append, args(n_tokens=2), 1, "append"),
+                                 (lib.bitdecode_cache_prefill, args((2,)), 1, "length"),
+                                 (lib.bitdecode_cache_prefill, args((300,), n_tokens=400), 1, "length"),
+                                 (lib.bitdecode_cache_prefill, args(k_res=0), 1, "null"),
+                                 (lib.bitdecode_cache_prefill, args(packed_lens=0x1000), 1, "null"),
+                                 (lib.bitdecode_cache_prefill, args(v=0x1004), 1, "aligned"),
+                                 (lib.bitdecode_cache_prefill, args(kres_stride_t=4), 1, "strides"),
+                                 (lib.bitdecode_cache_prefill, args(cache_tokens=100), 1, "cache_tokens"),
+                                 (lib.bitdecode_cache_prefill, args(b=70000), 1, "batch"),
+                                 (lib.bitdecode_cache_prefill, args(bits=2, quant_mode=1), 2, "k-tensor"),
+                                 (lib.bitdecode_cache_prefill, args(d=64), 2, "head_dim")):
+        assert entry(ctypes.byref(a), None) == code, (text, lib.bitdecode_last_error())
+        assert text in lib.bitdecode_last_error().decode()
