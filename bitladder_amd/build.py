@@ -1,4 +1,4 @@
-"""Builds libbitdecode.so (hand-written HIP for gfx950) in-tree with hipcc."""
+"""Builds libbitdecode.so (hand-written HIP for gfx950) and the host extension in-tree."""
 from __future__ import annotations
 
 import os
@@ -6,6 +6,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(_HERE, "csrc")
@@ -28,6 +29,20 @@ PER_FILE = {
     "api.hip": [],
 }
 PROBE_SRC = "probe.hip"
+# host side of the drop-in calls: a Python extension over torch's tensors, no device code
+HOST_SRC = "hostpath.cpp"
+HOST_PATH = os.path.join(_HERE, "_hostpath.so")
+
+
+def host_cmd() -> list:
+    import torch
+    root = os.path.dirname(torch.__file__)
+    abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
+    return [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+            f"-D_GLIBCXX_USE_CXX11_ABI={abi}", "-isystem", os.path.join(root, "include"),
+            "-isystem", os.path.join(os.path.dirname(os.path.dirname(hipcc())), "include"),
+            "-isystem", sysconfig.get_paths()["include"], os.path.join(CSRC, HOST_SRC), "-o", HOST_PATH,
+            "-L" + os.path.join(root, "lib"), "-lc10", "-lc10_hip", "-ltorch_cpu", "-ltorch_python"]
 
 
 def hipcc() -> str:
@@ -62,6 +77,7 @@ def build(verbose: bool = False) -> str:
     if verbose:
         print(" ".join(probe_cmd), flush=True)
     probe_proc = subprocess.Popen(probe_cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    host_proc = subprocess.Popen(host_cmd(), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     for src, extra in PER_FILE.items():
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         cmd = [cc, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
@@ -77,6 +93,9 @@ def build(verbose: bool = False) -> str:
     out, _ = probe_proc.communicate()
     if probe_proc.returncode != 0:
         raise RuntimeError(f"hipcc failed on {PROBE_SRC}:\n{out}")
+    out, _ = host_proc.communicate()
+    if host_proc.returncode != 0:
+        raise RuntimeError(f"{HOST_SRC} failed:\n{out}")
     cmd = [cc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:

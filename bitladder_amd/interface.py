@@ -174,55 +174,70 @@ def _plan_cache() -> dict:
     return c
 
 
-def _call_key(tensors, scalars, kwargs):
-    """Hashable key of a drop-in call: a tensor counts by address, shape, strides and element type (the argument
-    block holds nothing else of it), everything else by value; the current stream is part of the key because
-    the workspace belongs to it."""
-    parts = []
-    for t in tensors:
-        parts.append(None if t is None else (t.data_ptr(), t.shape, t.stride(), t.dtype))
-    for name in sorted(kwargs):
-        v = kwargs[name]
-        parts.append((name, v.data_ptr(), v.shape, v.stride(), v.dtype) if isinstance(v, torch.Tensor) else (name, v))
-    dev = tensors[0].device
-    return (tuple(parts), scalars, dev.index, _stream_ptr(dev) if dev.type == "cuda" else 0)
+def _pack_cache() -> dict:
+    """The same for pack calls."""
+    c = getattr(_tls, "packs", None)
+    if c is None:
+        c = _tls.packs = {}
+    return c
 
 
-def _run_kept(key, q, kwargs, make_plan):
+_NO_KWARGS: dict = {}
+_host_run = None
+
+
+def _host():
+    """`run` of the native host path (csrc/hostpath.cpp)."""
+    global _host_run
+    if _host_run is None:
+        try:
+            from . import _hostpath
+        except ImportError as e:
+            raise ImportError("bitladder_amd/_hostpath.so is missing or does not load: build it with "
+                              "`python -m bitladder_amd.build`") from e
+        _hostpath.setup(torch.Tensor, torch.nn.Parameter, _lib.check)
+        _host_run = _hostpath.run
+    return _host_run
+
+
+def _remember(cache: dict, key: bytes, owner, args, fn, lse_shape) -> None:
+    """Keeps a validated argument block under its key (the entry's layout is hostpath.cpp's)."""
+    if len(cache) >= _MAX_PLANS:
+        cache.pop(next(iter(cache)), None)
+    out, lse = (-1, -1) if isinstance(args, _lib.QpackArgs) else (_lib.FwdArgs.out.offset, _lib.FwdArgs.softmax_lse.offset)
+    cache[key] = (owner, ctypes.addressof(args), ctypes.sizeof(args), out, lse,
+                  ctypes.cast(fn, ctypes.c_void_p).value, lse_shape)
+
+
+def _run_kept(tensors, scalars, q, kwargs, make_plan):
     """Runs a plain (non-plan) decode call.  A decode loop makes such a call again and again over the same
     memory: the validated argument block of a thread's last distinct calls (up to 512) is kept and found again by the
-    address, shape, strides and element type of every tensor, which saves 40 % of the host's time per call."""
+    address, shape, strides and element type of every tensor and the value of everything else, on the stream whose
+    workspace it holds.  Finding it, the output tensor and the launch are native code: a call
+    over 1K tokens takes the kernel's 6.7 us, 10.0 (the host's time) with the key and the output made in Python; a pack call costs
+    the host 4.3 us, 9.1 with its validation each time."""
     return_lse = kwargs.get("return_lse", False)
-    if q.is_cuda and torch.cuda.is_current_stream_capturing():
-        # Recorded into a HIP graph: the graph bakes the workspace address in and may be replayed on any stream,
-        # at any time.  The call gets a workspace of its own, allocated (and zero-filled by a fill kernel) inside
-        # the capture, so it lives in the graph's memory pool for as long as the graph does; none of the caches is used.
-        plan = make_plan(False)
-        with _on_device(plan.device):
-            plan.run()
-        return (plan.out, plan.lse) if return_lse else plan.out
-    cache = _plan_cache()
-    plan = cache.get(key)
-    if plan is None:
-        plan = make_plan(True)
-        out, lse = plan.out, plan.lse
+    key = NotImplemented
+    if q.is_cuda:
+        cache = _plan_cache()
+        key = (_host_run or _host())(cache, tensors, scalars, kwargs, False)
+        if key is not NotImplemented and type(key) is not bytes:
+            return key
+        if key is NotImplemented and torch.cuda.is_current_stream_capturing():
+            # Recorded into a HIP graph: the graph bakes the workspace address in and may be replayed on any stream,
+            # at any time.  The call gets a workspace of its own, allocated (and zero-filled by a fill kernel) inside
+            # the capture, so it lives in the graph's memory pool for as long as the graph does; none of the caches is used.
+            plan = make_plan(False)
+            with _on_device(plan.device):
+                plan.run()
+            return (plan.out, plan.lse) if return_lse else plan.out
+    plan = make_plan(True)
+    out, lse = plan.out, plan.lse
+    if key is not NotImplemented:
         # a kept plan must not keep the caller's tensors alive: it holds addresses, and its workspace
-        fwd = plan.fwd
-        plan._keep = plan._keep[-1:] if fwd.workspace else ()
+        plan._keep = plan._keep[-1:] if plan.fwd.workspace else ()
         plan.out = plan.lse = None
-        if len(cache) >= _MAX_PLANS:
-            cache.pop(next(iter(cache)))
-        cache[key] = plan
-    else:
-        fwd = plan.fwd
-        out = kwargs.get("out")
-        if out is None:         # a new output (and LSE) tensor per call, as the reference returns
-            out = torch.empty_like(q)
-            fwd.out = out.data_ptr()
-        lse = None
-        if return_lse:
-            lse = torch.empty(plan.lse_shape, dtype=torch.float32, device=q.device)
-            fwd.softmax_lse = lse.data_ptr()
+        _remember(cache, key, plan, plan.args, plan._fn, plan.lse_shape)
     with _on_device(plan.device):
         plan.run()
     return (out, lse) if return_lse else out
@@ -255,6 +270,14 @@ def kvcache_pack_int(k_cache: torch.Tensor, k_pack: torch.Tensor, k_params: torc
     `dst_offsets` (int32 [b] device tensor) give the token position, a multiple of 128, at which
     the n new tokens are written, so a full fp16 residual block can be appended to the cache.
     """
+    key = NotImplemented
+    if k_cache.is_cuda:
+        cache = _pack_cache()
+        key = (_host_run or _host())(
+            cache, (k_cache, v_cache, k_pack, k_params, v_pack, v_params, opt_block_table, cu_seqlens_k, dst_offsets),
+            (quant_mode, group_size, num_bits, dst_offset), _NO_KWARGS, True)
+        if key is None:
+            return
     mode = _check_quant(quant_mode, group_size, num_bits)
     if k_cache.dim() != 4 or v_cache.shape != k_cache.shape:
         raise RuntimeError("k_cache and v_cache must both be [batch, seqlen, nheads_k, head_dim]")
@@ -298,6 +321,8 @@ def kvcache_pack_int(k_cache: torch.Tensor, k_pack: torch.Tensor, k_params: torc
         _set_paging(a, opt_block_table, cb)
     with _on_device(device):
         _lib.check(_lib.lib().bitdecode_qpack(ctypes.byref(a), _stream_ptr(device)))
+    if key is not NotImplemented:
+        _remember(cache, key, a, a, _lib.lib().bitdecode_qpack, ())
 
 
 class DecodePlan:
@@ -487,11 +512,10 @@ def fwd_kvcache_int(q: torch.Tensor,
     if q.dim() == 4 and q.shape[1] > 1:
         return _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale, quant_mode,
                                group_size, num_bits, **kwargs)
-    key = _call_key((q, k_pack, k_params, v_pack, v_params, opt_block_table),
-                    (softmax_scale, quant_mode, group_size, num_bits), kwargs)
     # the split workspace comes from a per-stream cache: no allocation and no fill after the first call
     # (the reference allocates its accumulators per call, decode_api.cpp:292-295, 375-390)
-    return _run_kept(key, q, kwargs, lambda shared: plan_fwd_kvcache_int(
+    return _run_kept((q, k_pack, k_params, v_pack, v_params, opt_block_table),
+                     (softmax_scale, quant_mode, group_size, num_bits), q, kwargs, lambda shared: plan_fwd_kvcache_int(
         q, k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale, quant_mode, group_size, num_bits,
         _stream_ws=shared, **kwargs))
 
@@ -524,9 +548,8 @@ def _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, soft
     if out is not None:
         kwargs["out"] = out
     kwargs["return_lse"] = return_lse
-    key = _call_key((q, k_pack, k_params, v_pack, v_params, opt_block_table),
-                    (softmax_scale, quant_mode, group_size, num_bits), kwargs)
-    return _run_kept(key, q, kwargs, lambda shared: plan_fwd_kvcache_int(
+    return _run_kept((q, k_pack, k_params, v_pack, v_params, opt_block_table),
+                     (softmax_scale, quant_mode, group_size, num_bits), q, kwargs, lambda shared: plan_fwd_kvcache_int(
         q, k_pack, k_params, v_pack, v_params, opt_block_table, softmax_scale, quant_mode, group_size, num_bits,
         _stream_ws=shared, _rows=True, **kwargs))
 
@@ -606,8 +629,7 @@ def fwd_kvcache_int_append(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Te
     advances `lengths` on the device.  `max_len` is a host upper bound of `lengths` before the step (it
     sizes the grid; the capacity of the cache always works).  Keyword-only: num_splits, out, return_lse.
     """
-    key = _call_key((q, k_new, v_new, k_pack, k_params, v_pack, v_params, k_residual, v_residual, lengths,
-                     opt_block_table), ("step", max_len, softmax_scale, quant_mode, group_size, num_bits), kwargs)
-    return _run_kept(key, q, kwargs, lambda shared: plan_fwd_kvcache_int_append(
+    return _run_kept((q, k_new, v_new, k_pack, k_params, v_pack, v_params, k_residual, v_residual, lengths,
+                      opt_block_table), ("step", max_len, softmax_scale, quant_mode, group_size, num_bits), q, kwargs, lambda shared: plan_fwd_kvcache_int_append(
         q, k_new, v_new, k_pack, k_params, v_pack, v_params, k_residual, v_residual, lengths, max_len,
         opt_block_table, softmax_scale, quant_mode, group_size, num_bits, _stream_ws=shared, **kwargs))
