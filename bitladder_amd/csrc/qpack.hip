@@ -1,7 +1,7 @@
 // Quantize-pack kernel: fp16/bf16 K,V -> 2/4-bit codes + scale/zero in the gfx950 layout of
 // layout.h.  One workgroup (256 threads) packs one 128-token chunk of one (batch, kv-head) with the
-// shared chunk routine of qpack_chunk.h.  HBM-bound: reads 64 KB, writes chunk_code_bytes*2 + params
-// per chunk.
+// shared chunk routine of qpack_chunk.h, or two workgroups do where the chunks leave compute units idle.  HBM-bound:
+// reads 64 KB, writes chunk_code_bytes*2 + params per chunk.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -12,11 +12,24 @@
 namespace bitdecode {
 namespace {
 
-template <int BITS, int GS, bool BF16, bool KT, bool STREAM>
+// How a launch cuts its chunks.  Up to three rounds of workgroups over the 256 compute units a chunk's K and V go to a
+// workgroup each: twice as many in flight, and each a chain (fetch, statistics, codes, store) half as long.  Measured, us for one
+// workgroup per chunk | two, 4 bits group 128 / 4 bits group 32 / 2 bits group 128:
+//     8 chunks   6.6 | 4.5     7.6 | 5.1     6.5 | 4.4          128   8.2 | 6.2     8.9 | 6.8     7.7 | 6.0
+//   256          9.5 | 8.1    10.0 | 8.5     8.6 | 7.8          384  10.8 | 9.8    12.5 | 10.3   11.2 | 9.4
+//   512         12.9 | 11.4   14.4 | 13.5   12.8 | 11.1         640  14.0 | 13.1   16.8 | 15.8   14.9 | 12.7
+// Beyond that they are within 3 % of each other either way ("k-tensor" 2-4 % slower with two at 768-1024 chunks) and
+// one workgroup keeps its chunk.  From 512 chunks on input and output are streamed past the caches.
+enum class Cut { kSides, kSidesStream, kStream };
+Cut choose_cut(int64_t chunks) {
+    return chunks < 512 ? Cut::kSides : chunks < 768 ? Cut::kSidesStream : Cut::kStream;
+}
+
+template <int BITS, int GS, bool BF16, bool KT, Cut CUT>
 __global__ __launch_bounds__(qp::kPackThreads) void qpack_kernel(QpackParams P) {
     __shared__ qp::PackLds<GS> L;
     const int tid = threadIdx.x;
-    const int ci_src = blockIdx.x, hk = blockIdx.y, bi = blockIdx.z;
+    const int ci_src = CUT != Cut::kStream ? blockIdx.x >> 1 : blockIdx.x, hk = blockIdx.y, bi = blockIdx.z;
     const int dst_base = P.dst_offsets ? P.dst_offsets[bi] : P.dst_offset;
     if (dst_base < 0) return;       // a negative per-sequence offset skips that sequence (whole workgroup)
     const int dst_tok = dst_base + ci_src * kChunk;
@@ -28,10 +41,15 @@ __global__ __launch_bounds__(qp::kPackThreads) void qpack_kernel(QpackParams P) 
     const uint16_t* ks = P.k + bi * P.k_sb + static_cast<int64_t>(ci_src) * kChunk * P.k_st + hk * P.k_sh;
     const uint16_t* vs = P.v + bi * P.v_sb + static_cast<int64_t>(ci_src) * kChunk * P.v_st + hk * P.v_sh;
     const int64_t k_st = P.k_st, v_st = P.v_st;
+    if constexpr (CUT != Cut::kStream) {
+        qp::pack_chunk_side<BITS, GS, BF16, KT, CUT == Cut::kSidesStream>(
+            L, tid, blockIdx.x & 1, [=](int n) { return ks + n * k_st; }, [=](int n) { return vs + n * v_st; }, D);
+        return;
+    }
     // 4 bits, group 128: with the V tile prefetched the kernel needs 133 registers and only three
     // workgroups fit a CU; fetched after the K side it needs 114, a fourth workgroup fits (LDS: 40 KB
     // each) and the kernel is 10 % faster.  (At group 64 a fourth workgroup was measured 3 % slower.)
-    qp::pack_chunk<BITS, GS, BF16, !(BITS == 4 && GS == 128), KT, STREAM>(
+    qp::pack_chunk<BITS, GS, BF16, !(BITS == 4 && GS == 128), KT, true>(
         L, tid, true, [=](int n) { return ks + n * k_st; }, [=](int n) { return vs + n * v_st; }, D);
 }
 
@@ -39,13 +57,14 @@ __global__ __launch_bounds__(qp::kPackThreads) void qpack_kernel(QpackParams P) 
 // the longest prompt's last whole one (behind a shorter prompt that is padding, which no decode reads), and the one whose
 // chunk the prompt ends in copies what lies behind the prompt's last whole chunk into the fp16 window.  Same bound and same
 // chunk routine as qpack_kernel; what it saves are two copies per sequence for the windows and the upload of the lengths.
-template <int BITS, int GS, bool BF16, bool KT, bool STREAM>
+template <int BITS, int GS, bool BF16, bool KT, Cut CUT>
 __global__ __launch_bounds__(qp::kPackThreads) void cache_prefill_kernel(CacheParams P) {
     __shared__ qp::PackLds<GS> L;
     const int tid = threadIdx.x;
-    const int ci = blockIdx.x, hk = blockIdx.y, bi = P.first + blockIdx.z;
+    const int ci = CUT != Cut::kStream ? blockIdx.x >> 1 : blockIdx.x, hk = blockIdx.y, bi = P.first + blockIdx.z;
+    const bool v_side = CUT != Cut::kStream && (blockIdx.x & 1);
     const int n = P.lengths[blockIdx.z], whole = n / kChunk, rest = n % kChunk;
-    if (ci == 0 && hk == 0 && tid == 0) {
+    if (ci == 0 && hk == 0 && tid == 0 && !v_side) {
         P.total[bi] = n;
         if (P.packed_lens) {
             P.packed_lens[bi] = n - rest;
@@ -55,7 +74,7 @@ __global__ __launch_bounds__(qp::kPackThreads) void cache_prefill_kernel(CachePa
     const uint16_t* ks = P.k + bi * P.k_sb + static_cast<int64_t>(ci) * kChunk * P.k_st + hk * P.k_sh;
     const uint16_t* vs = P.v + bi * P.v_sb + static_cast<int64_t>(ci) * kChunk * P.v_st + hk * P.v_sh;
     const int64_t k_st = P.k_st, v_st = P.v_st;
-    if (ci == whole) {
+    if (ci == whole && !v_side) {
         uint16_t* kw = P.k_res + bi * P.kres_sb + hk * P.kres_sh;
         uint16_t* vw = P.v_res + bi * P.vres_sb + hk * P.vres_sh;
         const int col = (tid & 15) * 8;
@@ -68,7 +87,12 @@ __global__ __launch_bounds__(qp::kPackThreads) void cache_prefill_kernel(CachePa
     if (ci >= P.pack_chunks) return;
     const qp::ChunkDst D = qp::chunk_dst<BITS, GS, KT>(P.k_pack, P.k_params, P.v_pack, P.v_params, P.kpack_bh, P.kparams_bh,
                                                    P.vpack_bh, P.vparams_bh, ChunkPlace{static_cast<int64_t>(bi) * P.hk + hk, ci});
-    qp::pack_chunk<BITS, GS, BF16, !(BITS == 4 && GS == 128), KT, STREAM>(
+    if constexpr (CUT != Cut::kStream) {
+        qp::pack_chunk_side<BITS, GS, BF16, KT, CUT == Cut::kSidesStream>(
+            L, tid, v_side, [=](int r) { return ks + r * k_st; }, [=](int r) { return vs + r * v_st; }, D);
+        return;
+    }
+    qp::pack_chunk<BITS, GS, BF16, !(BITS == 4 && GS == 128), KT, true>(
         L, tid, true, [=](int r) { return ks + r * k_st; }, [=](int r) { return vs + r * v_st; }, D);
 }
 
@@ -99,14 +123,15 @@ __device__ __forceinline__ void append_token(const CacheParams& P, int hk, int b
 __global__ __launch_bounds__(64) void cache_append_kernel(CacheParams P) {
     append_token(P, blockIdx.x, P.first + blockIdx.y, P.lengths[blockIdx.y], threadIdx.x);
 }
-// The same when some window becomes full: its workgroups also pack it behind the prefix, 127 rows from the window and the
+// The same when some window becomes full: its workgroups, one for K and one for V, also pack it behind the prefix, 127 rows from the window and the
 // last one from the new token.
 template <int BITS, int GS, bool BF16, bool KT>
 __global__ __launch_bounds__(qp::kPackThreads) void cache_append_pack_kernel(CacheParams P) {
     __shared__ qp::PackLds<GS> L;
     const int tid = threadIdx.x, hk = blockIdx.x, bi = P.first + blockIdx.y;
     const int n = P.lengths[blockIdx.y];
-    append_token(P, hk, bi, n, tid);
+    const bool v_side = blockIdx.z != 0;
+    if (!v_side) append_token(P, hk, bi, n, tid);
     if (n % kChunk != kChunk - 1) return;
     const uint16_t* kn = P.k + bi * P.k_sb + hk * P.k_sh;
     const uint16_t* vn = P.v + bi * P.v_sb + hk * P.v_sh;
@@ -116,27 +141,28 @@ __global__ __launch_bounds__(qp::kPackThreads) void cache_append_pack_kernel(Cac
     const qp::ChunkDst D = qp::chunk_dst<BITS, GS, KT>(P.k_pack, P.k_params, P.v_pack, P.v_params, P.kpack_bh, P.kparams_bh,
                                                    P.vpack_bh, P.vparams_bh,
                                                    ChunkPlace{static_cast<int64_t>(bi) * P.hk + hk, n / kChunk});
-    qp::pack_chunk<BITS, GS, BF16, !(BITS == 4 && GS == 128), KT, false>(
-        L, tid, true, [=](int r) { return r == kChunk - 1 ? kn : kw + r * k_st; },
+    qp::pack_chunk_side<BITS, GS, BF16, KT>(
+        L, tid, v_side, [=](int r) { return r == kChunk - 1 ? kn : kw + r * k_st; },
         [=](int r) { return r == kChunk - 1 ? vn : vw + r * v_st; }, D);
 }
-
-// a bulk pack (more chunks than two rounds of workgroups over the 256 compute units) streams its input
-// and output past the caches; an append of a block per sequence does not
-constexpr int64_t kStreamChunks = 512;
 
 template <int BITS, int GS, bool BF16, bool KT>
 hipError_t launch_cache_tt(const CacheParams& P, int n, bool append, hipStream_t stream) {
     if (append) {
-        hipLaunchKernelGGL((cache_append_pack_kernel<BITS, GS, BF16, KT>), dim3(P.hk, n), dim3(qp::kPackThreads), 0, stream, P);
+        hipLaunchKernelGGL((cache_append_pack_kernel<BITS, GS, BF16, KT>), dim3(P.hk, n, 2), dim3(qp::kPackThreads), 0, stream, P);
         return hipGetLastError();
     }
     // (one workgroup more per head for the windows of the prompts that end behind the last packed chunk)
-    const dim3 grid(P.pack_chunks + 1, P.hk, n);
-    if (static_cast<int64_t>(P.pack_chunks) * P.hk * n >= kStreamChunks) {
-        hipLaunchKernelGGL((cache_prefill_kernel<BITS, GS, BF16, KT, true>), grid, dim3(qp::kPackThreads), 0, stream, P);
-    } else {
-        hipLaunchKernelGGL((cache_prefill_kernel<BITS, GS, BF16, KT, false>), grid, dim3(qp::kPackThreads), 0, stream, P);
+    const int across = P.pack_chunks + 1;
+    switch (choose_cut(static_cast<int64_t>(P.pack_chunks) * P.hk * n)) {
+        case Cut::kStream:
+            hipLaunchKernelGGL((cache_prefill_kernel<BITS, GS, BF16, KT, Cut::kStream>), dim3(across, P.hk, n), dim3(qp::kPackThreads), 0, stream, P);
+            break;
+        case Cut::kSides:
+            hipLaunchKernelGGL((cache_prefill_kernel<BITS, GS, BF16, KT, Cut::kSides>), dim3(2 * across, P.hk, n), dim3(qp::kPackThreads), 0, stream, P);
+            break;
+        default:
+            hipLaunchKernelGGL((cache_prefill_kernel<BITS, GS, BF16, KT, Cut::kSidesStream>), dim3(2 * across, P.hk, n), dim3(qp::kPackThreads), 0, stream, P);
     }
     return hipGetLastError();
 }
@@ -165,30 +191,36 @@ hipError_t launch_cache(const CacheParams& P, int n, bool append, hipStream_t st
     return hipErrorInvalidValue;
 }
 
-template <int BITS, int GS, bool KT, bool STREAM>
+template <int BITS, int GS, bool KT, Cut CUT>
 hipError_t launch_qpack_tt(const QpackParams& P, dim3 grid, hipStream_t stream) {
+    if (CUT != Cut::kStream) grid.x *= 2;
     if (P.bf16) {
-        hipLaunchKernelGGL((qpack_kernel<BITS, GS, true, KT, STREAM>), grid, dim3(256), 0, stream, P);
+        hipLaunchKernelGGL((qpack_kernel<BITS, GS, true, KT, CUT>), grid, dim3(256), 0, stream, P);
     } else {
-        hipLaunchKernelGGL((qpack_kernel<BITS, GS, false, KT, STREAM>), grid, dim3(256), 0, stream, P);
+        hipLaunchKernelGGL((qpack_kernel<BITS, GS, false, KT, CUT>), grid, dim3(256), 0, stream, P);
     }
     return hipGetLastError();
+}
+template <int BITS, int GS, bool KT>
+hipError_t launch_qpack_cut(const QpackParams& P, hipStream_t stream) {
+    const dim3 grid(P.n_tokens / kChunk, P.hk, P.b);
+    switch (choose_cut(static_cast<int64_t>(grid.x) * grid.y * grid.z)) {
+        case Cut::kStream: return launch_qpack_tt<BITS, GS, KT, Cut::kStream>(P, grid, stream);
+        case Cut::kSides: return launch_qpack_tt<BITS, GS, KT, Cut::kSides>(P, grid, stream);
+        default: return launch_qpack_tt<BITS, GS, KT, Cut::kSidesStream>(P, grid, stream);
+    }
 }
 
 template <int BITS, int GS>
 hipError_t launch_qpack_t(const QpackParams& P, hipStream_t stream) {
-    dim3 grid(P.n_tokens / kChunk, P.hk, P.b);
-    const bool stream_data = static_cast<int64_t>(grid.x) * grid.y * grid.z >= kStreamChunks;
     if (P.ktensor) {      // K quantized per token like V: 4 bits only, as in the reference (qpack.h:385)
         if constexpr (BITS == 4) {
-            return stream_data ? launch_qpack_tt<BITS, GS, true, true>(P, grid, stream)
-                               : launch_qpack_tt<BITS, GS, true, false>(P, grid, stream);
+            return launch_qpack_cut<BITS, GS, true>(P, stream);
         } else {
             return hipErrorInvalidValue;
         }
     }
-    return stream_data ? launch_qpack_tt<BITS, GS, false, true>(P, grid, stream)
-                       : launch_qpack_tt<BITS, GS, false, false>(P, grid, stream);
+    return launch_qpack_cut<BITS, GS, false>(P, stream);
 }
 
 }  // namespace

@@ -170,28 +170,13 @@ __device__ __forceinline__ void st16(void* p, u4 v) {
 // With KT ("k-tensor" mode, qpack.h:378-470 of the reference) K is quantized like V, per token over groups
 // of GS channels; its codes keep the K layout, its parameters go per chunk as
 // [64-token half][channel group][16-token tile][token] (scale, zero) pairs.
-template <int BITS, int GS, bool BF16, bool PREFETCH_V, bool KT = false, bool STREAM = false, class RowK, class RowV>
-__device__ __forceinline__ void pack_chunk(PackLds<GS>& L, int tid, bool active, RowK krow, RowV vrow,
-                                           const ChunkDst& D) {
+// (K) and (V): one tensor's side of a chunk, from the tile in LDS to the packed bytes.
+template <int BITS, int GS, bool BF16, bool KT, bool STREAM>
+__device__ __forceinline__ void pack_k_side(PackLds<GS>& L, int tid, bool active, const ChunkDst& D) {
 #pragma clang fp contract(off)
     constexpr int NG = kChunk / GS, NCG = kHeadDim / GS;
     constexpr float M = static_cast<float>((1 << BITS) - 1);
     uint16_t* const tile = L.tile;
-
-    // ---- global loads of both tiles: thread -> row tid/16 + 16*x, 16-byte column block tid%16
-    const int lrow = (tid >> 4) & 15, lcol = (tid & 15) * 8;
-    u4 kreg[8], vreg[8];
-    if (active) {
-#pragma unroll
-        for (int x = 0; x < 8; ++x) kreg[x] = ld16<STREAM>(krow(lrow + 16 * x) + lcol);
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-            if constexpr (PREFETCH_V) vreg[x] = ld16<STREAM>(vrow(lrow + 16 * x) + lcol);
-        }
-#pragma unroll
-        for (int x = 0; x < 8; ++x) *reinterpret_cast<u4*>(&tile[(lrow + 16 * x) * kRowHalves + lcol]) = kreg[x];
-    }
-    __syncthreads();
 
     // ================= K: per-channel groups of GS tokens (KT: per-token groups of GS channels) =================
     if constexpr (KT) {
@@ -297,18 +282,16 @@ __device__ __forceinline__ void pack_chunk(PackLds<GS>& L, int tid, bool active,
             st16<STREAM>(kc + tp * 1024 + l * 16, out);
         }
     }
-    __syncthreads();
+}
+
+template <int BITS, int GS, bool BF16, bool STREAM>
+__device__ __forceinline__ void pack_v_side(PackLds<GS>& L, int tid, bool active, const ChunkDst& D) {
+#pragma clang fp contract(off)
+    constexpr int NCG = kHeadDim / GS;
+    constexpr float M = static_cast<float>((1 << BITS) - 1);
+    uint16_t* const tile = L.tile;
 
     // ================= V: per-token groups of GS channels =================
-    if (active) {
-#pragma unroll
-        for (int x = 0; x < 8; ++x) {
-            if constexpr (!PREFETCH_V) vreg[x] = ld16<STREAM>(vrow(lrow + 16 * x) + lcol);
-        }
-#pragma unroll
-        for (int x = 0; x < 8; ++x) *reinterpret_cast<u4*>(&tile[(lrow + 16 * x) * kRowHalves + lcol]) = vreg[x];
-    }
-    __syncthreads();
     if (active) {
         row_group_stats<GS, BF16>(tile, tid, [&](int n, int cg, float mn, float mx) {
             const int sb = n >> 5, T = (n >> 4) & 1, q = (n >> 2) & 3, r = n & 3, i = 4 * T + r;
@@ -367,6 +350,51 @@ __device__ __forceinline__ void pack_chunk(PackLds<GS>& L, int tid, bool active,
             st16<STREAM>(vc + sb2 * 2048 + hf * 1024 + l * 16, out);
         }
     }
+}
+
+// The tile's rows, 16 bytes per thread and load: thread -> row tid/16 + 16*x, 16-byte column block tid%16
+template <bool STREAM, class Row>
+__device__ __forceinline__ void fetch_tile(u4 (&reg)[8], int tid, Row row) {
+    const int lrow = (tid >> 4) & 15, lcol = (tid & 15) * 8;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) reg[x] = ld16<STREAM>(row(lrow + 16 * x) + lcol);
+}
+__device__ __forceinline__ void stage_tile(uint16_t* tile, int tid, const u4 (&reg)[8]) {
+    const int lrow = (tid >> 4) & 15, lcol = (tid & 15) * 8;
+#pragma unroll
+    for (int x = 0; x < 8; ++x) *reinterpret_cast<u4*>(&tile[(lrow + 16 * x) * kRowHalves + lcol]) = reg[x];
+}
+
+template <int BITS, int GS, bool BF16, bool PREFETCH_V, bool KT = false, bool STREAM = false, class RowK, class RowV>
+__device__ __forceinline__ void pack_chunk(PackLds<GS>& L, int tid, bool active, RowK krow, RowV vrow,
+                                           const ChunkDst& D) {
+    u4 kreg[8], vreg[8];
+    if (active) {
+        fetch_tile<STREAM>(kreg, tid, krow);
+        if constexpr (PREFETCH_V) fetch_tile<STREAM>(vreg, tid, vrow);
+        stage_tile(L.tile, tid, kreg);
+    }
+    __syncthreads();
+    pack_k_side<BITS, GS, BF16, KT, STREAM>(L, tid, active, D);
+    __syncthreads();
+    if (active) {
+        if constexpr (!PREFETCH_V) fetch_tile<STREAM>(vreg, tid, vrow);
+        stage_tile(L.tile, tid, vreg);
+    }
+    __syncthreads();
+    pack_v_side<BITS, GS, BF16, STREAM>(L, tid, active, D);
+}
+
+// The same by two workgroups, one for K (v_side = false) and one for V: the sides share nothing but the LDS tile.
+template <int BITS, int GS, bool BF16, bool KT, bool STREAM = false, class RowK, class RowV>
+__device__ __forceinline__ void pack_chunk_side(PackLds<GS>& L, int tid, bool v_side, RowK krow, RowV vrow, const ChunkDst& D) {
+    u4 reg[8];
+    if (v_side) fetch_tile<STREAM>(reg, tid, vrow);
+    else fetch_tile<STREAM>(reg, tid, krow);
+    stage_tile(L.tile, tid, reg);
+    __syncthreads();
+    if (v_side) pack_v_side<BITS, GS, BF16, STREAM>(L, tid, true, D);
+    else pack_k_side<BITS, GS, BF16, KT, STREAM>(L, tid, true, D);
 }
 
 }  // namespace qp
