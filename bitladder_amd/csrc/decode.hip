@@ -251,41 +251,18 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
 // pm (the reverse).  Element i = 4*T + r of a sub-block is tile 2*ks + T, accumulator register r.
 // A tile's hi and lo columns hold the two parts of its scores; their sum is the score.
 //
-// Plain form: every lane adds up the 16 scores of its head and takes the 16 exponentials, the lo
-// column repeating what the hi column does.
-template <int NCG>
-__device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t hi_cols, float scale, WaveState<NCG>& st,
-                                                   h8 (&p16)[2], h8 (&pz)[2], h8 (&pm)[2]) {
-    float t[16];
-#pragma unroll
-    for (int tt = 0; tt < 4; ++tt) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r) t[4 * tt + r] = sc[tt][r] + partner(sc[tt][r]);
-    }
-    softmax_step<16, NCG>(t, scale, st, p_shift(4));
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-        u4 pw;
-#pragma unroll
-        for (int x = 0; x < 4; ++x) {
-            pw[x] = __builtin_bit_cast(uint32_t, pk_rtz(t[8 * ks + 2 * x], t[8 * ks + 2 * x + 1]));
-        }
-        p16[ks] = __builtin_bit_cast(h8, pw);
-        pz[ks] = __builtin_bit_cast(h8, pw & hi_cols);
-        pm[ks] = __builtin_bit_cast(h8, pw & ~hi_cols);
-    }
-}
-// Shared form, same values: the hi column takes sub-block 0 and the lo column sub-block 1 (eight sums
-// and exponentials per lane instead of sixteen), and the packed probabilities are exchanged
+// The hi column takes sub-block 0 and the lo column sub-block 1 (eight sums and exponentials per lane, where both doing
+// all of it would be sixteen), and the packed probabilities are exchanged
 // afterwards.  The sums of sub-block 0 are made in every lane; DPP adds that write only the two
 // upper banks of each row of 16 lanes then put the sums of sub-block 1 over them in the lo columns.
 // The compiler does not see that the asm reads MFMA results: the block takes all of them as operands,
 // so that it comes after the last MFMA, and waits out the longest MFMA-to-VALU distance itself.
-// Pays where a wave works through many units (2-4 % at 2 bits), not with one 4-bit unit per wave.
-template <int NCG>
-__device__ __forceinline__ void step_probabilities_shared(const f4 (&sc)[4], uint32_t hi_cols, float scale,
-                                                          WaveState<NCG>& st, h8 (&p16)[2], h8 (&pz)[2],
-                                                          h8 (&pm)[2]) {
+// Both columns doing all sixteen, the same bits: 2-4 % slower at 2 bits, 1-3 % where a wave has several 4-bit units (16
+// ragged sequences of 1K-8K 18.4 against 18.1 us, 6 paged ones of 10K at group 32 19.4 against 18.9, 8 query rows over 2 x 8K
+// 15.4 against 15.0), equal with one 4-bit unit per wave.
+template <int BITS, int NCG>
+__device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t hi_cols, float scale, WaveState<NCG>& st,
+                                                   h8 (&p16)[2], h8 (&pz)[2], h8 (&pm)[2]) {
     float t[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) t[i] = sc[i / 4][i % 4] + partner(sc[i / 4][i % 4]);
@@ -307,7 +284,7 @@ __device__ __forceinline__ void step_probabilities_shared(const f4 (&sc)[4], uin
                    "=&v"(mx)
                  : "v"(sc[2][0]), "v"(sc[2][1]), "v"(sc[2][2]), "v"(sc[2][3]), "v"(sc[3][0]), "v"(sc[3][1]),
                    "v"(sc[3][2]), "v"(sc[3][3]));
-    softmax_step<8, NCG, true>(t, scale, st, mx, p_shift(2));
+    softmax_step<8, NCG, true>(t, scale, st, mx, p_shift(BITS));
     u4 pw;
 #pragma unroll
     for (int x = 0; x < 4; ++x) pw[x] = __builtin_bit_cast(uint32_t, pk_rtz(t[2 * x], t[2 * x + 1]));
@@ -797,11 +774,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
 
         static_assert(TPS == 4 && NKS == 2, "four tiles, two sub-blocks per step");
         h8 p16[NKS], pz[NKS], pm[NKS];
-        if constexpr (BITS == 2) {
-            step_probabilities_shared<NCG>(sc, hi_cols, P.scale_log2, st, p16, pz, pm);
-        } else {
-            step_probabilities<NCG>(sc, hi_cols, P.scale_log2, st, p16, pz, pm);
-        }
+        step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pz, pm);
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) st.l = mfma32(ones, pz[ks], st.l);
         // V side of the step, row by row.  A row holds one channel half (tiles ct = 4*hf .. 4*hf+3) of one
