@@ -206,8 +206,9 @@ __device__ __forceinline__ float colmax(float x) {
 template <int NCG>
 struct WaveState {
     float m;          // running max of the raw scores (q.k units) of this lane's head
+    // (l and ob: an MFMA makes all four rows alike; only row 0 is kept in step with the maximum and read)
     f4 l;             // sum of p, accumulated by MFMA against a ones operand (hi columns only)
-    f4 ob[NCG];       // V bias per channel group, accumulated by MFMA (all four rows equal)
+    f4 ob[NCG];       // V bias per channel group, accumulated by MFMA
     f4 o[8];          // O^T tiles: lane (head, q) holds channels 16*ct + 4*q + r
 };
 
@@ -226,9 +227,9 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
             // (not in a wave's first step, which has nothing to rescale: 512 to 8K tokens of one sequence, one unit per wave,
             // 0.12 us of 6.0 to 7.3)
             const float alpha = __builtin_amdgcn_exp2f((st.m - m_use) * scale);
-            st.l *= alpha;
+            st.l[0] *= alpha;
 #pragma unroll
-            for (int c = 0; c < NCG; ++c) st.ob[c] *= alpha;
+            for (int c = 0; c < NCG; ++c) st.ob[c][0] *= alpha;
 #pragma unroll
             for (int ct = 0; ct < 8; ++ct) st.o[ct] *= alpha;
         }
@@ -1659,12 +1660,12 @@ void fwd_splitkv_kernel(FwdParams P) {
     const uint32_t lo_words = static_cast<uint32_t>(P.nsplit) * P.b * n_h * kPartialWords;
     const uint32_t slot_words = (lo_words / kPartialWords * (2 * kPartialWords + 2) + 63) / 64 * 64;
     // ---- merge the waves of this workgroup through LDS (each wave's slot is its own region)
-    const float lsum = st.l[0] + partner(st.l[0]);      // rows are equal; lo columns hold 0
+    const float lsum = st.l[0] + partner(st.l[0]);      // lo columns hold 0
 #pragma unroll
     for (int ct = 0; ct < 8; ++ct) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float v = st.o[ct][r] + st.ob[ct / (GS / 16)][r];
+            const float v = st.o[ct][r] + st.ob[ct / (GS / 16)][0];
             st.o[ct][r] = v + partner(v);      // hi + lo
         }
     }
