@@ -532,8 +532,9 @@ def _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, soft
         raise ValueError("out must match q in shape, dtype and device")
     if q.stride(3) != 1 or q.data_ptr() % 16 or any(s % 8 for s in q.stride()[:3]):
         q = q.contiguous()
-    # the workspace holds a record per row, head and split: many rows of a large batch go in several launches
-    per = max(1, 32768 // max(1, b * h))
+    # the workspace holds a record of 1040 bytes per row, head and split, below 2 GiB in all, and a launch takes at most 4096
+    # rows: more than that goes in several launches
+    per = max(1, min(4096, min(32768, 2000000 // max(1, int(kwargs.get("num_splits", 0)))) // max(1, b * h)))
     if m > per or (out is not None and out.stride(3) != 1):
         res = out if out is not None else torch.empty_like(q)
         parts = []

@@ -51,3 +51,22 @@ def test_rows_equal_the_calls_for_each_row(device, h, h_k, m, bits, gs, mode, dt
         err = (out[:, r:r + 1].float() - one.float()).abs()
         assert (err <= 1e-3 + (2 ** -8 * one.float().abs() if dtype == "bf16" else 0)).all(), (r, err.max().item())
         assert (lse[:, r] - lse1).abs().max().item() < 1e-4, r
+
+
+@pytest.mark.parametrize("m,h,num_splits", [(4100, 1, 0), (1030, 4, 512)])
+def test_more_rows_than_one_launch_takes(device, m, h, num_splits):
+    """More rows than a launch accepts, and more records than its workspace may hold: several launches, the same rows."""
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
+    g = torch.Generator(device=device).manual_seed(m)
+    k, v = (torch.randn((1, 256, 1, 128), generator=g, device=device).half() for _ in range(2))
+    cache = H.alloc_cache(1, 256, 1, 4, 128, device)
+    kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, 256, "k-channel", 128, 4)
+    q = torch.randn((1, m, h, 128), generator=g, device=device).half()
+    out, lse = fwd_kvcache_int(q, *cache, None, 0.09, "k-channel", 128, 4, num_splits=num_splits, return_lse=True)
+    assert out.shape == q.shape and lse.shape == (1, m, h)
+    for r0 in (0, m // 2, m - 8):
+        want, wlse = fwd_kvcache_int(q[:, r0:r0 + 8].contiguous(), *cache, None, 0.09, "k-channel", 128, 4,
+                                     num_splits=min(num_splits, 2), return_lse=True)
+        # (other split counts round the partial outputs differently: one fp16 rounding of a mean of unit normals)
+        assert (out[:, r0:r0 + 8].float() - want.float()).abs().max() < 2e-3
+        assert (lse[:, r0:r0 + 8] - wlse).abs().max() < 1e-4
