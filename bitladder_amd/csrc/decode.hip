@@ -1404,7 +1404,7 @@ constexpr int fwd_lds_bytes() {
 // waves of the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; they are
 // neighbours on one XCD, so all but the first find them in its L2.  (Before, the rows were folded into the head dimension
 // on the host, 8 / g rows per launch, the cache read once per launch: eight rows of 32 / 8 heads over 2 x 8K tokens took
-// four launches and eight copies, 112 us; one launch takes 15.3.)
+// four launches and eight copies, 112 us; one launch takes 15.1.)
 template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, bool ROWS>
 // (second bound: waves per SIMD the register count has to leave room for.  Two workgroups of the 8-wave kernels share
 // a compute unit when sequences differ in length, 4 waves per SIMD like the 16-wave kernels: 128 registers.  The

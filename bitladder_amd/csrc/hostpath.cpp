@@ -6,7 +6,7 @@
 // per call is the key, the output tensor and the launch.  In Python that took 6.6 us next to the launch's 3.4 (the key alone
 // 2.8: address, shape, strides and element type of up to ten tensors), more than the kernel of a short context runs.
 // Calls in a row, kernel included: 1K tokens of one sequence 10.0 -> 6.7 us, 4K tokens of 32 kv heads 10.3 -> 7.3, a block
-// packed for each of 16 sequences 9.5 -> 7.3 (its own time on the host 9.1 -> 4.3).
+// packed for each of 16 sequences 9.5 -> 7.3, 5.2 with the pack kernel as it is now (its own time on the host 9.1 -> 4.3).
 //
 //   run(cache, tensors, scalars, kwargs, any_time)
 //

@@ -100,7 +100,7 @@ __global__ __launch_bounds__(qp::kPackThreads) void cache_prefill_kernel(CachePa
 // thread per sequence counts it.  A few kilobytes: a launch and one round trip to memory, whatever the batch.  (As torch
 // operations: two indexed stores of 5.5 us, an addition, and three uploads of integers that each wait for the stream.
 // 8 prompts of 1K-8K tokens and 8 tokens each by append and decode: 911 us before, 300 with this and the prefill above;
-// 4 prompts of 700-2000 tokens and 16 decode steps: 307 and 240.)
+// 4 prompts of 700-2000 tokens and 16 decode steps: 307 and 240; 247 and 158 with the native host path.)
 __device__ __forceinline__ void append_token(const CacheParams& P, int hk, int bi, int n, int tid) {
     const int r = n % kChunk;
     if (tid < 32) {
