@@ -123,7 +123,10 @@ class BitKVCache:
 
     def _device_lengths(self):
         """Packed and window lengths as device tensors: those the last write left if the host's lengths are still theirs
-        and the stream is the one that wrote them (their memory belongs to it), else uploaded."""
+        and the stream is the one that wrote them (their memory belongs to it), else uploaded.  Not under capture: a
+        graph would keep the addresses of arrays that later writes free or change, and an upload cannot be recorded."""
+        if self.total.is_cuda and torch.cuda.is_current_stream_capturing():
+            raise RuntimeError("decode takes its lengths from the host and cannot be captured: capture a plan_step plan")
         if self._published is not None:
             packed, res, stream, host_packed, host_res = self._published
             if host_packed == self.packed_len and host_res == self.res_len and _stream_ptr(packed.device) == stream:

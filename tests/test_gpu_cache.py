@@ -79,3 +79,29 @@ def test_cache_capacity_is_enforced(device):
     with pytest.raises(ValueError):
         cache.prefill(torch.zeros((1, 256, 1, 128), dtype=torch.float16, device=device),
                       torch.zeros((1, 256, 1, 128), dtype=torch.float16, device=device))
+
+
+def test_decode_is_refused_under_capture(device):
+    """The lengths of a decode are the host's at the time of the call; a graph would replay addresses of length arrays that
+    the next append replaces.  Captured on the stream of the writes, where those arrays would be at hand."""
+    from bitladder_amd import BitKVCache
+    stream = torch.cuda.Stream(device)
+    k = torch.randn((2, 130, 2, 128), device=device).half()
+    q = torch.randn((2, 1, 8, 128), device=device).half()
+    cache = BitKVCache(2, 2, 256, device=device)
+    torch.cuda.synchronize()
+    with torch.cuda.stream(stream):
+        cache.prefill(k, k, [130, 70])
+        cache.append(k[:, :1], k[:, :1])
+        before = cache.decode(q, SCALE)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        copy = q + 0
+        with pytest.raises(RuntimeError, match="captured"):
+            cache.decode(q, SCALE)
+    graph.replay()
+    torch.cuda.synchronize()
+    assert torch.equal(copy, q)
+    with torch.cuda.stream(stream):      # the cache goes on as before
+        assert torch.equal(cache.decode(q, SCALE), before)
+    stream.synchronize()
