@@ -11,7 +11,8 @@
 //   run(cache, tensors, scalars, kwargs, any_time)
 //
 // hit: launches and returns the output (or (output, lse); None for a call without one).  miss: returns the key, under
-// which the caller stores an entry.  NotImplemented: an argument of another kind (a tensor subclass, say) or, unless
+// which the caller stores an entry.  NotImplemented: an argument of another kind (a tensor subclass, a number given as a
+// tensor: its value may be another one at the same address the next time) or, unless
 // `any_time`, a stream that is being captured; the caller then goes the long way.
 //
 // An entry is the tuple (owner, address of the block, its bytes, offset of its output pointer or -1, offset of its lse
@@ -47,11 +48,19 @@ bool plain_tensor(PyObject* o) {
     return reinterpret_cast<PyObject*>(Py_TYPE(o)) == g_tensor_type || reinterpret_cast<PyObject*>(Py_TYPE(o)) == g_parameter_type;
 }
 
-// appends what the argument block takes from the value; false: not a kind that is known here
-bool put_value(std::string& key, PyObject* o) {
+// keyword arguments that are tensors to the kernel (another one given as a tensor is a number, read on the host)
+bool names_tensor(PyObject* name) {
+    for (const char* n : {"out", "seqlens_k", "k_residual", "v_residual", "residual_len"})
+        if (PyUnicode_CompareWithASCIIString(name, n) == 0) return true;
+    return false;
+}
+
+// appends what the argument block takes from the value: of a tensor its address and form, so `tensor` only where the block
+// holds no number read from it; false: not a kind that is known here
+bool put_value(std::string& key, PyObject* o, bool tensor = false) {
     if (o == Py_None) {
         key.push_back('n');
-    } else if (plain_tensor(o)) {
+    } else if (tensor && plain_tensor(o)) {
         const at::Tensor& t = THPVariable_Unpack(o);
         if (t.layout() != at::kStrided || !t.has_storage()) return false;
         key.push_back('t');
@@ -114,13 +123,13 @@ PyObject* run(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     key.reserve(1024);
     put(key, stream);
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(tensors); ++i)
-        if (!put_value(key, PyTuple_GET_ITEM(tensors, i))) Py_RETURN_NOTIMPLEMENTED;
+        if (!put_value(key, PyTuple_GET_ITEM(tensors, i), true)) Py_RETURN_NOTIMPLEMENTED;
     for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(scalars); ++i)
         if (!put_value(key, PyTuple_GET_ITEM(scalars, i))) Py_RETURN_NOTIMPLEMENTED;
     PyObject *name = nullptr, *value = nullptr, *out = nullptr;
     bool want_lse = false;
     for (Py_ssize_t pos = 0; PyDict_Next(kwargs, &pos, &name, &value);) {
-        if (!put_value(key, name) || !put_value(key, value)) Py_RETURN_NOTIMPLEMENTED;
+        if (!put_value(key, name) || !put_value(key, value, names_tensor(name))) Py_RETURN_NOTIMPLEMENTED;
         if (PyUnicode_CompareWithASCIIString(name, "out") == 0) out = value == Py_None ? nullptr : value;
         if (PyUnicode_CompareWithASCIIString(name, "return_lse") == 0) want_lse = PyObject_IsTrue(value) == 1;
     }

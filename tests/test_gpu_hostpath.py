@@ -114,3 +114,40 @@ def test_pack_calls_found_again_and_captured(device):
             assert torch.equal(x[0, :, 1:], y[0, :, 1:]) and torch.equal(x[1, :, :3], y[1, :, :3])
     with pytest.raises(RuntimeError):
         kvcache_pack_int(kd[:, :100], *other[:2], vd[:, :100], *other[2:], None, None, 100, "k-channel", 128, 4)
+
+
+def test_numbers_given_as_tensors_are_read_with_every_call(device):
+    """A number may be a tensor of one element; another value at the same address is another call."""
+    import numpy as np
+    from bitladder_amd import fwd_kvcache_int, fwd_kvcache_int_append, kvcache_pack_int
+    q, kd, vd, cache = _setup(device)
+    number, whole = np.zeros(1), np.zeros(1, dtype=np.int64)
+
+    def given(x):      # a new tensor object over the same memory
+        (whole if isinstance(x, int) else number)[0] = x
+        return torch.from_numpy(whole if isinstance(x, int) else number).reshape(())
+
+    for scale in (SCALE, 2 * SCALE):
+        assert torch.equal(fwd_kvcache_int(q, *cache, None, given(scale), "k-channel", 128, 4),
+                           fwd_kvcache_int(q, *cache, None, scale, "k-channel", 128, 4))
+        assert torch.equal(fwd_kvcache_int(q.repeat(1, 3, 1, 1), *cache, None, given(scale), "k-channel", 128, 4),
+                           fwd_kvcache_int(q.repeat(1, 3, 1, 1), *cache, None, scale, "k-channel", 128, 4))
+    for n in (256, 512):
+        assert torch.equal(fwd_kvcache_int(q, *cache, None, SCALE, "k-channel", 128, 4, seqlen_k=given(n)),
+                           fwd_kvcache_int(q, *cache, None, SCALE, "k-channel", 128, 4, seqlen_k=n))
+    got, want = H.alloc_cache(2, 512, 2, 4, 128, device), H.alloc_cache(2, 512, 2, 4, 128, device)
+    for offset in (128, 256):
+        for dst, x in ((got, given(offset)), (want, offset)):
+            kvcache_pack_int(kd[:, :128], dst[0], dst[1], vd[:, :128], dst[2], dst[3], None, None, 0, "k-channel", 128, 4,
+                             dst_offset=x)
+    for a, b in zip(got, want):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16))
+    new = kd[:, :1].contiguous()
+    window = torch.zeros((2, 128, 2, 128), dtype=torch.float16, device=device)
+    for bound in (384, 512):
+        outs = []
+        for x in (given(bound), bound):
+            lengths = torch.tensor([300, 130], dtype=torch.int32, device=device)
+            outs.append(fwd_kvcache_int_append(q, new, new, *cache, window, window, lengths, x, None, SCALE, "k-channel",
+                                               128, 4))
+        assert torch.equal(*outs)
