@@ -82,7 +82,7 @@ bool put_value(std::string& key, PyObject* o, bool tensor = false) {
         if (overflow) return false;
         key.push_back('i');
         put(key, v);
-    } else if (PyUnicode_CheckExact(o)) {
+    } else if (PyUnicode_Check(o)) {
         Py_ssize_t n = 0;
         const char* s = PyUnicode_AsUTF8AndSize(o, &n);
         if (!s) {
@@ -92,6 +92,19 @@ bool put_value(std::string& key, PyObject* o, bool tensor = false) {
         key.push_back('s');
         put(key, n);
         key.append(s, n);
+    } else if (!THPVariable_Check(o) && PyIndex_Check(o)) {      // a whole number of another type (numpy's, an enum's)
+        THPObjectPtr whole(PyNumber_Index(o));
+        if (whole && PyLong_CheckExact(whole.get())) return put_value(key, whole.get());
+        PyErr_Clear();
+        return false;
+    } else if (!THPVariable_Check(o) && PyNumber_Check(o)) {      // a fraction of another type
+        THPObjectPtr fraction(PyNumber_Float(o));
+        if (!fraction) {
+            PyErr_Clear();
+            return false;
+        }
+        key.push_back('g');
+        put(key, PyFloat_AS_DOUBLE(fraction.get()));
     } else {
         return false;
     }

@@ -151,3 +151,23 @@ def test_numbers_given_as_tensors_are_read_with_every_call(device):
             outs.append(fwd_kvcache_int_append(q, new, new, *cache, window, window, lengths, x, None, SCALE, "k-channel",
                                                128, 4))
         assert torch.equal(*outs)
+
+
+def test_numbers_of_other_libraries_are_found_again_by_value(device):
+    import enum
+    import numpy as np
+    from bitladder_amd import fwd_kvcache_int, interface
+
+    class Mode(str, enum.Enum):
+        CHANNEL = "k-channel"
+
+    q, kd, vd, cache = _setup(device)
+    for kind in (np.float32, np.float16):
+        interface._plan_cache().clear()
+        for _ in range(3):
+            for scale in (0.125, 0.25):
+                got = fwd_kvcache_int(q, *cache, None, kind(scale), Mode.CHANNEL, np.int64(128), np.int32(4), seqlen_k=np.int64(256))
+                assert torch.equal(got, fwd_kvcache_int(q, *cache, None, scale, "k-channel", 128, 4, seqlen_k=256))
+        assert len(interface._plan_cache()) == 4      # two scales, each in two types
+    with pytest.raises((TypeError, ValueError)):
+        fwd_kvcache_int(q, *cache, None, 1j, "k-channel", 128, 4)
