@@ -62,7 +62,8 @@ class BitKVCache:
         self.res_len = [0] * batch
         self.total = torch.zeros(batch, dtype=torch.int32, device=dev)     # tokens held, as `step` needs them
         self._rows = torch.arange(batch, device=dev)
-        # packed and window lengths on the device as the last `prefill` or `append` left them (_publish_lengths)
+        # packed and window lengths on the device as the last write left them: [packed, window, stream, and the host's
+        # lists of the same lengths] (_write, _device_lengths)
         self._published = None
 
     # ------------------------------------------------------------------ lengths
@@ -106,10 +107,7 @@ class BitKVCache:
         a.vres_stride_b, a.vres_stride_t, a.vres_stride_h = vr.stride()[:3]
         a.k_pack, a.k_params = self.k_pack.data_ptr(), self.k_params.data_ptr()
         a.v_pack, a.v_params = self.v_pack.data_ptr(), self.v_params.data_ptr()
-        # new arrays with every call: an earlier `decode` may still be reading the old ones on another stream
-        packed = torch.empty(b, dtype=torch.int32, device=device)
-        res = torch.empty_like(packed)
-        a.total, a.packed_lens, a.res_lens = self.total.data_ptr(), packed.data_ptr(), res.data_ptr()
+        a.total = self.total.data_ptr()
         a.lengths = (ctypes.c_int32 * b)(*lengths)
         a.b, a.n_tokens, a.h_k, a.d = b, k.shape[1], h_k, 128
         a.cache_tokens = S
@@ -117,9 +115,22 @@ class BitKVCache:
         a.quant_mode = _lib.K_TENSOR if self.quant_mode == "k-tensor" else _lib.K_CHANNEL
         with _on_device(device):
             stream = _stream_ptr(device)
+            # The same arrays from write to write: a cache per layer then finds its `decode` calls again, whose key holds
+            # the addresses.  Only calls on the stream that writes them read them (_device_lengths), so they may be
+            # written over; another stream gets arrays of its own.  The record is one list, changed in place, for all
+            # copies of the cache that share the arrays.
+            record = self._published
+            if record is None or record[2] != stream or record[0].device != device or record[0].shape != (b,):
+                record = self._published = [torch.empty(b, dtype=torch.int32, device=device),
+                                            torch.empty(b, dtype=torch.int32, device=device), stream, None, None]
+            a.packed_lens, a.res_lens = record[0].data_ptr(), record[1].data_ptr()
+            record[3] = record[4] = None      # (until the caller says which lengths they are)
             _lib.check(getattr(_lib.lib(), entry)(ctypes.byref(a), stream))
-        self._published = (packed, res, stream)      # (the caller adds the host's lengths)
         return True
+
+    def _publish(self) -> None:
+        """The arrays of the write just made hold the host's lengths."""
+        self._published[3:] = [list(self.packed_len), list(self.res_len)]
 
     def _device_lengths(self):
         """Packed and window lengths as device tensors: those the last write left if the host's lengths are still theirs
@@ -146,7 +157,7 @@ class BitKVCache:
         self.packed_len = [x // BLOCK * BLOCK for x in lengths]
         self.res_len = [x - p for x, p in zip(lengths, self.packed_len)]
         if self._write("bitdecode_cache_prefill", k, v, lengths):
-            self._published += (list(self.packed_len), list(self.res_len))
+            self._publish()
             return
         n_pack = max(self.packed_len)
         if n_pack:
@@ -171,7 +182,7 @@ class BitKVCache:
             if self._write("bitdecode_cache_append", k1, v1, self.lengths):
                 self.packed_len = [p + BLOCK if r == BLOCK - 1 else p for p, r in zip(self.packed_len, self.res_len)]
                 self.res_len = [(r + 1) % BLOCK for r in self.res_len]
-                self._published += (list(self.packed_len), list(self.res_len))
+                self._publish()
                 return
         if k_new.dim() == 4:
             k_new, v_new = k_new[:, 0], v_new[:, 0]

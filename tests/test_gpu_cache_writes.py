@@ -83,3 +83,50 @@ def test_prefill_of_whole_tensors_restarts_the_cache(device):
     assert cache.lengths == [64, 64] and cache.total.tolist() == [64, 64] and torch.equal(cache.k_res[:, :64], k[:, :64])
     with pytest.raises(ValueError):
         cache.prefill(torch.zeros((2, 300, 2, 128), device=device).half(), torch.zeros((2, 300, 2, 128), device=device).half())
+
+
+def test_a_cache_per_layer_finds_its_decode_calls_again(device):
+    """The device lengths of a cache keep their place from token to token, so a call is another one only when the bound of
+    its packed length changes; on another stream they are other arrays."""
+    from bitladder_amd import BitKVCache, interface
+    layers, tokens = 6, 40
+    k, q = torch.randn((2, 110, 2, 128), device=device).half(), torch.randn((2, 1, 4, 128), device=device).half()
+    caches = [BitKVCache(2, 2, 256, device=device) for _ in range(layers)]
+    interface._plan_cache().clear()
+    for c in caches:
+        c.prefill(k, k, [110, 30])
+    for t in range(tokens):
+        outs = []
+        for c in caches:
+            c.append(k[:, t:t + 1], k[:, t:t + 1])
+            outs.append(c.decode(q))
+            assert [x.tolist() for x in c._device_lengths()] == [c.packed_len, c.res_len]
+        assert all(torch.equal(o, outs[0]) for o in outs)
+    assert len(interface._plan_cache()) == 2 * layers      # below and from 128 tokens on
+    first = caches[0]._device_lengths()[0]
+    side = torch.cuda.Stream(device)
+    side.wait_stream(torch.cuda.current_stream(device))
+    with torch.cuda.stream(side):
+        assert caches[0]._device_lengths()[0] is not first
+        caches[0].append(k[:, :1], k[:, :1])
+        assert caches[0]._device_lengths()[0] is not first
+        got = caches[0].decode(q)
+    side.synchronize()
+    caches[1].append(k[:, :1], k[:, :1])
+    assert first.tolist() == [128, 0] and torch.equal(got, caches[1].decode(q))
+
+
+def test_a_copy_of_a_cache_keeps_its_own_lengths(device):
+    """A shallow copy shares the tensors: the writes of one leave the other's decode at its own lengths."""
+    import copy
+    from bitladder_amd import BitKVCache
+    k, q = torch.randn((2, 110, 2, 128), device=device).half(), torch.randn((2, 1, 4, 128), device=device).half()
+    cache = BitKVCache(2, 2, 256, device=device)
+    cache.prefill(k, k, [90, 30])
+    before, fork = cache.decode(q), copy.copy(cache)
+    for t in range(3):
+        cache.append(k[:, t:t + 1], k[:, t:t + 1])
+        assert torch.equal(fork.decode(q), before)
+    after, deep = cache.decode(q), copy.deepcopy(cache)
+    cache.append(k[:, :1], k[:, :1])
+    assert torch.equal(deep.decode(q), after) and deep.lengths == [93, 33]
