@@ -34,6 +34,10 @@ class BitKVCache:
     `res_len[i] < 128` after every call.
     """
 
+    # packed and window lengths on the device as the last write left them: [packed, window, stream, and the host's lists of
+    # the same lengths] (_write, _device_lengths); of the class, for caches that were saved before there were any
+    _published: Optional[list] = None
+
     def __init__(self, batch: int, kv_heads: int, max_tokens: int, *, num_bits: int = 4, group_size: int = 128,
                  dtype: torch.dtype = torch.float16, device="cuda", head_dim: int = 128,
                  quant_mode: str = "k-channel"):
@@ -62,9 +66,6 @@ class BitKVCache:
         self.res_len = [0] * batch
         self.total = torch.zeros(batch, dtype=torch.int32, device=dev)     # tokens held, as `step` needs them
         self._rows = torch.arange(batch, device=dev)
-        # packed and window lengths on the device as the last write left them: [packed, window, stream, and the host's
-        # lists of the same lengths] (_write, _device_lengths)
-        self._published = None
 
     # ------------------------------------------------------------------ lengths
     @property
