@@ -79,8 +79,8 @@ class BitKVCache:
     def _write(self, entry: str, k: torch.Tensor, v: torch.Tensor, lengths: list[int]) -> bool:
         """`prefill` or `append` in one launch: tokens k / v [b, n, h_k, 128], lengths per sequence, to the packed cache,
         the window, `total` and a new pair of device length arrays.  False if the tensors are not what the kernels take
-        (another element type than the cache's, unaligned or strided rows, a capture in progress, no GPU): the caller then
-        works with torch operations."""
+        (another element type than the cache's, unaligned or strided rows, a capture in progress, no GPU) or the cache is one
+        that they do not: the caller then works with torch operations."""
         kr, vr = self.k_res, self.v_res
         if (not kr.is_cuda or self.b < 1 or k.dim() != 4 or k.shape != v.shape or k.shape[0] != self.b or
                 k.shape[2] != self.h_k or k.shape[3] != 128 or kr.shape != (self.b, BLOCK, self.h_k, 128) or
@@ -88,6 +88,9 @@ class BitKVCache:
                 self.total.stride(0) != 1):
             return False
         device, dtype = kr.device, kr.dtype
+        if (self.b > 65535 or not 0 < self.h_k <= 65535 or self.capacity == 0 or self.bits not in (2, 4) or
+                self.gs not in (32, 64, 128) or dtype not in (torch.float16, torch.bfloat16)):
+            return False
         args = (k, v, kr, vr)
         for t in args:
             st = t.stride()

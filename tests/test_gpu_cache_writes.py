@@ -130,3 +130,25 @@ def test_a_copy_of_a_cache_keeps_its_own_lengths(device):
     after, deep = cache.decode(q), copy.deepcopy(cache)
     cache.append(k[:, :1], k[:, :1])
     assert torch.equal(deep.decode(q), after) and deep.lengths == [93, 33]
+
+
+def test_caches_that_the_kernels_do_not_take_are_written_by_torch_operations(device):
+    """More sequences than the kernels' limit, no capacity, and formats without a decode, whose windows can be filled."""
+    from bitladder_amd import BitKVCache
+    many = BitKVCache(70000, 1, 128, device=device)
+    k = torch.randn((70000, 1, 1, 128), device=device).half()
+    many.append(k, k)
+    assert many.lengths == [1] * 70000 and torch.equal(many.k_res[:, :1], k)
+    # (one key: the output is its value, rounded once more)
+    assert (many.decode(k).float() - k.float()).abs().max() < 2 ** -9
+    empty = BitKVCache(2, 1, 0, device=device)
+    empty.prefill(k[:2], k[:2], [0, 0])
+    assert empty.lengths == [0, 0] and not empty.decode(k[:2]).any()
+    with pytest.raises(ValueError):
+        empty.append(k[:2], k[:2])
+    for options in (dict(dtype=torch.float32), dict(num_bits=8), dict(group_size=16)):
+        c = BitKVCache(2, 1, 128, device=device, **options)
+        x = k[:2].to(c.dtype)
+        c.prefill(x, x)
+        c.append(x, x)
+        assert c.lengths == [2, 2] == c.total.tolist() and torch.equal(c.k_res[:, 1:2], x)
