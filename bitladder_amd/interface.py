@@ -531,7 +531,8 @@ def _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, soft
     if out is not None and (out.shape != q.shape or out.dtype != q.dtype or out.device != q.device):
         raise ValueError("out must match q in shape, dtype and device")
     if q.stride(3) != 1 or q.data_ptr() % 16 or any(s % 8 for s in q.stride()[:3]):
-        q = q.contiguous()
+        # (a copy in any case: contiguous() returns a tensor whose only odd stride is that of a dimension of one)
+        q = q.clone(memory_format=torch.contiguous_format)
     # the workspace holds a record of 1040 bytes per row, head and split, below 2 GiB in all, and a launch takes at most 4096
     # rows: more than that goes in several launches
     per = max(1, min(4096, min(32768, 2000000 // max(1, int(kwargs.get("num_splits", 0)))) // max(1, b * h)))

@@ -70,3 +70,28 @@ def test_more_rows_than_one_launch_takes(device, m, h, num_splits):
         # (other split counts round the partial outputs differently: one fp16 rounding of a mean of unit normals)
         assert (out[:, r0:r0 + 8].float() - want.float()).abs().max() < 2e-3
         assert (lse[:, r0:r0 + 8] - wlse).abs().max() < 1e-4
+
+
+def test_rows_of_any_stride_and_alignment(device):
+    """q as the reference's own reshape takes it: whatever the strides, also those of dimensions of one."""
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
+    g = torch.Generator(device=device).manual_seed(3)
+    k, v = (torch.randn((1, 256, 2, 128), generator=g, device=device).half() for _ in range(2))
+    cache = H.alloc_cache(1, 256, 2, 4, 128, device)
+    kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, 256, "k-channel", 128, 4)
+    args = (*cache, None, SCALE, "k-channel", 128, 4)
+    want = None
+    data = torch.randn((1, 3, 4, 128), generator=g, device=device).half()
+    flat = torch.zeros(8192, dtype=torch.float16, device=device)
+    for offset, strides in ((0, (1536, 512, 128, 1)), (0, (1541, 512, 128, 1)), (1, (1536, 512, 128, 1)),
+                            (0, (1536, 516, 129, 1)), (0, (1536, 1024, 256, 2)), (0, (1536, 128, 384, 1))):
+        q = flat.as_strided(data.shape, strides, offset)
+        q.copy_(data)
+        out = fwd_kvcache_int(q, *args)
+        want = out if want is None else want
+        assert torch.equal(out, want), (offset, strides)
+        held = torch.full((8192,), 7.0, dtype=torch.float16, device=device)
+        given = held.as_strided(data.shape, strides, offset)
+        assert fwd_kvcache_int(q, *args, out=given) is given and torch.equal(given, want)
+        given.fill_(7.0)
+        assert (held == 7.0).all()
