@@ -425,6 +425,9 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     const int cus = query_cus();
     if (nsplit == 0)
         nsplit = choose_splits_for(a->b, a->h_k * row_blocks, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k && !step);
+    // (the built-in scratch takes every call that leaves the count to the library: it chooses no more than fits)
+    while (static_scratch && a->num_splits == 0 && nsplit > 1 && slots_bytes(a->b, n_h, nsplit) > kStaticScratchBytes - kStaticCounterBytes)
+        --nsplit;
     if (nsplit > 1 && slots_bytes(a->b, n_h, nsplit) >= (size_t(1) << 31))
         return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d heads: partial outputs of 2 GiB or more", nsplit, a->b, n_h);
     // the kernel divides workgroup ids and unit counts by the split count and the head count with a

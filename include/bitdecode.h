@@ -129,7 +129,7 @@ int bitdecode_fwd(const bitdecode_fwd_args* args, void* stream);
  * arrival counters live in an 8 MiB array inside the library's code object (one copy per GPU, held until the
  * process ends), and the call allocates nothing.  Limits: b * h <= 4096 and
  * bitdecode_fwd_workspace_bytes(b, h, num_splits) - 256 * b * h <= 7 MiB (1040 bytes per split and query
- * head), otherwise BITDECODE_EWORKSPACE.  Every call clears the part of the array it uses with a small fill
+ * head), otherwise BITDECODE_EWORKSPACE; num_splits = 0 chooses no more splits than fit.  Every call clears the part of the array it uses with a small fill
  * kernel in front of the decode kernel (calls of different shapes follow one another on the one array), so a
  * call is two or three launches.  All calls on one GPU share that array: calls that overlap in time on one
  * GPU (two streams, two host threads) race; calls on one stream do not.  The first call on a device looks up

@@ -97,3 +97,23 @@ def test_static_scratch_entry_matches_the_workspace_entry(device):
     a.num_splits = 512                                             # 512 x 64 rows x 264 B = 8.65 MB > 7 MiB
     rc = L.bitdecode_fwd_static(ctypes.byref(a), torch.cuda.current_stream(device).cuda_stream)
     assert rc == 3 and b"built-in scratch" in L.bitdecode_last_error()
+
+
+def test_static_scratch_takes_every_split_count_the_library_chooses(device):
+    """304 (sequence, kv head) pairs with eight query heads each: with three splits their records would be 7.6 MB, above the
+    7 MiB of the scratch.  Against the call with a workspace; the split counts may differ, so by their rounding (2^-11 of
+    |out| < 1 in each of the two)."""
+    from bitladder_amd import _lib, kvcache_pack_int, plan_fwd_kvcache_int
+    b, h, h_k, S = 38, 64, 8, 8192
+    g = torch.Generator(device=device).manual_seed(1)
+    k, v = (torch.randn((b, S, h_k, 128), generator=g, device=device).half() for _ in range(2))
+    cache = H.alloc_cache(b, S, h_k, 4, 128, device)
+    kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, S, "k-channel", 128, 4)
+    q = torch.randn((b, 1, h, 128), generator=g, device=device).half()
+    plan = plan_fwd_kvcache_int(q, *cache, None, SCALE, "k-channel", 128, 4, return_lse=True)
+    plan.run()
+    want, want_lse = plan.out.clone(), plan.lse.clone()
+    plan.args.num_splits = 0
+    out, lse = _run_static(plan, device)
+    torch.cuda.synchronize()
+    assert (out.float() - want.float()).abs().max() < 1e-3 and (lse - want_lse).abs().max() < 1e-4
