@@ -488,6 +488,8 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
         P.q_sr = rows_args->q_stride_row;
         P.out_sr = rows_args->out_stride_row;
     }
+    // (decode.hip: kPartialLoFrom)
+    if (nsplit > 1 && static_cast<int64_t>(a->b) * a->h_k * row_blocks > cus) P.h |= INT32_MIN;
     P.scale = a->softmax_scale;
     P.scale_log2 = fabsf(a->softmax_scale) * 1.4426950408889634f;   // decode_api.cpp:128-142
     P.neg_scale = a->softmax_scale < 0.0f;

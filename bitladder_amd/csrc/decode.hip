@@ -1054,7 +1054,12 @@ struct PartialWords {
         return __builtin_amdgcn_ballot_w64(fmaxf(__builtin_fabsf(n0), __builtin_fabsf(n1)) >= from) != 0;
     }
 };
-constexpr float kPartialLoFrom = 2.0f;      // a split sends the residual words from this output magnitude on
+// A split sends the residual words from this output magnitude on.  Launches that are split although every compute unit
+// has a workgroup without it (api.hip: choose_splits) send them always: one split would keep the sums in fp32 throughout,
+// and its error is not exceeded (against 64 bits, 264 and 384 pairs of 4K tokens, 4 bits g128: one split 2.73e-4 and
+// 3.94e-4 of the norm; with the words 2.64e-4 (three splits) and 3.39e-4 (two), without 3.05e-4 and 3.99e-4).  Sending costs
+// those launches 1-6 % (34.1 -> 35.7 and 39.4 -> 41.6 us).  The sign of `h` says so: a field of its own took the others 0.05-0.15 us.
+constexpr float kPartialLoFrom = 2.0f;
 __device__ __forceinline__ float half_lo(uint32_t w) { return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w))); }
 __device__ __forceinline__ float half_hi(uint32_t w) { return static_cast<float>(__builtin_bit_cast(_Float16, static_cast<uint16_t>(w >> 16))); }
 
@@ -1197,7 +1202,7 @@ __device__ __forceinline__ void merge_splits_n(uint32_t* o_part, uint32_t lo_wor
             d1 = sd1;
         }
         lacc += w;
-        // splits that sent residual words (rare: outputs of magnitude 2 or more), in ascending order; the words are set
+        // splits that sent residual words (outputs of magnitude 2 or more, or more pairs than compute units), in ascending order; the words are set
         // back to "not written" here, by their only reader
         uint64_t sent = __builtin_amdgcn_ballot_w64(mine && lane < BLOCK && ml.y < 0.0f);
         while (sent) {
@@ -1548,9 +1553,9 @@ void fwd_splitkv_kernel(FwdParams P) {
         if constexpr (KT) {
             const kblock ob = karg_block<BLOCK_AT(o_part)>();       // o_part ... bits
             tk = BLOCK_PTR(const int*, ob, o_part, tickets) +
-                 (static_cast<int64_t>(bi) * BLOCK_I32(ob, o_part, h) + h0) * kTicketStride + kSlotWord;
+                 (static_cast<int64_t>(bi) * (BLOCK_I32(ob, o_part, h) & INT32_MAX) + h0) * kTicketStride + kSlotWord;
         } else {
-            tk = P.tickets + (static_cast<int64_t>(bi) * P.h + h0) * kTicketStride + kSlotWord;
+            tk = P.tickets + (static_cast<int64_t>(bi) * (P.h & INT32_MAX) + h0) * kTicketStride + kSlotWord;
         }
         const uint64_t heads = (1ull << g) - 1;
         uint64_t saved;
@@ -1655,6 +1660,8 @@ void fwd_splitkv_kernel(FwdParams P) {
         tickets = BLOCK_PTR(int*, ob, o_part, tickets);
         n_h = BLOCK_I32(ob, o_part, h);
     }
+    const float lo_from = n_h < 0 ? 0.0f : kPartialLoFrom;
+    n_h &= INT32_MAX;
     // layout of the split workspace (kernels.h: split_slot_words): residual words behind the partial outputs of a
     // slot, the second slot behind the first
     const uint32_t lo_words = static_cast<uint32_t>(P.nsplit) * P.b * n_h * kPartialWords;
@@ -1759,7 +1766,8 @@ void fwd_splitkv_kernel(FwdParams P) {
             uint32_t* const rec_o = o_part + rec * kPartialWords + lane;
             float* const rec_ml = ml_part + rec * 2;
             const PartialWords W(O0, O1, L);
-            const bool sends_lo = W.large(kPartialLoFrom);      // uniform
+            // uniform; not by a split without keys, whose sum of zero has no sign to say so with
+            const bool sends_lo = L > 0.0f && W.large(lo_from);
             if (sends_lo) st_dev1(rec_o + mine_words + lo_words, W.lo());
             st_dev1(rec_o + mine_words, W.hi());
             // (max, sum) is never two zero words: a zero maximum travels as -0; a negative sum says "residual words sent"

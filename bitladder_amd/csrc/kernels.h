@@ -104,7 +104,8 @@ struct FwdParams {
     uint16_t* out;
     int64_t out_sb, out_sh;
     float* lse;         // optional [b][h]
-    int h, bits;
+    int h;              // workspace rows per sequence; sign bit: the splits always send the residual words of their outputs
+    int bits;
     // ---- the rest
     int gs, bf16;
     // Decode step with append (lengths != nullptr): sequence i holds lengths[i] tokens, the last
