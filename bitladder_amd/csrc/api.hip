@@ -88,11 +88,18 @@ int query_cus() {
 // 8K tokens, 4 bits g128 | 2 bits g128 | 4 bits g32:
 //   24 pairs, 11 and 10 splits: 10.6 and 10.0 | 9.3 (10 splits) | 15.4 and 12.1      48 pairs (10K), 6 and 5: 19.4 and 16.5 | 21.7 and 12.7 | 29.5 and 19.3
 //   80 pairs,  4 and  3 splits: 22.8 and 18.6 | 23.1 and 15.6 | 34.4 and 23.7        160 pairs (4K), 2 and 1: 24.0 and 23.7 | 23.4 and 18.0 | 34.9 and 30.5
-// With more pairs than half the units, one workgroup each leaves units idle (or, above 256 pairs, most units with
-// one and some with two); two or three splits then even that out at 4 bits, where the waves of several workgroups
-// overlap on a unit, and from 4K tokens on, where the extra merges pay: 136 pairs of 8K tokens 41.3 us with one
-// split, 31.3 with three; 264 pairs of 4K 39.5 and 34.9; 384 pairs 44.1 and 41.0 with two.  At 2 bits (one
-// workgroup of 16 waves per unit) it never paid (136 pairs: 29.2 against 29.9 us).
+// With more pairs than half the units, one workgroup each leaves units idle; two or three splits then even that out at 4
+// bits, where the waves of several workgroups overlap on a unit (at group 32, one workgroup per unit, the rounds even out),
+// from 4K tokens on, where the extra merges pay.  us with 1 | 2 | 3 splits, 4 bits g128, 8K tokens: 136 pairs 38.9 | 40.9 | 31.7,
+// 168 pairs 42.2 | 42.8 | 35.5, 200 pairs 43.6 | 45.8 | 47.4; g32 53.9 | 58.0 | 43.5, 57.2 | 60.4 | 45.3, 58.0 | 62.7 | 65.0.
+// Above one workgroup per unit the splits also send residual words (decode.hip: kPartialLoFrom), and it pays up to one and
+// a half, a third split from 6K tokens on, and at group 32 from 6K tokens on; 4K | 8K tokens, g128 / g64 / g32:
+//   264 pairs, 1, 2 and 3 splits: 38.1 36.0 35.7 | 71.3 64.4 60.2 / 41.9 38.1 38.7 / 55.8 51.5 52.5 | 106 89.3 85.6
+//   384 pairs, 1 and 2: 42.6 41.6 | 79.0 74.5 / 45.8 44.3 / 57.9 58.3 | 110 98      (32K tokens, g128: 306 and 266)
+//   424 pairs, 1 and 3: 43.4 52.0 | 82.1 91.0 / 47.2 54.8 | 89.8 97.4 / 60.8 77.0 | 115 119      -- one split
+//   600 pairs, 1 and 2: 64.5 65.5 | 125 120 / 69.5 68.4 | 132 124 / 89.9 93.7 | 169 163          -- one split
+//   800 pairs, 1 and 2: 83.4 86.0 | 164 160 / 90.2 90.7 / 117 124 | 221 214                      -- one split
+// At 2 bits (one workgroup of 16 waves per unit) it never paid below one per unit (200 pairs: 32.6 against 37.7 us).
 //
 // By the work: a workgroup wants a unit for every wave of the 8-wave kernels at 4 bits (a unit for each of 4 waves,
 // one per SIMD, at 2 bits, up to 16 splits: the merging wave takes 16 records per round trip, and a wave's time per unit
@@ -105,10 +112,11 @@ int choose_splits(int b, int hk, int max_seqlen_k, int max_res_len, int num_cus,
     if (units <= 0) return 1;
     const int64_t pairs = std::max<int64_t>(1, static_cast<int64_t>(b) * hk);
     int by_machine = static_cast<int>(std::max<int64_t>(1, num_cus / pairs));
-    if (bits == 4 && 2 * pairs > num_cus && packed_units >= 64) {
+    const bool over = pairs > num_cus, long_enough = packed_units >= 96;
+    if (bits == 4 && 2 * pairs > num_cus && packed_units >= 64 && (!over || (2 * pairs <= 3 * num_cus && (gs >= 64 || long_enough)))) {
         // share of the machine's time that the busiest unit uses: ceil(n * pairs / units) / n, against pairs / units
         double best = 0.0;
-        for (int n = 1; n <= 3; ++n) {
+        for (int n = 1; n <= (over && !long_enough ? 2 : 3); ++n) {
             const int64_t wgs = n * pairs, rounds = (wgs + num_cus - 1) / num_cus;
             const double fill = static_cast<double>(wgs) / static_cast<double>(rounds * num_cus);
             if (fill > 1.1 * best) {

@@ -313,6 +313,20 @@ def test_split_choice_and_workspace_size():
     assert lib.bitdecode_fwd_workspace_bytes(1, 3, 5) == 3 * 256 + 2 * ((3 * 5 * 130 * 4 + 255) // 256 * 256)
 
 
+@pytest.mark.parametrize("pairs,tokens,by_group", [      # splits at group 128, 64, 32 of 4 bits on 256 compute units
+    (128, 4096, (2, 2, 2)), (136, 4096, (3, 3, 3)), (136, 4032 // 128 * 128, (1, 1, 1)), (168, 8192, (3, 3, 3)),
+    (176, 8192, (1, 1, 1)), (256, 8192, (1, 1, 1)), (264, 3968, (1, 1, 1)), (264, 4096, (2, 2, 1)), (264, 6144, (3, 3, 3)),
+    (336, 8192, (3, 3, 3)), (344, 8192, (2, 2, 2)), (384, 4096, (2, 2, 1)), (384, 6144, (2, 2, 2)), (384, 32768, (2, 2, 2)),
+    (392, 8192, (1, 1, 1)), (424, 8192, (1, 1, 1)), (520, 8192, (1, 1, 1)), (800, 8192, (1, 1, 1)),
+])
+def test_split_choice_of_many_pairs(pairs, tokens, by_group):
+    lib = _lib.lib()
+    assert tuple(lib.bitdecode_num_splits(pairs // 8, 8, tokens, 0, 256, 4, gs) for gs in (128, 64, 32)) == by_group
+    # 2 bits: no more workgroups than units
+    n = lib.bitdecode_num_splits(pairs // 8, 8, tokens, 0, 256, 2, 128)
+    assert n == 1 or n * pairs <= 256
+
+
 def test_python_entry_points_validate_before_touching_the_gpu():
     import torch
     from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
