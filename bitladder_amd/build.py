@@ -34,8 +34,13 @@ HOST_SRC = "hostpath.cpp"
 HOST_PATH = os.path.join(_HERE, "_hostpath.so")
 
 
-def host_cmd() -> list:
-    import torch
+def host_cmd() -> list | None:
+    """Command line of the host extension; None without torch, whose tensors it is about: the library itself (the C ABI)
+    needs no torch."""
+    try:
+        import torch
+    except ImportError:
+        return None
     root = os.path.dirname(torch.__file__)
     abi = int(torch._C._GLIBCXX_USE_CXX11_ABI)
     return [os.environ.get("CXX", "g++"), "-O2", "-fPIC", "-shared", "-std=c++17", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
@@ -77,7 +82,10 @@ def build(verbose: bool = False) -> str:
     if verbose:
         print(" ".join(probe_cmd), flush=True)
     probe_proc = subprocess.Popen(probe_cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
-    host_proc = subprocess.Popen(host_cmd(), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    host = host_cmd()
+    if host is None:
+        print("torch is not installed: the C ABI only, without " + os.path.basename(HOST_PATH), file=sys.stderr)
+    host_proc = host and subprocess.Popen(host, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     for src, extra in PER_FILE.items():
         obj = os.path.join(objdir, src.replace(".hip", ".o"))
         cmd = [cc, *COMMON, *extra, "-c", os.path.join(CSRC, src), "-o", obj]
@@ -93,9 +101,10 @@ def build(verbose: bool = False) -> str:
     out, _ = probe_proc.communicate()
     if probe_proc.returncode != 0:
         raise RuntimeError(f"hipcc failed on {PROBE_SRC}:\n{out}")
-    out, _ = host_proc.communicate()
-    if host_proc.returncode != 0:
-        raise RuntimeError(f"{HOST_SRC} failed:\n{out}")
+    if host_proc:
+        out, _ = host_proc.communicate()
+        if host_proc.returncode != 0:
+            raise RuntimeError(f"{HOST_SRC} failed:\n{out}")
     cmd = [cc, "--offload-arch=" + ARCH, "-shared", "-fPIC", "-o", LIB_PATH, *objs]
     r = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
     if r.returncode != 0:
