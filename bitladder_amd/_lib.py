@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbitdecode.so")
 
-ABI_VERSION = 5
+ABI_VERSION = 6
 FP16, BF16 = 0, 1
 K_CHANNEL, K_TENSOR = 0, 1
 
@@ -121,7 +121,10 @@ def lib():
                 f"{LIB_PATH} is missing: build it with `python -m bitladder_amd.build` "
                 "(there is no CPU or PyTorch fallback for the HIP kernels)")
         L = ctypes.CDLL(LIB_PATH)
+        # (before anything that an older library may not have)
         L.bitdecode_abi_version.restype = ctypes.c_int
+        if L.bitdecode_abi_version() != ABI_VERSION:
+            raise ImportError("libbitdecode.so ABI version mismatch; rebuild it")
         L.bitdecode_last_error.restype = ctypes.c_char_p
         L.bitdecode_num_splits.restype = ctypes.c_int
         L.bitdecode_num_splits.argtypes = [_i32] * 7
@@ -144,8 +147,6 @@ def lib():
             fn.argtypes = [ctypes.POINTER(CacheArgs), _vp]
         L.bitdecode_fwd_append_workspace_bytes.restype = ctypes.c_size_t
         L.bitdecode_fwd_append_workspace_bytes.argtypes = [_i32] * 3
-        if L.bitdecode_abi_version() != ABI_VERSION:
-            raise ImportError("libbitdecode.so ABI version mismatch; rebuild it")
         _lib = L
     return _lib
 

@@ -19,7 +19,7 @@
 extern "C" {
 #endif
 
-#define BITDECODE_ABI_VERSION 5
+#define BITDECODE_ABI_VERSION 6
 
 enum {
     BITDECODE_OK = 0,

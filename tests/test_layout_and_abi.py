@@ -193,6 +193,21 @@ def test_library_exports_every_declared_symbol():
     assert lib.bitdecode_abi_version() == _lib.ABI_VERSION
 
 
+def test_a_library_of_another_version_is_named_as_such(monkeypatch):
+    """... also where it lacks entry points that this version binds."""
+    class Entry:
+        def __call__(self):
+            return _lib.ABI_VERSION - 1
+
+    class Older:
+        bitdecode_abi_version = Entry()
+
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setattr(_lib.ctypes, "CDLL", lambda path: Older)
+    with pytest.raises(ImportError, match="ABI version"):
+        _lib.lib()
+
+
 def test_struct_mirrors_match_header_field_order():
     header = open(os.path.join(ROOT, "include", "bitdecode.h")).read()
     for cname, cls in (("bitdecode_qpack_args", _lib.QpackArgs), ("bitdecode_fwd_args", _lib.FwdArgs),
