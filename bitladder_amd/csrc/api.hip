@@ -162,10 +162,28 @@ bool use_few_waves(int bits, int gs, int max_s, int max_r, int nsplit, bool devi
 // Lengths drawn from 1K-8K, 8 kv heads, 4 bits: 9 sequences 16.3 us with 3 splits, 15.4 with 7; 12 sequences 21.7 with
 // 2, 17.4 with 5.  Where the doubling does not apply, sequences that occupy more than half of the units are cut in two:
 // the short ones end early anyway (20 sequences: 35.4 us with one split, 27.7 with two; 2 bits 28.5 and 23.2).
+//
+// Long sequences on a number of pairs that does not divide the units: rounded down, the grid leaves units idle while the
+// longest sequence's workgroups are as long as ever; rounded up, a few units get two workgroups, which costs nothing if a short
+// sequence's is among them and half the time again if all are equal.  Two full rounds are near the better of the two in
+// either case, from 28 blocks per workgroup on (fewer: the merges and the second start cost more) and up to 16 splits (one
+// round trip of the merge).  Six draws of lengths from S/8 to S, mean time with n rounded down and with two rounds as a
+// multiple of that with n rounded up, and all sequences equal, two rounds as a multiple of n rounded down; 4 bits g128, g32, 2 bits g64:
+//    96 pairs, 18K tokens   2: 1.12 1.18 1.12     5: 1.03 0.99 1.00     equal 1.07 1.02 1.02
+//   104 pairs, 18K          2: 1.10 1.19 1.12     4: 1.05 1.05 1.00     equal 1.14 1.13 1.13
+//    72 pairs, 28K          3: 1.11 1.15 1.17     7: 1.02 0.99 1.01     equal 1.12 1.02 0.99
+//    88 pairs, 57K          2: 1.24 1.31 1.36     5: 0.94 0.93 0.93     equal 0.97 0.99 0.94
+//    40 pairs, 57K          6: 1.05 1.09 1.08    12: 1.00 0.98 1.00     equal 1.08 1.11 1.17
+//    56 pairs, 18K, below   4: 1.02 1.06 1.02     9: 0.90 1.14 1.09     equal 1.08 1.14 1.15
 int choose_splits_for(int b, int hk, int max_s, int max_r, int num_cus, int bits, int gs, bool ragged) {
     int n1 = choose_splits(b, hk, max_s, max_r, num_cus, bits, gs);
-    if (!ragged || b < 2 || n1 > 3) return n1;
+    if (!ragged || b < 2) return n1;
     const int64_t pairs = static_cast<int64_t>(b) * hk;
+    if (2 * pairs < num_cus && num_cus % pairs != 0) {
+        const int rounds2 = choose_splits(b, hk, max_s, max_r, 2 * num_cus, bits, gs);
+        if (rounds2 > n1 && rounds2 <= 16 && max_s / rounds2 >= 28 * bitdecode::kChunk) return rounds2;
+    }
+    if (n1 > 3) return n1;
     if (2 * pairs > num_cus) n1 = pairs < num_cus ? std::min(2, choose_splits(1, 1, max_s, max_r, num_cus, bits, gs)) : 1;
     // (the 8-wave kernel of group size 32 takes 95 KB of LDS: one workgroup per unit, 20.0 us with 3 splits against 23.5
     // with 7 for 9 sequences)

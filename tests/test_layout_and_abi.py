@@ -342,6 +342,22 @@ def test_split_choice_of_many_pairs(pairs, tokens, by_group):
     assert n == 1 or n * pairs <= 256
 
 
+@pytest.mark.parametrize("pairs,tokens,ragged,equal", [      # (4 bits g128, 4 bits g32, 2 bits g64) with lengths on the device, without
+    (96, 18432, (5, 5, 5), (2, 2, 2)), (104, 14336, (4, 4, 4), (2, 2, 2)), (104, 14208, (2, 2, 2), (2, 2, 2)),
+    (72, 28672, (7, 7, 7), (3, 3, 3)), (72, 24960, (3, 3, 3), (3, 3, 3)), (40, 57344, (12, 12, 12), (6, 6, 6)),
+    (24, 131072, (10, 10, 10), (10, 10, 10)),                          # 21 splits: above one round trip of the merge
+    (64, 65536, (4, 4, 4), (4, 4, 4)), (128, 65536, (2, 2, 2), (2, 2, 2)),      # a number that divides the units
+    (96, 8192, (5, 2, 2), (2, 2, 2)),                                  # two workgroups of the 8-wave kernels per unit
+])
+def test_split_choice_of_long_ragged_batches(pairs, tokens, ragged, equal):
+    lib = _lib.lib()
+    for want, flag in ((ragged, 1), (equal, 0)):
+        assert tuple(lib.bitdecode_num_splits_for(pairs // 8, 8, tokens, 128, 256, bits, gs, flag)
+                     for bits, gs in ((4, 128), (4, 32), (2, 64))) == want
+    # one sequence has nothing to even out
+    assert lib.bitdecode_num_splits_for(1, pairs, tokens, 128, 256, 4, 128, 1) == lib.bitdecode_num_splits(1, pairs, tokens, 128, 256, 4, 128)
+
+
 def test_python_entry_points_validate_before_touching_the_gpu():
     import torch
     from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
