@@ -130,7 +130,11 @@ int choose_splits(int b, int hk, int max_seqlen_k, int max_res_len, int num_cus,
         by_work = (units + bitdecode::kFewWaves - 1) / bitdecode::kFewWaves;
     } else {
         const int nw = bitdecode::decode_waves(bits, gs);
-        by_work = units <= 8 ? 1 : std::max(std::min((units + 3) / 4, 16), (2 * units + nw - 1) / nw);
+        // (up to 8 units in one workgroup; not more than 4 in the 8 waves of group 32 if the window has none or more than 4
+        // tiles, whose waves then work one after the other: 6 units and 128 window tokens, 8 pairs, 9.7 us with one split and
+        // 9.0 with two, no window 8.4 and 7.8, but 32 window tokens 8.5 and 8.7; 16 waves: 8.1 and 8.1)
+        const bool one = units <= 8 && !(nw == 8 && units > 4 && (tiles == 0 || tiles > 4));
+        by_work = one ? 1 : std::max(std::min((units + 3) / 4, 16), (2 * units + nw - 1) / nw);
     }
     int n = std::min(std::min(by_machine, std::max(1, by_work)), 256);
     // drop splits that would be empty: ceil(units / n) units per split

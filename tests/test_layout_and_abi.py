@@ -358,6 +358,15 @@ def test_split_choice_of_long_ragged_batches(pairs, tokens, ragged, equal):
     assert lib.bitdecode_num_splits_for(1, pairs, tokens, 128, 256, 4, 128, 1) == lib.bitdecode_num_splits(1, pairs, tokens, 128, 256, 4, 128)
 
 
+@pytest.mark.parametrize("tokens,window,by_group", [      # 2 bits, groups 128, 64, 32
+    (512, 128, (1, 1, 1)), (640, 0, (1, 1, 2)), (640, 64, (1, 1, 1)), (640, 65, (1, 1, 2)), (1024, 128, (1, 1, 2)),
+    (1024, 1, (1, 1, 1)), (1152, 0, (3, 3, 3)), (0, 128, (1, 1, 1)),
+])
+def test_split_choice_of_short_two_bit_calls(tokens, window, by_group):
+    lib = _lib.lib()
+    assert tuple(lib.bitdecode_num_splits(1, 8, tokens, window, 256, 2, gs) for gs in (128, 64, 32)) == by_group
+
+
 def test_python_entry_points_validate_before_touching_the_gpu():
     import torch
     from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
