@@ -533,9 +533,13 @@ def _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, soft
     if q.stride(3) != 1 or q.data_ptr() % 16 or any(s % 8 for s in q.stride()[:3]):
         # (a copy in any case: contiguous() returns a tensor whose only odd stride is that of a dimension of one)
         q = q.clone(memory_format=torch.contiguous_format)
-    # the workspace holds a record of 1040 bytes per row, head and split, below 2 GiB in all, and a launch takes at most 4096
-    # rows: more than that goes in several launches
-    per = max(1, min(4096, min(32768, 2000000 // max(1, int(kwargs.get("num_splits", 0)))) // max(1, b * h)))
+    # A launch takes at most 4096 rows, and a split one's workspace, a record of 1040 bytes per row, head and split, is below 2
+    # GiB: more than that goes in several launches.  Where the split count is left to the library, launches of many rows are
+    # not split; they are cut at half a million rows x heads (and never below the eight of a workgroup: at 256 sequences of 32
+    # heads already, launches of fewer rows read the cache twice).
+    splits = int(kwargs.get("num_splits", 0))
+    rows = 2000000 // splits // max(1, b * h) if splits > 1 else max(8 // (h // h_k), 524288 // max(1, b * h))
+    per = max(1, min(4096, rows))
     if m > per or (out is not None and out.stride(3) != 1):
         res = out if out is not None else torch.empty_like(q)
         parts = []

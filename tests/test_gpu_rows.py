@@ -95,3 +95,19 @@ def test_rows_of_any_stride_and_alignment(device):
         assert fwd_kvcache_int(q, *args, out=given) is given and torch.equal(given, want)
         given.fill_(7.0)
         assert (held == 7.0).all()
+
+
+def test_many_sequences_take_their_rows_in_one_launch(device):
+    """Eight rows of 4096 sequences of 8 heads: one launch reads the cache once."""
+    from bitladder_amd import fwd_kvcache_int, interface, kvcache_pack_int
+    b, h = 4096, 8
+    g = torch.Generator(device=device).manual_seed(8)
+    k, v = (torch.randn((b, 128, h, 128), generator=g, device=device).half() for _ in range(2))
+    cache = H.alloc_cache(b, 128, h, 4, 128, device)
+    kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, 128, "k-channel", 128, 4)
+    q = torch.randn((b, 8, h, 128), generator=g, device=device).half()
+    interface._plan_cache().clear()
+    out = fwd_kvcache_int(q, *cache, None, SCALE, "k-channel", 128, 4)
+    assert len(interface._plan_cache()) == 1
+    for r in (0, 5, 7):
+        assert torch.equal(out[:, r:r + 1], fwd_kvcache_int(q[:, r:r + 1].contiguous(), *cache, None, SCALE, "k-channel", 128, 4))
