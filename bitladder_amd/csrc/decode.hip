@@ -1767,7 +1767,8 @@ void fwd_splitkv_kernel(FwdParams P) {
             float* const rec_ml = ml_part + rec * 2;
             const PartialWords W(O0, O1, L);
             // uniform; not by a split without keys, whose sum of zero has no sign to say so with
-            const bool sends_lo = L > 0.0f && W.large(lo_from);
+            // (no short cut: with the outputs behind a branch the compiler rounds them once, to fp16, instead of twice)
+            const bool sends_lo = W.large(lo_from) & (L > 0.0f);
             if (sends_lo) st_dev1(rec_o + mine_words + lo_words, W.lo());
             st_dev1(rec_o + mine_words, W.hi());
             // (max, sum) is never two zero words: a zero maximum travels as -0; a negative sum says "residual words sent"
