@@ -1406,8 +1406,9 @@ constexpr int fwd_lds_bytes() {
 // ROWS: several query rows per sequence.  The rows x heads (query row, query head) pairs of a kv head are numbered row
 // by row and cut into blocks of eight, one workgroup per block, so that every MFMA column but those of the last block
 // carries a query whatever the two counts are.  A pair takes the place of a query head: workspace rows, tickets and
-// waves of the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; they are
-// neighbours on one XCD, so all but the first find them in its L2.  (Before, the rows were folded into the head dimension
+// waves of the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; where the
+// grid is remapped (several splits, a multiple of eight pairs) they are neighbours on one XCD, and all but the first find them in
+// its L2; otherwise they are dealt to all XCDs.  (Before, the rows were folded into the head dimension
 // on the host, 8 / g rows per launch, the cache read once per launch: eight rows of 32 / 8 heads over 2 x 8K tokens took
 // four launches and eight copies, 112 us; one launch takes 15.1.)
 template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, bool ROWS>

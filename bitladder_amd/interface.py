@@ -166,8 +166,8 @@ _tls = threading.local()
 
 
 def _plan_cache() -> dict:
-    """Argument blocks of this thread's last distinct drop-in calls (a thread of its own each: a block is
-    patched with the call's output pointer before it is handed to the library)."""
+    """Argument blocks of this thread's last distinct drop-in calls, by the key of the native host path (which copies a block
+    to set the call's output in it and never writes the kept one)."""
     c = getattr(_tls, "plans", None)
     if c is None:
         c = _tls.plans = {}
