@@ -328,6 +328,16 @@ def test_split_choice_and_workspace_size():
     assert lib.bitdecode_fwd_workspace_bytes(1, 3, 5) == 3 * 256 + 2 * ((3 * 5 * 130 * 4 + 255) // 256 * 256)
 
 
+def test_the_grid_gives_no_compute_unit_a_second_workgroup():
+    lib = _lib.lib()
+    for pairs, want in ((1, 16), (8, 16), (24, 10), (40, 6), (48, 5), (72, 3), (80, 3), (96, 2), (120, 2)):
+        for bits, gs in ((4, 128), (4, 32), (2, 128), (2, 32)):
+            h_k = 8 if pairs % 8 == 0 else 1
+            assert lib.bitdecode_num_splits(pairs // h_k, h_k, 8192, 64, 256, bits, gs) == want, (pairs, bits, gs)
+    # ... of a device with fewer units, too
+    assert lib.bitdecode_num_splits(1, 8, 32768, 64, 32, 4, 128) == 4 and lib.bitdecode_num_splits(1, 8, 32768, 64, 30, 2, 64) == 3
+
+
 @pytest.mark.parametrize("pairs,tokens,by_group", [      # splits at group 128, 64, 32 of 4 bits on 256 compute units
     (128, 4096, (2, 2, 2)), (136, 4096, (3, 3, 3)), (136, 4032 // 128 * 128, (1, 1, 1)), (168, 8192, (3, 3, 3)),
     (176, 8192, (1, 1, 1)), (256, 8192, (1, 1, 1)), (264, 3968, (1, 1, 1)), (264, 4096, (2, 2, 1)), (264, 6144, (3, 3, 3)),
