@@ -99,6 +99,13 @@ __device__ __forceinline__ h2 pk_rtz(float a, float b) {
     return __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
+// rounded to nearest, one v_cvt_pk_f16_f32 (the bias of a truncation does not quite cancel between a sum of p * v and the sum of p:
+// see kHeadroom for what it makes of the error)
+__device__ __forceinline__ h2 pk_rne(float a, float b) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    return __builtin_convertvector((f2{a, b}), h2);
+}
+
 // 16 bytes of fp16 (or bf16 converted to fp16; exact inside the fp16 normal range)
 template <bool BF16>
 __device__ __forceinline__ h8 cvt_h8(u4 raw) {
@@ -185,49 +192,79 @@ __device__ __forceinline__ float partner(float x) {
 }
 // (every lane has a source lane, so the "bound control" flag changes nothing but tells the compiler
 // that no previous value of the result survives, which saves it a move)
-__device__ __forceinline__ uint32_t partner(uint32_t x) {
-    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x128, 0xf, 0xf, true));
+// the partner's value in the lo columns (8-15) and zero in the hi ones, and the reverse: DPP row_shr:8 / row_shl:8, which
+// leave zero where a row of 16 lanes has no source lane
+__device__ __forceinline__ uint32_t to_lo_columns(uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x118, 0xf, 0xf, true));
+}
+__device__ __forceinline__ uint32_t to_hi_columns(uint32_t x) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(0, static_cast<int>(x), 0x108, 0xf, 0xf, true));
 }
 // max over the four lanes that share a column (lane, lane^16, lane^32, lane^48).
 // v_permlane16_swap exchanges the odd 16-lane rows of its first register with the even rows of
 // its second one, v_permlane32_swap does the same with 32-lane halves; fed two copies of x they
 // leave (rows 0,0,2,2 / rows 1,1,3,3) and (lower,lower / upper,upper), whose element-wise max is
 // the reduction.  Written as asm: the compiler builtin folds the two results into one here.
-// The s_nop covers the wait states the swap needs after a VALU write of its operands.
+// The s_nops cover the wait states a swap or a DPP read needs after a VALU write of its operands.  The maxima are written
+// out as well: around an asm result fmaxf costs three instructions, as it quiets both operands first, and every one of them is
+// in the chain between the scores and the probabilities (nine of sixteen here; with those of row_max16 512 to 4K tokens
+// of one sequence 0.02-0.04 us).
+#define COLMAX(x, y)                                       \
+    "v_mov_b32 " y ", " x "\n\ts_nop 1\n\t"               \
+    "v_permlane16_swap_b32 " x ", " y "\n\t"              \
+    "v_max_f32 " x ", " x ", " y "\n\t"                   \
+    "v_mov_b32 " y ", " x "\n\ts_nop 1\n\t"               \
+    "v_permlane32_swap_b32 " x ", " y "\n\t"              \
+    "v_max_f32 " x ", " x ", " y
 __device__ __forceinline__ float colmax(float x) {
-    float y = x;
-    asm volatile("s_nop 1\n\tv_permlane16_swap_b32 %0, %1" : "+v"(x), "+v"(y));
-    x = fmaxf(x, y);
-    y = x;
-    asm volatile("s_nop 1\n\tv_permlane32_swap_b32 %0, %1" : "+v"(x), "+v"(y));
-    return fmaxf(x, y);
+    float y;
+    asm volatile("s_nop 0\n\t" COLMAX("%0", "%1") : "+v"(x), "=&v"(y));
+    return x;
 }
 
 template <int NCG>
 struct WaveState {
-    float m;          // running max of the raw scores (q.k units) of this lane's head
-    // (l and ob: an MFMA makes all four rows alike; only row 0 is kept in step with the maximum and read)
-    f4 l;             // sum of p, accumulated by MFMA against a ones operand (hi columns only)
-    f4 ob[NCG];       // V bias per channel group, accumulated by MFMA
+    float m;          // reference of the exponentials (raw scores, q.k units) of this lane's head: no score so far is above it (kNoScore: none yet)
+    // (l and ob: an MFMA makes all four rows alike; only row 0 is kept in step with the reference and read)
+    f4 l;             // sum of p, accumulated by MFMA against a ones operand; both columns of a head hold it
+    // Zero part of the V bias, one MFMA per 32 tokens for all channel groups: row m of its A operand has the zeros of group
+    // m % NCG, so register c is group c's (with one MFMA per group six MFMAs and LDS reads more per 64 tokens at group 32).
+    // Both columns of a head hold it.
+    f4 zb;
+    f4 ob[NCG];       // offset part of the V bias per channel group, hi and lo
     f4 o[8];          // O^T tiles: lane (head, q) holds channels 16*ct + 4*q + r
 };
 
+// The reference of a head without scores: below every sum of 128 products of fp16 values, and finite, so that differences with
+// it need no special case (p of a masked score, -inf, is zero whatever the reference).
+constexpr float kNoScore = -1e30f;
+
+// When a score exceeds the reference, the new reference is put this far above it (base-2 units), so that the next maxima do
+// not move it again: a move rescales all accumulators, 35 to 41 instructions, and with eight heads some maximum moves in most of a wave's
+// steps.  8 sequences of 64K at 2 bits 63.5 -> 61.4 us, 6 sequences of 10K at 4 bits g32 18.3 -> 17.8.  p stays at 2^pshift or
+// below (its product with the V scale has to stay in range) and is at least 2^(pshift - headroom) for the largest score.  An fp16 p keeps
+// its precision down to 2^-14, so the headroom costs only what lies 11 binades and more below the largest p; rounding p to
+// nearest (pk_rne) gains more: error against 64 bits, 4 bits g128 over 32K 4.9e-4 -> 3.9e-4 of the norm (3.8e-4 without headroom),
+// 2 bits g64 over 4K 4.6e-4 -> 3.9e-4 (3.8e-4).
+constexpr float kHeadroom = 3.0f;
+
 // Online-softmax step over N raw scores t (q.k units); on return t holds
-// p = 2^pshift * exp2(scale * (t - running max)).  Accumulators are rescaled only when the
-// running max of some head moved (wave-uniform branch).  With HALVES the hi column and the lo
-// column of a head hold different halves of the step's scores, and the maximum is taken over both.
-template <int N, int NCG, bool HALVES = false>
+// p = 2^pshift * exp2(scale * (t - reference)).  Accumulators are rescaled only when the
+// reference of some head moved (wave-uniform branch).  mx: the largest new score of
+// the lane's head, the same in all its lanes.
+template <int N, int NCG>
 __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st, float mx, float pshift) {
-    if constexpr (HALVES) mx = fmaxf(mx, partner(mx));
-    mx = colmax(mx);
-    const float m_new = fmaxf(st.m, mx);
-    const float m_use = (m_new == -INFINITY) ? 0.0f : m_new;
-    if (__builtin_amdgcn_ballot_w64(m_new > st.m) != 0) {
-        if (__builtin_amdgcn_ballot_w64(st.m > -INFINITY) != 0) {
+    if (__builtin_amdgcn_ballot_w64(mx > st.m) != 0) {
+        // (the headroom in raw score units; worked out here: as a kernel argument it took the short calls 0.1-0.2 us)
+        const float headroom = fminf(kHeadroom * __builtin_amdgcn_rcpf(scale), 1e30f);
+        const float m_new = mx > st.m ? mx + headroom : st.m;
+        if (__builtin_amdgcn_ballot_w64(st.m != kNoScore) != 0) {
             // (not in a wave's first step, which has nothing to rescale: 512 to 8K tokens of one sequence, one unit per wave,
             // 0.12 us of 6.0 to 7.3)
-            const float alpha = __builtin_amdgcn_exp2f((st.m - m_use) * scale);
+            const float alpha = __builtin_amdgcn_exp2f((st.m - m_new) * scale);
             st.l[0] *= alpha;
+#pragma unroll
+            for (int c = 0; c < NCG; ++c) st.zb[c] *= alpha;
 #pragma unroll
             for (int c = 0; c < NCG; ++c) st.ob[c][0] *= alpha;
 #pragma unroll
@@ -235,7 +272,7 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
         }
         st.m = m_new;
     }
-    const float c0 = pshift - m_use * scale;
+    const float c0 = pshift - st.m * scale;
 #pragma unroll
     for (int i = 0; i < N; ++i) t[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[i], scale, c0));
 }
@@ -244,12 +281,11 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
     float mx = t[0];
 #pragma unroll
     for (int i = 1; i < N; ++i) mx = fmaxf(mx, t[i]);
-    softmax_step<N, NCG>(t, scale, st, mx, pshift);
+    softmax_step<N, NCG>(t, scale, st, colmax(mx), pshift);
 }
 
 // Accumulators of the four S^T tiles of a 64-token step -> probabilities as operands of the second
-// product, per 32-token sub-block ks: p16 (every column), pz (p in the hi columns, 0 in the lo ones),
-// pm (the reverse).  Element i = 4*T + r of a sub-block is tile 2*ks + T, accumulator register r.
+// product, per 32-token sub-block ks: p16 (every column), pm (p in the lo columns, 0 in the hi ones).  Element i = 4*T + r of a sub-block is tile 2*ks + T, accumulator register r.
 // A tile's hi and lo columns hold the two parts of its scores; their sum is the score.
 //
 // The hi column takes sub-block 0 and the lo column sub-block 1 (eight sums and exponentials per lane, where both doing
@@ -263,46 +299,44 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
 // 15.4 against 15.0), equal with one 4-bit unit per wave.
 template <int BITS, int NCG>
 __device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t hi_cols, float scale, WaveState<NCG>& st,
-                                                   h8 (&p16)[2], h8 (&pz)[2], h8 (&pm)[2]) {
+                                                   h8 (&p16)[2], h8 (&pm)[2]) {
     float t[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) t[i] = sc[i / 4][i % 4] + partner(sc[i / 4][i % 4]);
-    float mx;      // maximum of the lane's eight sums
+    float mx, y;      // maximum of the lane's eight sums, then of the head's (both columns)
     asm volatile("s_nop 7\n\ts_nop 3\n\t"
-                 "v_add_f32_dpp %0, %9, %9 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %1, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %2, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %3, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %4, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %5, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %6, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
-                 "v_add_f32_dpp %7, %16, %16 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %0, %10, %10 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %1, %11, %11 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %2, %12, %12 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %3, %13, %13 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %4, %14, %14 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %5, %15, %15 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %6, %16, %16 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
+                 "v_add_f32_dpp %7, %17, %17 row_ror:8 row_mask:0xf bank_mask:0xc\n\t"
                  "v_max3_f32 %8, %0, %1, %2\n\t"
                  "v_max3_f32 %8, %8, %3, %4\n\t"
                  "v_max3_f32 %8, %8, %5, %6\n\t"
-                 "v_max_f32 %8, %8, %7"
+                 "v_max_f32 %8, %8, %7\n\ts_nop 1\n\t"
+                 "v_max_f32_dpp %8, %8, %8 row_ror:8 row_mask:0xf bank_mask:0xf\n\t" COLMAX("%8", "%9")
                  : "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]), "+v"(t[4]), "+v"(t[5]), "+v"(t[6]), "+v"(t[7]),
-                   "=&v"(mx)
+                   "=&v"(mx), "=&v"(y)
                  : "v"(sc[2][0]), "v"(sc[2][1]), "v"(sc[2][2]), "v"(sc[2][3]), "v"(sc[3][0]), "v"(sc[3][1]),
                    "v"(sc[3][2]), "v"(sc[3][3]));
-    softmax_step<8, NCG, true>(t, scale, st, mx, p_shift(BITS));
-    u4 pw;
-#pragma unroll
-    for (int x = 0; x < 4; ++x) pw[x] = __builtin_bit_cast(uint32_t, pk_rtz(t[2 * x], t[2 * x + 1]));
-    const u4 z0 = pw & hi_cols;       // the hi columns hold sub-block 0
-    const u4 m1 = pw & ~hi_cols;      // the lo columns hold sub-block 1
-    u4 z1, m0;
+    softmax_step<8, NCG>(t, scale, st, mx, p_shift(BITS));
+    u4 z0, m0, z1, m1;      // the hi columns hold sub-block 0, the lo columns sub-block 1
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
-        z1[x] = partner(m1[x]);
-        m0[x] = partner(z0[x]);
+        const uint32_t pw = __builtin_bit_cast(uint32_t, pk_rne(t[2 * x], t[2 * x + 1]));
+        m0[x] = to_lo_columns(pw);
+        z1[x] = to_hi_columns(pw);
+        z0[x] = (pw & hi_cols) | m0[x];
+        m1[x] = pw & ~hi_cols;
+        z1[x] |= m1[x];
     }
-    pz[0] = __builtin_bit_cast(h8, z0);
+    p16[0] = __builtin_bit_cast(h8, z0);
     pm[0] = __builtin_bit_cast(h8, m0);
-    pz[1] = __builtin_bit_cast(h8, z1);
+    p16[1] = __builtin_bit_cast(h8, z1);
     pm[1] = __builtin_bit_cast(h8, m1);
-    p16[0] = __builtin_bit_cast(h8, z0 | m0);
-    p16[1] = __builtin_bit_cast(h8, z1 | m1);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -604,20 +638,22 @@ struct KGroup {
 };
 
 // The workgroup's LDS copy of q: rows 0-7 = the eight head slots of the GQA group ([128] fp16
-// values each; slots past the group repeat head 0 and are never written out), row 8 = zeros.
-// A lane reads q three ways without any select: plain (its head), hi-only (zero row in the lo
-// columns) and lo-only (zero row in the hi columns).
+// values each; slots past the group repeat head 0 and are never written out), and zeros behind them.
+// A lane reads q three ways without any select: plain (its head), hi-only (zeros in the lo
+// columns) and lo-only (zeros in the hi columns).
 struct QRows {
     const uint8_t* q;    // row of this lane's head
-    const uint8_t* qz;   // same row in the hi columns, zero row in the lo columns
-    const uint8_t* qm;   // zero row in the hi columns, same row in the lo columns
+    const uint8_t* qz;   // same row in the hi columns, zeros in the lo columns
+    const uint8_t* qm;   // zeros in the hi columns, same row in the lo columns
 };
-// Rows are 272 bytes apart (256 + 16 of padding) so that the eight heads read by neighbouring
-// lanes fall into different LDS banks.
-constexpr int kQRowBytes = 272;
+// Rows are 288 bytes apart (256 + 32 of padding): a 16-byte read takes 16 lanes at a time, eight heads and two
+// neighbouring kg, which then cover the 64 banks once (4 cycles a read, measured; 8 with 272 bytes).  The zeros a lane reads lie in
+// the banks its own row would take.
+constexpr int kQRowBytes = 288;
+constexpr int kZeroRow = kMaxGroupHeads * kQRowBytes, kZeroBytes = 7 * 32 + 256, kQBytes = kZeroRow + kZeroBytes;
 __device__ __forceinline__ QRows q_rows(const uint8_t* sq, int head, int kg, bool lo_part) {
     const uint8_t* row = sq + head * kQRowBytes + kg * 16;
-    const uint8_t* zero = sq + 8 * kQRowBytes + kg * 16;
+    const uint8_t* zero = sq + kZeroRow + head * 32 + kg * 16;
     return QRows{row, lo_part ? zero : row, lo_part ? row : zero};
 }
 __device__ __forceinline__ h8 q_load(const uint8_t* row, int j) {
@@ -706,6 +742,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
     const u4* vcode = reinterpret_cast<const u4*>(reg + 4096) + lane;
     const uint8_t* kpar = reg + C::OFF_KP + kslot * C::KPB;
     const uint8_t* vpar = reg + C::OFF_VP + kg * 16;
+    const uint8_t* vzero = vpar + 64 + (lane & (NCG - 1)) * 128;      // row of the zero operand: channel group (row % NCG)
 #define ROW_READY(kind, idx) row_ready<BITS, GS, HAS_NEXT, pos_of<BITS, GS>(kind, idx), KT, FEW>(cur, next, lane16, region_lds, kslot)
 
     // the K parameters lead the queue: the first K group is prepared while the code rows arrive
@@ -774,10 +811,10 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
         }
 
         static_assert(TPS == 4 && NKS == 2, "four tiles, two sub-blocks per step");
-        h8 p16[NKS], pz[NKS], pm[NKS];
-        step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pz, pm);
+        h8 p16[NKS], pm[NKS];
+        step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pm);
 #pragma unroll
-        for (int ks = 0; ks < NKS; ++ks) st.l = mfma32(ones, pz[ks], st.l);
+        for (int ks = 0; ks < NKS; ++ks) st.l = mfma32(ones, p16[ks], st.l);
         // V side of the step, row by row.  A row holds one channel half (tiles ct = 4*hf .. 4*hf+3) of one
         // 32-token sub-block (4 bits) or of the whole step (2 bits).
         if (step == 0) {
@@ -802,9 +839,11 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                     for (int ks = (BITS == 4 ? ksr : 0); ks < (BITS == 4 ? ksr + 1 : NKS); ++ks) {
                         const int sb = step * NKS + ks;               // 32-token sub-block inside the unit
                         const u4 rs = *reinterpret_cast<const u4*>(vpar + (sb * NCG + cg) * 128);
-                        const u4 rz = *reinterpret_cast<const u4*>(vpar + (sb * NCG + cg) * 128 + 64);
                         pp[cg][ks] = split_mul_masked(p16[ks], pm[ks], cvt_h8<false>(rs));
-                        st.ob[cg] = mfma32(cvt_h8<false>(rz), pz[ks], st.ob[cg]);
+                        if (cg == 0) {      // the zeros of all channel groups
+                            const u4 rz = *reinterpret_cast<const u4*>(vzero + sb * NCG * 128);
+                            st.zb = mfma32(cvt_h8<false>(rz), p16[ks], st.zb);
+                        }
                         st.ob[cg] = mfma32(noff, pp[cg][ks], st.ob[cg]);
                     }
                 }
@@ -984,10 +1023,10 @@ __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P,
         }
     }
     softmax_step<4, NCG>(s, P.scale_log2, st, pshift);
-    const h2 p01 = pk_rtz(s[0], s[1]), p23 = pk_rtz(s[2], s[3]);
+    const h2 p01 = pk_rne(s[0], s[1]), p23 = pk_rne(s[2], s[3]);
     h4 pb = {p01[0], p01[1], p23[0], p23[1]};
-    if (lo_part) pb = h4{0, 0, 0, 0};
     st.l = mfma16(h4{1, 1, 1, 1}, pb, st.l);
+    if (lo_part) pb = h4{0, 0, 0, 0};
 #pragma unroll
     for (int ct = 0; ct < 8; ++ct) {
         uint16_t e[4];
@@ -1075,10 +1114,12 @@ __device__ __forceinline__ float row_ror(float x) {
 // reductions over each row of 16 lanes, result in every lane of the row; the additions are grouped the
 // same way in every run
 __device__ __forceinline__ float row_max16(float x) {
-    x = fmaxf(x, row_ror<8>(x));
-    x = fmaxf(x, row_ror<4>(x));
-    x = fmaxf(x, row_ror<2>(x));
-    return fmaxf(x, row_ror<1>(x));
+    asm volatile("s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:8 row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:4 row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:2 row_mask:0xf bank_mask:0xf\n\t"
+                 "s_nop 1\n\tv_max_f32_dpp %0, %0, %0 row_ror:1 row_mask:0xf bank_mask:0xf"
+                 : "+v"(x));
+    return x;
 }
 __device__ __forceinline__ float row_sum16(float x) {
     x += row_ror<8>(x);
@@ -1393,14 +1434,14 @@ __device__ __forceinline__ int sequence_of_position(const FwdParams& P, int p, i
 // the wave that draws the last ticket merges all partials of the head
 // (flash_fwd_kernel.h:1217-1298 formula) and resets the ticket.
 //
-// Dynamic LDS: [NW wave regions of UnitCfg::REGION bytes][q: 8 head rows + a zero row, 272 B apart]
+// Dynamic LDS: [NW wave regions of UnitCfg::REGION bytes][q: 8 head rows, 288 B apart][zeros]
 // [sM, sL: per-wave max and sum, 8 heads x NW floats each][append flag][tickets and slots of the 8 heads].  A wave's region is reused as its
 // V-transpose slab for fp16 tiles and as its slot of the cross-wave merge buffer (g x 128 floats <= 4 KB).
 // ---------------------------------------------------------------------------------------------
 template <int BITS, int GS, bool FEW>
 constexpr int fwd_lds_bytes() {
     using C = UnitCfg<BITS, GS, FEW>;
-    return C::NW * C::REGION + (kMaxGroupHeads + 1) * kQRowBytes + 2 * C::NW * kMaxGroupHeads * 4 + 16 + 2 * kMaxGroupHeads * 4;
+    return C::NW * C::REGION + kQBytes + 2 * C::NW * kMaxGroupHeads * 4 + 16 + 2 * kMaxGroupHeads * 4;
 }
 
 // ROWS: several query rows per sequence.  The rows x heads (query row, query head) pairs of a kv head are numbered row
@@ -1441,8 +1482,8 @@ void fwd_splitkv_kernel(FwdParams P) {
     constexpr int NCG = C::NCG, NW = C::NW, REGION = C::REGION;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     static_assert(sizeof(qp::PackLds<GS>) <= NW * REGION, "the pack tile reuses the wave regions");
-    uint8_t* const sq = lds + NW * REGION;                                   // [8 + zero row][128] 16-bit q
-    float* const sM = reinterpret_cast<float*>(sq + (kMaxGroupHeads + 1) * kQRowBytes);   // [8][NW]
+    uint8_t* const sq = lds + NW * REGION;                                   // [8][128] 16-bit q, zeros
+    float* const sM = reinterpret_cast<float*>(sq + kQBytes);   // [8][NW]
     float* const sL = sM + NW * kMaxGroupHeads;
     int* const s_last = reinterpret_cast<int*>(sL + NW * kMaxGroupHeads);
     int* const s_tick = s_last + 4;       // [8] tickets drawn for the heads of the group, -1 = not yet
@@ -1580,15 +1621,15 @@ void fwd_splitkv_kernel(FwdParams P) {
         uint8_t* dst = sq + (lane >> 4) * kQRowBytes + (lane & 15) * 16;
         *reinterpret_cast<h8*>(dst) = cvt_h8<BF16>(qa);
         *reinterpret_cast<h8*>(dst + 4 * kQRowBytes) = cvt_h8<BF16>(qb);
-        if (lane < 16) *reinterpret_cast<u4*>(sq + 8 * kQRowBytes + lane * 16) = u4{0, 0, 0, 0};
+        if (lane < kZeroBytes / 16) *reinterpret_cast<u4*>(sq + kZeroRow + lane * 16) = u4{0, 0, 0, 0};
     }
     // (head slots past the group hold head 0 again: finite values whose results are never stored)
     const QRows Q = q_rows(sq, head, kg, lo_part);
     PROF(1);
 
     WaveState<NCG> st;
-    st.m = -INFINITY;
-    st.l = f4{0, 0, 0, 0};
+    st.m = kNoScore;
+    st.l = st.zb = f4{0, 0, 0, 0};
 #pragma unroll
     for (int c = 0; c < NCG; ++c) st.ob[c] = f4{0, 0, 0, 0};
 #pragma unroll
@@ -1668,12 +1709,15 @@ void fwd_splitkv_kernel(FwdParams P) {
     const uint32_t lo_words = static_cast<uint32_t>(P.nsplit) * P.b * n_h * kPartialWords;
     const uint32_t slot_words = (lo_words / kPartialWords * (2 * kPartialWords + 2) + 63) / 64 * 64;
     // ---- merge the waves of this workgroup through LDS (each wave's slot is its own region)
-    const float lsum = st.l[0] + partner(st.l[0]);      // lo columns hold 0
+    const float lsum = st.l[0];
+    float bias[NCG];      // V bias of the lane's column: the zero part, which both columns hold, is taken from the hi one
+#pragma unroll
+    for (int c = 0; c < NCG; ++c) bias[c] = st.ob[c][0] + (lo_part ? 0.0f : st.zb[c]);
 #pragma unroll
     for (int ct = 0; ct < 8; ++ct) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float v = st.o[ct][r] + st.ob[ct / (GS / 16)][0];
+            const float v = st.o[ct][r] + bias[ct / (GS / 16)];
             st.o[ct][r] = v + partner(v);      // hi + lo
         }
     }
