@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbitdecode.so")
 
-ABI_VERSION = 6
+ABI_VERSION = 7
 FP16, BF16 = 0, 1
 K_CHANNEL, K_TENSOR = 0, 1
 
@@ -98,7 +98,7 @@ class CacheArgs(ctypes.Structure):
 EXPORTS = ("bitdecode_abi_version", "bitdecode_last_error", "bitdecode_num_splits",
            "bitdecode_fwd_workspace_bytes", "bitdecode_num_splits_for", "bitdecode_qpack", "bitdecode_fwd",
            "bitdecode_fwd_append", "bitdecode_fwd_append_workspace_bytes", "bitdecode_fwd_static",
-           "bitdecode_fwd_rows", "bitdecode_cache_prefill", "bitdecode_cache_append")
+           "bitdecode_fwd_rows", "bitdecode_row_blocks", "bitdecode_cache_prefill", "bitdecode_cache_append")
 
 _lib = None
 
@@ -128,6 +128,8 @@ def lib():
         L.bitdecode_last_error.restype = ctypes.c_char_p
         L.bitdecode_num_splits.restype = ctypes.c_int
         L.bitdecode_num_splits.argtypes = [_i32] * 7
+        L.bitdecode_row_blocks.restype = ctypes.c_int
+        L.bitdecode_row_blocks.argtypes = [_i32] * 6
         L.bitdecode_num_splits_for.restype = ctypes.c_int
         L.bitdecode_num_splits_for.argtypes = [_i32] * 8
         L.bitdecode_fwd_workspace_bytes.restype = ctypes.c_size_t

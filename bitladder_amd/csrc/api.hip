@@ -143,6 +143,30 @@ int choose_splits(int b, int hk, int max_seqlen_k, int max_res_len, int num_cus,
     return std::max(1, n);
 }
 
+// Several query rows per sequence: blocks of sixteen (query row, query head) pairs instead of eight?  A workgroup then unpacks the
+// codes for twice as many pairs, at half the vector instructions per pair, but a wave takes longer over a unit and over the merge.
+// So it pays with work: W = units of 64 tokens times blocks of eight pairs per compute unit.  us in blocks of eight | sixteen,
+// 32 / 8 heads unless said, 4 bits g128, 4 bits g32, 2 bits g128:
+//   1 x 4K, 8 rows            W  8:   8.6 |  9.9    9.4 | 10.5    9.2 | 10.3
+//   1 x 8K, 8 rows            W 16:  10.9 | 11.3   12.7 | 12.0   10.1 | 11.6       16 x 1K, 4 rows  W 16:  10.1 | 10.1   11.5 | 10.8   9.0 | 9.4
+//   1 x 12K, 8 rows           W 24:  12.9 | 11.9   14.8 | 12.8   11.9 | 12.2       3 x 4K, 8 rows   W 24:  14.7 | 12.3   17.2 | 13.7  13.1 | 10.9
+//   4 x 2K, 64 / 8, 8 rows    W 32:  16.9 | 12.4   20.1 | 13.9   13.4 | 11.5       32 x 2K, 8 / 8, 16 rows  W 64:  29.1 | 18.0   37.7 | 21.6  25.7 | 15.2
+// Where so few (sequence, kv head, block) triples are left that filling the machine takes more than 32 splits, the second round trip of
+// their merge outweighs it at 2 bits, and at 4 bits until W is larger:
+//   1 x 64K, 8 / 1, 8 rows    W 32:  17.7 | 18.6   21.0 | 19.9   16.7 | 17.9       1 x 128K, 8 / 1  W 64:  31.2 | 24.0   37.0 | 27.1  22.8 | 21.1 (g64 23.7 | 24.9)
+bool rows_wide(int b, int hk, int pairs, int max_s, int cus, int bits) {
+    if (pairs <= bitdecode::kMaxGroupHeads) return false;
+    const int64_t blocks8 = (pairs + bitdecode::kMaxGroupHeads - 1) / bitdecode::kMaxGroupHeads, blocks16 = (blocks8 + 1) / 2;
+    const bool many_splits = static_cast<int64_t>(b) * hk * blocks16 * 32 < cus;
+    if (many_splits && bits == 2) return false;
+    const int from = many_splits ? 48 : bits == 4 ? 20 : 28;
+    return static_cast<int64_t>(b) * hk * blocks8 * (max_s / 64) >= static_cast<int64_t>(from) * cus;
+}
+int row_blocks_of(int pairs, bool wide) {
+    const int block = wide ? bitdecode::kWidePairs : bitdecode::kMaxGroupHeads;
+    return (pairs + block - 1) / block;
+}
+
 // The 4-bit kernels also exist with 8 waves per workgroup (decode.hip: launch_fwd_tt), used whenever the packed
 // prefix is the bulk of the work.  With per-sequence lengths on the device the workgroups of the longest
 // sequences can be left streaming alone at the end, where 16 waves keep more bytes in flight per compute
@@ -218,6 +242,11 @@ int bitdecode_num_splits_for(int32_t b, int32_t h_k, int32_t max_seqlen_k, int32
     if (num_cus <= 0) num_cus = query_cus();
     if (check_quant(bits, group_size, BITDECODE_FP16, bitdecode::kHeadDim)) return -1;
     return choose_splits_for(b, h_k, max_seqlen_k, max_res_len, num_cus, bits, group_size, per_sequence_lengths != 0);
+}
+
+int bitdecode_row_blocks(int32_t b, int32_t h_k, int32_t pairs, int32_t max_seqlen_k, int32_t num_cus, int32_t bits) {
+    if (num_cus <= 0) num_cus = query_cus();
+    return row_blocks_of(std::max(1, pairs), rows_wide(b, h_k, pairs, max_seqlen_k, num_cus, bits));
 }
 
 // [tickets: one 256-byte block per (batch, query head)][o_part][ml_part]
@@ -404,7 +433,6 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     if (rows < 1 || rows > 4096) return fail(BITDECODE_EINVAL, "%d query rows per sequence (1 to 4096)", rows);
     if (rows_args && rows_args->q_stride_row % 8)
         return fail(BITDECODE_EINVAL, "q and residual strides must be multiples of 8 elements");
-    const int row_blocks = rows > 1 ? (rows * g + kMaxGroupHeads - 1) / kMaxGroupHeads : 1;
     const int n_h = a->h * rows;        // workspace rows per sequence
     int max_s = a->seqlens_k ? a->max_seqlen_k : a->seqlen_k;
     int max_r = a->res_lens ? a->max_res_len : a->res_len;
@@ -426,6 +454,9 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
         max_r = kChunk;
     }
     if (max_s < 0 || max_r < 0) return fail(BITDECODE_EINVAL, "negative length");
+    const int cus = query_cus();
+    const bool wide = rows > 1 && rows_wide(a->b, a->h_k, rows * g, max_s, cus, a->bits);
+    const int row_blocks = rows > 1 ? row_blocks_of(rows * g, wide) : 1;
     if (max_s % kChunk) return fail(BITDECODE_EINVAL, "packed length %d is not a multiple of 128", max_s);
     if (!a->block_table && max_s > a->cache_tokens)
         return fail(BITDECODE_EINVAL, "packed length %d exceeds cache capacity %d", max_s, a->cache_tokens);
@@ -452,11 +483,14 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     int nsplit = a->num_splits;
     if (nsplit < 0) return fail(BITDECODE_EINVAL, "num_splits %d is negative", nsplit);
     if (nsplit > 512) return fail(BITDECODE_EINVAL, "num_splits %d is above the limit of 512", nsplit);
-    const int cus = query_cus();
     if (nsplit == 0)
         nsplit = choose_splits_for(a->b, a->h_k * row_blocks, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k && !step);
     // (the built-in scratch takes every call that leaves the count to the library: it chooses no more than fits)
     while (static_scratch && a->num_splits == 0 && nsplit > 1 && slots_bytes(a->b, n_h, nsplit) > kStaticScratchBytes - kStaticCounterBytes)
+        --nsplit;
+    // (several query rows, count left to the library: no more splits than the caller's workspace holds, which it may have sized for
+    // a count of its own)
+    while (rows_args && a->num_splits == 0 && nsplit > 1 && bitdecode_fwd_workspace_bytes(a->b, n_h, nsplit) > (a->workspace ? a->workspace_bytes : 0))
         --nsplit;
     if (nsplit > 1 && slots_bytes(a->b, n_h, nsplit) >= (size_t(1) << 31))
         return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d heads: partial outputs of 2 GiB or more", nsplit, a->b, n_h);
@@ -511,7 +545,7 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     P.out_sb = a->out_stride_b; P.out_sh = a->out_stride_h;
     P.lse = a->softmax_lse;
     P.b = a->b; P.h = n_h; P.hk = a->h_k; P.g = g; P.nsplit = nsplit;
-    P.rows = rows; P.row_blocks = row_blocks;
+    P.rows = rows; P.row_blocks = row_blocks; P.rows_wide = wide;
     P.row_blocks_magic = division_magic(static_cast<uint32_t>(row_blocks));
     P.g_magic = division_magic(static_cast<uint32_t>(g));
     if (rows_args) {

@@ -339,6 +339,23 @@ __device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t h
     pm[1] = __builtin_bit_cast(h8, m1);
 }
 
+// The same where every column is a pair of its own (sixteen query row and head pairs): the sums are whole scores, and a lane
+// exponentiates all sixteen of its column.
+template <int BITS, int NCG>
+__device__ __forceinline__ void step_probabilities_wide(const f4 (&sc)[4], float scale, WaveState<NCG>& st, h8 (&p16)[2]) {
+    float t[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t[i] = sc[i / 4][i % 4];
+    softmax_step<16, NCG>(t, scale, st, p_shift(BITS));
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+        u4 w;
+#pragma unroll
+        for (int x = 0; x < 4; ++x) w[x] = __builtin_bit_cast(uint32_t, pk_rne(t[8 * ks + 2 * x], t[8 * ks + 2 * x + 1]));
+        p16[ks] = __builtin_bit_cast(h8, w);
+    }
+}
+
 // ---------------------------------------------------------------------------------------------
 // packed units, streamed through LDS
 // ---------------------------------------------------------------------------------------------
@@ -632,9 +649,12 @@ __device__ __forceinline__ void row_ready(const UnitAddr<BITS, GS>& cur, const U
 
 // Per-group state of the K side: Q with the group's scale folded in (exact hi/lo split) and the
 // score bias  sum_c q_c*zero_c - sum_c (q_c*scale_c)*offset_c  built on the MFMA pipe.
+template <bool WIDE>
 struct KGroup {
-    h8 qp[4];
+    h8 qp[4];                  // hi parts in columns 0-7, lo parts in columns 8-15; WIDE: hi parts
+    h8 qp_lo[WIDE ? 4 : 1];    // WIDE: lo parts
     f4 kb;
+    f4 kb_lo;                  // WIDE: the lo parts' (hi and lo are summed apart, so that the scores are those of a call for one row)
 };
 
 // The workgroup's LDS copy of q: rows 0-7 = the eight head slots of the GQA group ([128] fp16
@@ -650,7 +670,9 @@ struct QRows {
 // neighbouring kg, which then cover the 64 banks once (4 cycles a read, measured; 8 with 272 bytes).  The zeros a lane reads lie in
 // the banks its own row would take.
 constexpr int kQRowBytes = 288;
-constexpr int kZeroRow = kMaxGroupHeads * kQRowBytes, kZeroBytes = 7 * 32 + 256, kQBytes = kZeroRow + kZeroBytes;
+constexpr int kZeroRow = kMaxGroupHeads * kQRowBytes, kZeroBytes = 7 * 32 + 256;
+// (WIDE: 16 rows and no zeros; the banks come out the same, as 16 lanes then are 16 rows, half of them at the next kg)
+constexpr int q_bytes(bool wide) { return wide ? 2 * kMaxGroupHeads * kQRowBytes : kZeroRow + kZeroBytes; }
 __device__ __forceinline__ QRows q_rows(const uint8_t* sq, int head, int kg, bool lo_part) {
     const uint8_t* row = sq + head * kQRowBytes + kg * 16;
     const uint8_t* zero = sq + kZeroRow + head * 32 + kg * 16;
@@ -673,17 +695,34 @@ __device__ __forceinline__ h8 split_mul_masked(h8 a, h8 a_lo_only, h8 b) {
     return __builtin_elementwise_fma(a, b, -__builtin_bit_cast(h8, hi_in_lo_cols));
 }
 
-template <int BITS, bool BF16>
-__device__ __forceinline__ void start_group(KGroup& G, const uint8_t* kpar, const QRows& Q, int kg) {
+// a*b as an exact fp16 pair in two registers: lo = fma(a, b, -hi)
+__device__ __forceinline__ void split_mul(h8 a, h8 b, h8& hi, h8& lo) {
+    u4 h = __builtin_bit_cast(u4, a * b);
+#pragma unroll
+    for (int x = 0; x < 4; ++x) asm("" : "+v"(h[x]));      // (as in split_mul_masked)
+    hi = __builtin_bit_cast(h8, h);
+    lo = __builtin_elementwise_fma(a, b, -hi);
+}
+
+template <int BITS, bool WIDE>
+__device__ __forceinline__ void start_group(KGroup<WIDE>& G, const uint8_t* kpar, const QRows& Q, int kg) {
     const h8 noff = -code_offsets<BITS>();
     G.kb = f4{0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const h8 sc = cvt_h8<false>(*reinterpret_cast<const u4*>(kpar + (32 * j + 8 * kg) * 2));
         const h8 zr = cvt_h8<false>(*reinterpret_cast<const u4*>(kpar + 256 + (32 * j + 8 * kg) * 2));
-        G.qp[j] = split_mul_masked(q_load(Q.q, j), q_load(Q.qm, j), sc);
-        G.kb = mfma32(zr, q_load(Q.qz, j), G.kb);
-        G.kb = mfma32(noff, G.qp[j], G.kb);
+        if constexpr (WIDE) {
+            const h8 q = q_load(Q.q, j);
+            split_mul(q, sc, G.qp[j], G.qp_lo[j]);
+            G.kb = mfma32(zr, q, G.kb);
+            G.kb = mfma32(noff, G.qp[j], G.kb);
+            G.kb_lo = mfma32(noff, G.qp_lo[j], j == 0 ? f4{0, 0, 0, 0} : G.kb_lo);
+        } else {
+            G.qp[j] = split_mul_masked(q_load(Q.q, j), q_load(Q.qm, j), sc);
+            G.kb = mfma32(zr, q_load(Q.qz, j), G.kb);
+            G.kb = mfma32(noff, G.qp[j], G.kb);
+        }
     }
 }
 
@@ -699,11 +738,11 @@ __device__ __forceinline__ void start_group(KGroup& G, const uint8_t* kpar, cons
 // with the two q sums of every group prepared once per wave (KQ).
 template <int NCG>
 struct TokenQ {
-    h8 q[4];          // q of the lane's head in the hi columns, zero in the lo columns
+    h8 q[4];          // q of the lane's head in the hi columns, zero in the lo columns (WIDE: q of every column's pair)
     float noffq[NCG]; // - sum_c offset_c q_c per channel group, for the lane's column
     float qsum[NCG];  //   sum_c q_c
 };
-template <int BITS, int NCG>
+template <int BITS, int NCG, bool WIDE>
 __device__ __forceinline__ TokenQ<NCG> token_q(const QRows& Q) {
     TokenQ<NCG> T;
     const h8 noff = -code_offsets<BITS>();
@@ -713,7 +752,7 @@ __device__ __forceinline__ TokenQ<NCG> token_q(const QRows& Q) {
     for (int c = 0; c < NCG; ++c) no[c] = qs[c] = f4{0, 0, 0, 0};
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        T.q[j] = q_load(Q.qz, j);
+        T.q[j] = q_load(WIDE ? Q.q : Q.qz, j);
         no[j * NCG / 4] = mfma32(noff, T.q[j], no[j * NCG / 4]);
         qs[j * NCG / 4] = mfma32(ones, T.q[j], qs[j * NCG / 4]);
     }
@@ -725,7 +764,7 @@ __device__ __forceinline__ TokenQ<NCG> token_q(const QRows& Q) {
     return T;
 }
 
-template <int BITS, int GS, bool BF16, bool HAS_NEXT, bool KT = false, bool FEW = false>
+template <int BITS, int GS, bool BF16, bool HAS_NEXT, bool KT, bool FEW, bool WIDE>
 __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region_lds, int kslot,
                                              const UnitAddr<BITS, GS>& cur, const UnitAddr<BITS, GS>& next,
                                              const QRows& Q, const FwdParams& P, int lane, bool lo_part, const Magic& mg,
@@ -752,8 +791,8 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
         if (i == 1) ROW_READY(0, 1);
     }
     static_assert(C::NKP <= 2 && C::NVP <= 2, "parameter rows of a unit");
-    KGroup G;
-    if constexpr (!KT) start_group<BITS, BF16>(G, kpar, Q, kg);
+    KGroup<WIDE> G;
+    if constexpr (!KT) start_group<BITS, WIDE>(G, kpar, Q, kg);
 #pragma unroll
     for (int step = 0; step < NSTEP; ++step) {
         f4 sc[TPS];
@@ -790,13 +829,19 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                 continue;
             }
             if (tile != 0 && tile % TPG == 0) {
-                start_group<BITS, BF16>(G, kpar + ((tile * 16) / GS) * kKParamGroupBytes, Q, kg);
+                start_group<BITS, WIDE>(G, kpar + ((tile * 16) / GS) * kKParamGroupBytes, Q, kg);
             }
             f4 acc = G.kb;
+            [[maybe_unused]] f4 acc_lo;
+            if constexpr (WIDE) acc_lo = G.kb_lo;
             if constexpr (BITS == 4) {
                 const u4 w = kcode[64 * tile];
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc = mfma32(dq4(w[j], mg), G.qp[j], acc);
+                for (int j = 0; j < 4; ++j) {
+                    const h8 a = dq4(w[j], mg);
+                    acc = mfma32(a, G.qp[j], acc);
+                    if constexpr (WIDE) acc_lo = mfma32(a, G.qp_lo[j], acc_lo);
+                }
             } else {
                 const u4 w = kcode[64 * (tile / 2)];
 #pragma unroll
@@ -805,14 +850,23 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                     dq2(w[2 * (tile % 2) + jj], a0, a1, mg);
                     acc = mfma32(a0, G.qp[2 * jj], acc);
                     acc = mfma32(a1, G.qp[2 * jj + 1], acc);
+                    if constexpr (WIDE) {
+                        acc_lo = mfma32(a0, G.qp_lo[2 * jj], acc_lo);
+                        acc_lo = mfma32(a1, G.qp_lo[2 * jj + 1], acc_lo);
+                    }
                 }
             }
+            if constexpr (WIDE) acc += acc_lo;
             sc[tt] = acc;
         }
 
         static_assert(TPS == 4 && NKS == 2, "four tiles, two sub-blocks per step");
         h8 p16[NKS], pm[NKS];
-        step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pm);
+        if constexpr (WIDE) {
+            step_probabilities_wide<BITS, NCG>(sc, P.scale_log2, st, p16);
+        } else {
+            step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pm);
+        }
 #pragma unroll
         for (int ks = 0; ks < NKS; ++ks) st.l = mfma32(ones, p16[ks], st.l);
         // V side of the step, row by row.  A row holds one channel half (tiles ct = 4*hf .. 4*hf+3) of one
@@ -824,7 +878,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                 if (i == 1) ROW_READY(2, 1);
             }
         }
-        h8 pp[NCG][NKS];
+        h8 pp[NCG][NKS], pp_lo[WIDE ? NCG : 1][NKS];
         constexpr int CGH = NCG >= 2 ? NCG / 2 : 1;      // channel groups per channel half
 #pragma unroll
         for (int r = 0; r < RPS; ++r) {
@@ -839,12 +893,17 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                     for (int ks = (BITS == 4 ? ksr : 0); ks < (BITS == 4 ? ksr + 1 : NKS); ++ks) {
                         const int sb = step * NKS + ks;               // 32-token sub-block inside the unit
                         const u4 rs = *reinterpret_cast<const u4*>(vpar + (sb * NCG + cg) * 128);
-                        pp[cg][ks] = split_mul_masked(p16[ks], pm[ks], cvt_h8<false>(rs));
+                        if constexpr (WIDE) {
+                            split_mul(p16[ks], cvt_h8<false>(rs), pp[cg][ks], pp_lo[cg][ks]);
+                        } else {
+                            pp[cg][ks] = split_mul_masked(p16[ks], pm[ks], cvt_h8<false>(rs));
+                        }
                         if (cg == 0) {      // the zeros of all channel groups
                             const u4 rz = *reinterpret_cast<const u4*>(vzero + sb * NCG * 128);
                             st.zb = mfma32(cvt_h8<false>(rz), p16[ks], st.zb);
                         }
                         st.ob[cg] = mfma32(noff, pp[cg][ks], st.ob[cg]);
+                        if constexpr (WIDE) st.ob[cg] = mfma32(noff, pp_lo[cg][ks], st.ob[cg]);
                     }
                 }
             }
@@ -858,12 +917,18 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
             for (int x = 0; x < 4; ++x) {
                 const int ct = 4 * hf + x, cg = ct / CTPG;
                 if constexpr (BITS == 4) {
-                    st.o[ct] = mfma32(dq4(w[x], mg), pp[cg][ksr], st.o[ct]);
+                    const h8 a = dq4(w[x], mg);
+                    st.o[ct] = mfma32(a, pp[cg][ksr], st.o[ct]);
+                    if constexpr (WIDE) st.o[ct] = mfma32(a, pp_lo[cg][ksr], st.o[ct]);
                 } else {
                     h8 a0, a1;
                     dq2(w[x], a0, a1, mg);
                     st.o[ct] = mfma32(a0, pp[cg][0], st.o[ct]);
                     st.o[ct] = mfma32(a1, pp[cg][1], st.o[ct]);
+                    if constexpr (WIDE) {
+                        st.o[ct] = mfma32(a0, pp_lo[cg][0], st.o[ct]);
+                        st.o[ct] = mfma32(a1, pp_lo[cg][1], st.o[ct]);
+                    }
                 }
             }
         }
@@ -993,7 +1058,7 @@ __device__ __forceinline__ void load_fp16_tile(Fp16Tile& T, const WindowSrc& W, 
     }
 }
 
-template <bool BF16, int NCG>
+template <bool BF16, int NCG, bool WIDE>
 __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P, int n0, int R, int lane,
                                           const QRows& Q, bool lo_part, WaveState<NCG>& st, uint16_t* lds, float pshift) {
     const int col = lane & 15, kg = lane >> 4;
@@ -1013,12 +1078,13 @@ __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P,
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             // fp16 operands are exact: only the hi columns carry q
-            acc = mfma32(cvt_h8<BF16>(T.k[j]), q_load(Q.qz, j), acc);
+            acc = mfma32(cvt_h8<BF16>(T.k[j]), q_load(WIDE ? Q.q : Q.qz, j), acc);
         }
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const int tk = n0 + 4 * kg + r;
-            float tot = acc[r] + partner(acc[r]);   // outside the select: every lane executes the DPP
+            float tot = acc[r];
+            if constexpr (!WIDE) tot += partner(acc[r]);   // outside the select: every lane executes the DPP
             s[r] = tk < R ? tot : -INFINITY;
         }
     }
@@ -1026,7 +1092,7 @@ __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P,
     const h2 p01 = pk_rne(s[0], s[1]), p23 = pk_rne(s[2], s[3]);
     h4 pb = {p01[0], p01[1], p23[0], p23[1]};
     st.l = mfma16(h4{1, 1, 1, 1}, pb, st.l);
-    if (lo_part) pb = h4{0, 0, 0, 0};
+    if (!WIDE && lo_part) pb = h4{0, 0, 0, 0};
 #pragma unroll
     for (int ct = 0; ct < 8; ++ct) {
         uint16_t e[4];
@@ -1319,6 +1385,204 @@ __device__ __forceinline__ void write_head(uint16_t* out_row, float* lse, int la
 }
 
 // ---------------------------------------------------------------------------------------------
+// the same for sixteen pairs and eight waves (WIDE): each half of a wave owns a pair, its lane hl channels 4*hl .. 4*hl+3, so
+// that the chain behind the workgroup's barrier is as long as for one pair (one after the other: 2.0 us more).  What is a
+// scalar above is a value per half here; lane n of a row of 16 reaches the others by row_newbcast.
+// ---------------------------------------------------------------------------------------------
+__device__ __forceinline__ void st_dev_words(uint32_t* p, uint32_t a, uint32_t b) {
+    __hip_atomic_store(reinterpret_cast<uint64_t*>(p), a | (static_cast<uint64_t>(b) << 32), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint2 ld_dev_words(const uint32_t* p) {
+    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return uint2{static_cast<uint32_t>(v), static_cast<uint32_t>(v >> 32)};
+}
+// value of lane N of the lane's row of 16
+template <int N>
+__device__ __forceinline__ float row_bcast(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x150 + N, 0xf, 0xf, true));
+}
+// value of the same lane in the other row of the half
+__device__ __forceinline__ float other_row(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_ds_swizzle(__builtin_bit_cast(int, x), 0x401f));
+}
+__device__ __forceinline__ void add_weighted(float (&o)[4], float w, uint2 v) {
+    o[0] = __builtin_fmaf(w, half_lo(v.x), o[0]);
+    o[1] = __builtin_fmaf(w, half_hi(v.x), o[1]);
+    o[2] = __builtin_fmaf(w, half_lo(v.y), o[2]);
+    o[3] = __builtin_fmaf(w, half_hi(v.y), o[3]);
+}
+template <int K, int N>
+__device__ __forceinline__ void add_records(float (&e)[4], float (&d)[4], float w_row0, float w_row1, const uint2 (&v)[N]) {
+    if constexpr (K < N) {
+        const float w = row_bcast<K & 15>(K < 16 ? w_row0 : w_row1);
+        add_weighted(K % 2 ? d : e, w, v[K]);
+        add_records<K + 1, N>(e, d, w_row0, w_row1, v);
+    }
+}
+// merge_splits_n for the pairs of the active halves
+template <int N>
+__device__ __forceinline__ void wide_merge_splits(uint32_t* head_base, uint32_t lo_words, float* mlb, int nsplit, int lane,
+                                                  float (&O)[4], float& M, float& L) {
+    const int hl = lane & 31;
+    float lacc = 0.0f, Mu = 0.0f;
+    float e[4] = {0, 0, 0, 0}, d[4] = {0, 0, 0, 0};
+    for (int s0 = 0; s0 < nsplit; s0 += 32) {
+        const bool mine = s0 + hl < nsplit;
+        const int sl = min(s0 + hl, nsplit - 1), cnt = nsplit - s0;
+        const uint32_t* rec = head_base + s0 * kPartialWords + 2 * hl;
+        float2 ml;
+        uint2 v[N];
+        for (int spin = 0;; ++spin) {
+            ml = ld_dev2(mlb + 2 * sl);
+#pragma unroll
+            for (int k = 0; k < N; ++k) v[k] = ld_dev_words(rec + k * kPartialWords);
+            uint32_t mn = __float_as_uint(ml.x) | __float_as_uint(ml.y);
+#pragma unroll
+            for (int k = 0; k < N; ++k) {
+                v[k] = k < cnt ? v[k] : uint2{0x3c003c00u, 0x3c003c00u};      // (splits that do not exist: weight zero)
+                mn = min(mn, min(v[k].x, v[k].y));
+            }
+            if (__builtin_amdgcn_ballot_w64(mn == 0) == 0 || spin >= kMaxPolls) break;
+        }
+        if (s0 == 0) {
+            float mx = mine ? ml.x : -INFINITY;
+            for (int s = 32; s < nsplit; s += 32) {        // more splits than a block holds: the other maxima
+                float2 t = float2{-INFINITY, 0.0f};
+                for (int spin = 0;; ++spin) {
+                    bool ok = true;
+                    if (s + hl < nsplit) {
+                        t = ld_dev2(mlb + 2 * (s + hl));
+                        ok = (__float_as_uint(t.x) | __float_as_uint(t.y)) != 0;
+                    }
+                    if (__builtin_amdgcn_ballot_w64(!ok) == 0 || spin >= kMaxPolls) break;
+                }
+                mx = fmaxf(mx, t.x);
+            }
+            mx = row_max16(mx);
+            M = fmaxf(mx, other_row(mx));
+            Mu = (M == -INFINITY) ? 0.0f : M;
+        }
+        const float w = mine ? __builtin_amdgcn_exp2f(ml.x - Mu) * __builtin_fabsf(ml.y) : 0.0f;
+        const float wo = other_row(w);
+        add_records<0, N>(e, d, lane & 16 ? wo : w, lane & 16 ? w : wo, v);
+        lacc += w;
+        // residual words: of either half, one split after the other
+        const uint64_t sent = __builtin_amdgcn_ballot_w64(mine && ml.y < 0.0f);
+        uint32_t both = static_cast<uint32_t>(sent) | static_cast<uint32_t>(sent >> 32);
+        while (both) {
+            const int s = __builtin_ctz(both);
+            both &= both - 1;
+            const float ws = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(((lane & 32) + s) * 4, __builtin_bit_cast(int, w)));
+            if ((sent >> ((lane & 32) + s)) & 1) {
+                uint32_t* lo = head_base + lo_words + (s0 + s) * kPartialWords + 2 * hl;
+                uint2 r;
+                for (int spin = 0;; ++spin) {
+                    r = ld_dev_words(lo);
+                    if (__builtin_amdgcn_ballot_w64(r.x == 0 || r.y == 0) == 0 || spin >= kMaxPolls) break;
+                }
+                add_weighted(e, ws, r);
+                st_dev_words(lo, 0, 0);
+            }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 4; ++c) O[c] = e[c] + d[c];
+    const float lrow = row_sum16(lacc);
+    L = lrow + other_row(lrow);
+}
+template <bool BF16>
+__device__ __forceinline__ void wide_write(uint16_t* out_row, float* lse, int hl, const float (&O)[4], float M, float L, float pshift) {
+    const bool none = !(L > 0.0f);
+    const float inv = none ? 0.0f : __builtin_amdgcn_rcpf(L);
+    uint16_t r[4];
+#pragma unroll
+    for (int c = 0; c < 4; ++c) r[c] = to_out<BF16>(O[c] * inv);
+    if ((reinterpret_cast<uintptr_t>(out_row) & 7u) == 0) {
+        reinterpret_cast<uint2*>(out_row)[hl] = uint2{r[0] | (static_cast<uint32_t>(r[1]) << 16), r[2] | (static_cast<uint32_t>(r[3]) << 16)};
+    } else {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) out_row[4 * hl + c] = r[c];
+    }
+    if (hl == 0 && lse) *lse = none ? INFINITY : (M + __log2f(L) - pshift) * 0.69314718055994531f;
+}
+template <int W, int NW, int REGION>
+__device__ __forceinline__ void add_waves(float (&O)[4], float aw, const uint8_t* mine) {
+    if constexpr (W < NW) {
+        const f4 v = *reinterpret_cast<const f4*>(mine + W * REGION);
+        const float a = row_bcast<W>(aw);
+#pragma unroll
+        for (int c = 0; c < 4; ++c) O[c] = __builtin_fmaf(a, v[c], O[c]);
+        add_waves<W + 1, NW, REGION>(O, aw, mine);
+    }
+}
+// everything behind the workgroup's barrier; the protocol between the splits is written out in the kernel
+template <int BITS, int NW, int REGION, bool BF16>
+__device__ __forceinline__ void wide_tail(const FwdParams& P, const uint8_t* lds, const float* sM, const float* sL, const int* s_cnt,
+                                          int wave, int lane, int g, int bi, int hk, int blk, int h0, int split, int n_h,
+                                          uint32_t lo_words, uint32_t slot_words, float lo_from) {
+    static_assert(NW * 2 == kWidePairs, "a pair per half wave");
+    if (wave >= g) return;
+    const int hl = lane & 31, hh = wave + (lane >> 5) * NW;
+    const bool mine = hh < g;
+    const int64_t hrow = static_cast<int64_t>(bi) * n_h + h0 + hh;
+    const bool split_run = P.nsplit > 1;
+    int drawn = 0;
+    if (split_run && mine && hl == 0) {
+        drawn = __hip_atomic_fetch_add(&P.tickets[hrow * kTicketStride], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    const int x = kWidePairs * blk + hh, row = div_magic(x, P.g_magic), head = hk * P.g + x - row * P.g;
+    uint16_t* out_row = P.out + bi * P.out_sb + row * P.out_sr + head * P.out_sh;
+    float* lse_row = P.lse ? P.lse + (static_cast<int64_t>(bi) * P.rows + row) * (P.g * P.hk) + head : nullptr;
+
+    const int w = lane & (NW - 1);
+    const float mw = sM[hh * NW + w], lw = (lane & 15) < NW ? sL[hh * NW + w] : 0.0f;
+    float M = row_max16(mw);
+    const float aw = __builtin_amdgcn_exp2f(mw - (M == -INFINITY ? 0.0f : M));
+    float L = row_sum16(aw * lw);
+    float O[4] = {0, 0, 0, 0};
+    add_waves<0, NW, REGION>(O, aw, lds + hh * kHeadDim * 4 + hl * 16);
+    if (!split_run) {
+        if (mine) wide_write<BF16>(out_row, lse_row, hl, O, M, L, p_shift(BITS));
+        return;
+    }
+    const int par = s_cnt[hh] & 1;
+    const uint32_t mine_words = par ? slot_words : 0u, other_words = par ? 0u : slot_words;
+    const int64_t rec = hrow * P.nsplit + split;
+    uint32_t* const rec_o = P.o_part + rec * kPartialWords + 2 * hl;
+    float* const rec_ml = P.ml_part + rec * 2;
+    const PartialWords A(O[0], O[1], L), B(O[2], O[3], L);
+    const float top = fmaxf(fmaxf(__builtin_fabsf(A.n0), __builtin_fabsf(A.n1)), fmaxf(__builtin_fabsf(B.n0), __builtin_fabsf(B.n1)));
+    const bool sends_lo = ((__builtin_amdgcn_ballot_w64(top >= lo_from) >> (lane & 32)) & 0xffffffffull) != 0 && L > 0.0f;
+    if (mine) {
+        if (sends_lo) st_dev_words(rec_o + mine_words + lo_words, A.lo(), B.lo());
+        st_dev_words(rec_o + mine_words, A.hi(), B.hi());
+        if (hl == 0) st_dev2(rec_ml + mine_words, M == 0.0f ? -0.0f : M, sends_lo ? -L : L);
+        st_dev_words(rec_o + other_words, 0, 0);
+        if (hl == 0) st_dev2(rec_ml + other_words, 0.0f, 0.0f);
+    }
+    const int d0 = __builtin_amdgcn_readlane(drawn, 0), d1 = __builtin_amdgcn_readlane(drawn, 32);
+    const bool last = mine && (lane & 32 ? d1 : d0) == P.nsplit - 1;
+    if (last) {
+        if (hl == 0) {
+            __hip_atomic_store(&P.tickets[hrow * kTicketStride], 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            __hip_atomic_store(&P.tickets[hrow * kTicketStride + kSlotWord], par ^ 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        uint32_t* const head_base = P.o_part + mine_words + hrow * P.nsplit * kPartialWords;
+        float* const mlb = P.ml_part + mine_words + hrow * P.nsplit * 2;
+        if (P.nsplit <= 4) {
+            wide_merge_splits<4>(head_base, lo_words, mlb, P.nsplit, lane, O, M, L);
+        } else if (P.nsplit <= 8) {
+            wide_merge_splits<8>(head_base, lo_words, mlb, P.nsplit, lane, O, M, L);
+        } else if (P.nsplit <= 16) {
+            wide_merge_splits<16>(head_base, lo_words, mlb, P.nsplit, lane, O, M, L);
+        } else {
+            wide_merge_splits<32>(head_base, lo_words, mlb, P.nsplit, lane, O, M, L);
+        }
+        wide_write<BF16>(out_row, lse_row, hl, O, M, L, p_shift(BITS));
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
 // decode step with append: per-sequence length, the workgroup that stores and packs, the counter
 // ---------------------------------------------------------------------------------------------
 // The length is stable for every workgroup that reads it: it is advanced only after all workgroups of
@@ -1438,26 +1702,32 @@ __device__ __forceinline__ int sequence_of_position(const FwdParams& P, int p, i
 // [sM, sL: per-wave max and sum, 8 heads x NW floats each][append flag][tickets and slots of the 8 heads].  A wave's region is reused as its
 // V-transpose slab for fp16 tiles and as its slot of the cross-wave merge buffer (g x 128 floats <= 4 KB).
 // ---------------------------------------------------------------------------------------------
-template <int BITS, int GS, bool FEW>
+template <int BITS, int GS, bool FEW, bool WIDE>
 constexpr int fwd_lds_bytes() {
     using C = UnitCfg<BITS, GS, FEW>;
-    return C::NW * C::REGION + kQBytes + 2 * C::NW * kMaxGroupHeads * 4 + 16 + 2 * kMaxGroupHeads * 4;
+    constexpr int cols = WIDE ? kWidePairs : kMaxGroupHeads;
+    return C::NW * C::REGION + q_bytes(WIDE) + 2 * C::NW * cols * 4 + 16 + 2 * cols * 4;
 }
 
 // ROWS: several query rows per sequence.  The rows x heads (query row, query head) pairs of a kv head are numbered row
-// by row and cut into blocks of eight, one workgroup per block, so that every MFMA column but those of the last block
-// carries a query whatever the two counts are.  A pair takes the place of a query head: workspace rows, tickets and
-// waves of the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; where the
+// by row and cut into blocks, one workgroup per block.  Blocks of eight run as a group of heads does (kRowsFew).  In blocks of
+// sixteen (kRowsWide, WIDE; api.hip: rows_wide) every MFMA column is a pair of its own, and the hi and the lo parts of the split products
+// go through two MFMAs instead of two columns of one.  Unpacking, the largest part of the vector instructions, is then done once for
+// sixteen pairs instead of eight, the products in the lanes that need them and the hi + lo additions by the MFMA
+// accumulation: per 64 tokens and sixteen pairs about 420 issue slots instead of 780.  A pair takes the place of a query head: workspace
+// rows, tickets and the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; where the
 // grid is remapped (several splits, a multiple of eight pairs) they are neighbours on one XCD, and all but the first find them in
-// its L2; otherwise they are dealt to all XCDs.  (Before, the rows were folded into the head dimension
-// on the host, 8 / g rows per launch, the cache read once per launch: eight rows of 32 / 8 heads over 2 x 8K tokens took
-// four launches and eight copies, 112 us; one launch takes 15.1.)
-template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, bool ROWS>
+// its L2; otherwise they are dealt to all XCDs.  Eight rows of 32 / 8 heads over 2 x 8K tokens: 112 us with the rows
+// folded into the head dimension on the host (four launches), 14.5 in blocks of eight, 11.9 in blocks of sixteen.
+template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, int ROWS_KIND>
 // (second bound: waves per SIMD the register count has to leave room for.  Two workgroups of the 8-wave kernels share
 // a compute unit when sequences differ in length, 4 waves per SIMD like the 16-wave kernels: 128 registers.  The
-// per-token-K kernel of group size 32 needs more and runs one workgroup per unit.)
-__global__ __launch_bounds__((UnitCfg<BITS, GS, FEW>::NW * 64), (FEW && !(KT && GS == 32) ? 4 : 1))
+// per-token-K kernel of group size 32 needs more and runs one workgroup per unit, and so do the wide ones.)
+__global__ __launch_bounds__((UnitCfg<BITS, GS, FEW>::NW * 64), (FEW && !(KT && GS == 32) ? (ROWS_KIND == kRowsWide ? 2 : 4) : 1))
 void fwd_splitkv_kernel(FwdParams P) {
+    constexpr bool ROWS = ROWS_KIND != kRowsNone, WIDE = ROWS_KIND == kRowsWide;
+    constexpr int kCols = WIDE ? kWidePairs : kMaxGroupHeads;      // heads or pairs of a workgroup
+    static_assert(!WIDE || (FEW && !APPEND && kWidePairs * kHeadDim * 4 <= 8192), "8 waves; a wave's slot of the merge in its region");
     static_assert(!KT || BITS == 4, "per-token K parameters: 4 bits");
     // The decode step with append has more parameter fields than scalar registers, and the per-token-K kernels
     // have no vector register to spare for scalar spills: they fetch what only the window and the tail need from
@@ -1483,12 +1753,12 @@ void fwd_splitkv_kernel(FwdParams P) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     static_assert(sizeof(qp::PackLds<GS>) <= NW * REGION, "the pack tile reuses the wave regions");
     uint8_t* const sq = lds + NW * REGION;                                   // [8][128] 16-bit q, zeros
-    float* const sM = reinterpret_cast<float*>(sq + kQBytes);   // [8][NW]
-    float* const sL = sM + NW * kMaxGroupHeads;
-    int* const s_last = reinterpret_cast<int*>(sL + NW * kMaxGroupHeads);
-    int* const s_tick = s_last + 4;       // [8] tickets drawn for the heads of the group, -1 = not yet
-    int* const s_cnt = s_tick + kMaxGroupHeads;      // [8] slot of this launch for each head of the group
-    if (threadIdx.x < kMaxGroupHeads) s_tick[threadIdx.x] = -1;      // (read after the workgroup barrier of the tail)
+    float* const sM = reinterpret_cast<float*>(sq + q_bytes(WIDE));   // [kCols][NW]
+    float* const sL = sM + NW * kCols;
+    int* const s_last = reinterpret_cast<int*>(sL + NW * kCols);
+    int* const s_tick = s_last + 4;       // [kCols] tickets drawn for the heads of the group, -1 = not yet
+    int* const s_cnt = s_tick + kCols;    // [kCols] slot of this launch for each head of the group
+    if (threadIdx.x < kCols) s_tick[threadIdx.x] = -1;      // (read after the workgroup barrier of the tail)
 
     PROF_DECL;
     PROF(0);
@@ -1527,11 +1797,11 @@ void fwd_splitkv_kernel(FwdParams P) {
         if (P.seq_perm) bi = sequence_of_position(P, bi, lane);
     }
     const int col = lane & 15, kg = lane >> 4;
-    const int head = col & 7;          // query head inside the GQA group
+    const int head = WIDE ? col : col & 7;          // query head inside the GQA group (ROWS: pair inside the block)
     const bool lo_part = col >= 8;     // columns 8-15 carry the lo halves of the split products
     // heads (ROWS: row and head pairs) of this workgroup, and the number of the first one
-    const int g = ROWS ? min(kMaxGroupHeads, P.g * P.rows - kMaxGroupHeads * blk) : P.g;
-    const int h0 = ROWS ? hk * P.g * P.rows + kMaxGroupHeads * blk : hk * P.g;
+    const int g = ROWS ? min(kCols, P.g * P.rows - kCols * blk) : P.g;
+    const int h0 = ROWS ? hk * P.g * P.rows + kCols * blk : hk * P.g;
 
     int S, R, r_new = -1, step_len = 0;
     if constexpr (APPEND) {
@@ -1560,14 +1830,21 @@ void fwd_splitkv_kernel(FwdParams P) {
     // oldest entry of each wave's own load queue.
     int u = u0 + wave;
     u4 qa_raw, qb_raw, qa, qb;
+    [[maybe_unused]] u4 qc_raw, qd_raw, qc, qd;      // (WIDE: rows 8 .. 15)
     {
         const int hq = lane >> 4;                         // head within a row of four
         if constexpr (ROWS) {
             const uint16_t* q0 = P.q + bi * P.q_sb + (hk * P.g) * P.q_sh + (lane & 15) * 8;
-            const int xa = kMaxGroupHeads * blk + (hq < g ? hq : 0), xb = kMaxGroupHeads * blk + (hq + 4 < g ? hq + 4 : 0);
-            const int ra = div_magic(xa, P.g_magic), rb = div_magic(xb, P.g_magic);
-            qa_raw = load_untracked(q0 + ra * P.q_sr + (xa - ra * P.g) * P.q_sh);
-            qb_raw = load_untracked(q0 + rb * P.q_sr + (xb - rb * P.g) * P.q_sh);
+            const auto pair = [&](int i) {
+                const int x = kCols * blk + (i < g ? i : 0), r = div_magic(x, P.g_magic);
+                return load_untracked(q0 + r * P.q_sr + (x - r * P.g) * P.q_sh);
+            };
+            qa_raw = pair(hq);
+            qb_raw = pair(hq + 4);
+            if constexpr (WIDE) {
+                qc_raw = pair(hq + 8);
+                qd_raw = pair(hq + 12);
+            }
         } else {
             const uint16_t* q0 = P.q + bi * P.q_sb + (hk * g) * P.q_sh + (lane & 15) * 8;
             qa_raw = load_untracked(q0 + (hq < g ? hq : 0) * P.q_sh);
@@ -1582,8 +1859,10 @@ void fwd_splitkv_kernel(FwdParams P) {
         issue_first_rows<BITS, GS, KT, FEW>(A, lane * 16, region_lds);
         PROF(15);
         wait_then_take<C::DEPTH - 1>(qa, qb, qa_raw, qb_raw);
+        if constexpr (WIDE) wait_then_take<C::DEPTH - 1>(qc, qd, qc_raw, qd_raw);
     } else {
         wait_then_take<0>(qa, qb, qa_raw, qb_raw);
+        if constexpr (WIDE) wait_then_take<0>(qc, qd, qc_raw, qd_raw);
     }
     if (P.nsplit > 1 && wave == 0) {
         // Which slot of the split workspace this launch uses: a word per head next to its counter, flipped by the
@@ -1615,13 +1894,21 @@ void fwd_splitkv_kernel(FwdParams P) {
         for (int i = 0; i < 4; ++i) {
             qa[i] ^= 0x80008000u;
             qb[i] ^= 0x80008000u;
+            if constexpr (WIDE) {
+                qc[i] ^= 0x80008000u;
+                qd[i] ^= 0x80008000u;
+            }
         }
     }
     {
         uint8_t* dst = sq + (lane >> 4) * kQRowBytes + (lane & 15) * 16;
         *reinterpret_cast<h8*>(dst) = cvt_h8<BF16>(qa);
         *reinterpret_cast<h8*>(dst + 4 * kQRowBytes) = cvt_h8<BF16>(qb);
-        if (lane < kZeroBytes / 16) *reinterpret_cast<u4*>(sq + kZeroRow + lane * 16) = u4{0, 0, 0, 0};
+        if constexpr (WIDE) {
+            *reinterpret_cast<h8*>(dst + 8 * kQRowBytes) = cvt_h8<BF16>(qc);
+            *reinterpret_cast<h8*>(dst + 12 * kQRowBytes) = cvt_h8<BF16>(qd);
+        }
+        if (!WIDE && lane < kZeroBytes / 16) *reinterpret_cast<u4*>(sq + kZeroRow + lane * 16) = u4{0, 0, 0, 0};
     }
     // (head slots past the group hold head 0 again: finite values whose results are never stored)
     const QRows Q = q_rows(sq, head, kg, lo_part);
@@ -1645,17 +1932,17 @@ void fwd_splitkv_kernel(FwdParams P) {
         TokenQ<NCG> KQ;
         const TokenQ<NCG>* KQp = nullptr;
         if constexpr (KT) {
-            KQ = token_q<BITS, NCG>(Q);
+            KQ = token_q<BITS, NCG, WIDE>(Q);
             KQp = &KQ;
         }
         int kslot = 0;
         for (int un = u + NW; un < u1; un += NW) {        // units that have a successor: it is fetched from inside
             const UnitAddr<BITS, GS> An = unit_addr<BITS, GS, KT>(P, bi, hk, un);
-            compute_unit<BITS, GS, BF16, true, KT, FEW>(region, region_lds, kslot, A, An, Q, P, lane, lo_part, mg, st, KQp);
+            compute_unit<BITS, GS, BF16, true, KT, FEW, WIDE>(region, region_lds, kslot, A, An, Q, P, lane, lo_part, mg, st, KQp);
             A = An;
             kslot ^= 1;
         }
-        compute_unit<BITS, GS, BF16, false, KT, FEW>(region, region_lds, kslot, A, A, Q, P, lane, lo_part, mg, st, KQp);
+        compute_unit<BITS, GS, BF16, false, KT, FEW, WIDE>(region, region_lds, kslot, A, A, Q, P, lane, lo_part, mg, st, KQp);
     }
     PROF(3);
     // ---- fp16 window tiles of this wave (the region becomes the V-transpose slab)
@@ -1675,7 +1962,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             while (true) {
                 const int tn = t + stride;
                 const bool more = tn < nT;
-                fp16_tile<BF16, NCG>(T, P, t * 16, R, lane_w, Q, lo_part, st, slab, p_shift(BITS));
+                fp16_tile<BF16, NCG, WIDE>(T, P, t * 16, R, lane_w, Q, lo_part, st, slab, p_shift(BITS));
                 if (!more) break;
                 load_fp16_tile<APPEND>(T, W, tn * 16, R, lane_w, r_new);
                 t = tn;
@@ -1712,13 +1999,13 @@ void fwd_splitkv_kernel(FwdParams P) {
     const float lsum = st.l[0];
     float bias[NCG];      // V bias of the lane's column: the zero part, which both columns hold, is taken from the hi one
 #pragma unroll
-    for (int c = 0; c < NCG; ++c) bias[c] = st.ob[c][0] + (lo_part ? 0.0f : st.zb[c]);
+    for (int c = 0; c < NCG; ++c) bias[c] = st.ob[c][0] + (!WIDE && lo_part ? 0.0f : st.zb[c]);
 #pragma unroll
     for (int ct = 0; ct < 8; ++ct) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
             const float v = st.o[ct][r] + bias[ct / (GS / 16)];
-            st.o[ct][r] = v + partner(v);      // hi + lo
+            st.o[ct][r] = WIDE ? v : v + partner(v);      // hi + lo
         }
     }
     if (col < g) {
@@ -1728,7 +2015,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             *reinterpret_cast<f4*>(&sO[col * kHeadDim + 16 * ct + 4 * kg]) = st.o[ct];
         }
     }
-    if (kg == 0 && col < kMaxGroupHeads) {
+    if (kg == 0 && col < kCols) {
         sM[col * NW + wave] = col < g ? st.m * P.scale_log2 : -INFINITY;     // base-2 units
         sL[col * NW + wave] = col < g ? lsum : 0.0f;
     }
@@ -1760,6 +2047,10 @@ void fwd_splitkv_kernel(FwdParams P) {
     // that read it had ended.  What would break it: a workspace in host-coherent or fine-grained memory with other
     // scope rules, two launches in flight on one workspace, another shape on a workspace that was not zeroed
     // again, or a workspace that was not zero at its first launch.
+    if constexpr (WIDE) {
+        wide_tail<BITS, NW, REGION, BF16>(P, lds, sM, sL, s_cnt, wave, lane, g, bi, hk, blk, h0, split, n_h, lo_words, slot_words, lo_from);
+        return;
+    }
     bool last = false;
     float O0 = 0.0f, O1 = 0.0f, M = -INFINITY, L = 0.0f;
     // loads in flight of the wave that merges the splits (merge_splits): 16 where the kernel is at its register limit
@@ -1779,7 +2070,7 @@ void fwd_splitkv_kernel(FwdParams P) {
     uint16_t* out_row = out + bi * out_sb + hq * out_sh;
     float* lse_row = lse_out ? lse_out + hrow : nullptr;
     if constexpr (ROWS) {
-        const int x = kMaxGroupHeads * blk + wave, row = div_magic(x, P.g_magic);
+        const int x = kCols * blk + wave, row = div_magic(x, P.g_magic);
         const int head_of_row = hk * P.g + x - row * P.g;
         out_row = out + bi * out_sb + row * P.out_sr + head_of_row * out_sh;
         if (lse_out) lse_row = lse_out + (static_cast<int64_t>(bi) * P.rows + row) * (P.g * P.hk) + head_of_row;
@@ -1869,21 +2160,21 @@ void fwd_splitkv_kernel(FwdParams P) {
     PROF_FLUSH();
 }
 
-template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, bool ROWS>
+template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, int ROWS_KIND>
 hipError_t launch_fwd_ttt(const FwdParams& P, hipStream_t stream) {
-    constexpr int kLds = fwd_lds_bytes<BITS, GS, FEW>();
+    constexpr int kLds = fwd_lds_bytes<BITS, GS, FEW, ROWS_KIND == kRowsWide>();
     // the dynamic-LDS limit is raised once per kernel and device (idempotent, so a race between
     // two host threads only repeats the call)
     static std::atomic<bool> configured[64] = {};
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return e;
     if (dev < 0 || dev >= 64 || !configured[dev].load(std::memory_order_acquire)) {
-        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW, ROWS>),
+        hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(&fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW, ROWS_KIND>),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, kLds);
         if (e != hipSuccess) return e;
         if (dev >= 0 && dev < 64) configured[dev].store(true, std::memory_order_release);
     }
-    hipLaunchKernelGGL((fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW, ROWS>), dim3(P.nsplit * P.hk * P.b * (ROWS ? P.row_blocks : 1)),
+    hipLaunchKernelGGL((fwd_splitkv_kernel<BITS, GS, BF16, APPEND, KT, FEW, ROWS_KIND>), dim3(P.nsplit * P.hk * P.b * (ROWS_KIND != kRowsNone ? P.row_blocks : 1)),
                        dim3(UnitCfg<BITS, GS, FEW>::NW * 64), kLds, stream, P);
     return hipGetLastError();
 }
@@ -1894,19 +2185,20 @@ hipError_t launch_fwd_ttt(const FwdParams& P, hipStream_t stream) {
 // 128K tokens and from 1 to 16 sequences of equal length.  The 16 waves keep more bytes in flight per compute
 // unit, which only pays when a few workgroups are left streaming alone (ragged batches).  A 2-bit unit admits
 // only four rows in flight, and there the 8 waves lose 2-3 %: not built.
-template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool ROWS>
+template <int BITS, int GS, bool BF16, bool APPEND, bool KT, int ROWS_KIND>
 hipError_t launch_fwd_tt(const FwdParams& P, hipStream_t stream) {
     if constexpr (few_waves_variant(BITS, GS)) {
-        if (P.few_waves) return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, true, ROWS>(P, stream);
+        if (P.few_waves) return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, true, ROWS_KIND>(P, stream);
     }
-    return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, false, ROWS>(P, stream);
+    return launch_fwd_ttt<BITS, GS, BF16, APPEND, KT, false, ROWS_KIND>(P, stream);
 }
 
 template <int BITS, int GS, bool BF16, bool KT>
 hipError_t launch_fwd_b(const FwdParams& P, hipStream_t stream) {
-    if (P.lengths) return launch_fwd_tt<BITS, GS, BF16, true, KT, false>(P, stream);
-    return P.rows > 1 ? launch_fwd_tt<BITS, GS, BF16, false, KT, true>(P, stream)
-                      : launch_fwd_tt<BITS, GS, BF16, false, KT, false>(P, stream);
+    if (P.lengths) return launch_fwd_tt<BITS, GS, BF16, true, KT, kRowsNone>(P, stream);
+    if (P.rows_wide) return launch_fwd_ttt<BITS, GS, BF16, false, KT, true, kRowsWide>(P, stream);
+    return P.rows > 1 ? launch_fwd_tt<BITS, GS, BF16, false, KT, kRowsFew>(P, stream)
+                      : launch_fwd_tt<BITS, GS, BF16, false, KT, kRowsNone>(P, stream);
 }
 
 template <int BITS, int GS>

@@ -117,8 +117,9 @@ struct FwdParams {
     const uint16_t* k_new;
     const uint16_t* v_new;
     int64_t knew_sb, knew_sh, vnew_sb, vnew_sh;
-    // Several query rows per sequence (rows > 1): the rows * g pairs of a kv head in blocks of eight (decode.hip, ROWS);
-    // h then counts pairs (rows * query heads).
+    // Several query rows per sequence (rows > 1): the rows * g pairs of a kv head in blocks of eight or (rows_wide) sixteen
+    // (decode.hip, ROWS); h then counts pairs (rows * query heads).
+    int rows_wide;
     int rows, row_blocks;
     uint32_t row_blocks_magic, g_magic;
     int64_t q_sr, out_sr;

@@ -44,6 +44,8 @@ namespace bitdecode {
 constexpr int kHeadDim = 128;
 constexpr int kChunk = 128;               // tokens per chunk (pack granularity)
 constexpr int kMaxGroupHeads = 8;         // query heads per kv head handled by one MFMA tile
+constexpr int kWidePairs = 16;            // (query row, query head) pairs per workgroup where there are more than kMaxGroupHeads of them
+enum { kRowsNone, kRowsFew, kRowsWide };  // one query row; several, in blocks of kMaxGroupHeads pairs; in blocks of kWidePairs
 
 // bytes of K (or V) codes per chunk
 constexpr int chunk_code_bytes(int bits) { return kChunk * kHeadDim * bits / 8; }

@@ -467,8 +467,8 @@ def plan_fwd_kvcache_int(q: torch.Tensor,
     a.quant_mode = mode
     a.softmax_scale = float(softmax_scale)
     with _on_device(device):
-        # (several query rows: a workgroup per eight row and head pairs of a kv head, workspace rows by pairs)
-        blocks = 1 if m == 1 else (m * (h // h_k) + 7) // 8
+        # (several query rows: a workgroup per block of row and head pairs of a kv head, workspace rows by pairs)
+        blocks = 1 if m == 1 else _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), a.max_seqlen_k, 0, num_bits)
         ns, nbytes = _split_plan(device.index, b, h * m, h_k * blocks, a.max_seqlen_k, a.max_res_len,
                                  seqlens_k is not None, num_bits, group_size, int(num_splits))
         a.num_splits = ns
@@ -535,10 +535,10 @@ def _fwd_query_rows(q, k_pack, k_params, v_pack, v_params, opt_block_table, soft
         q = q.clone(memory_format=torch.contiguous_format)
     # A launch takes at most 4096 rows, and a split one's workspace, a record of 1040 bytes per row, head and split, is below 2
     # GiB: more than that goes in several launches.  Where the split count is left to the library, launches of many rows are
-    # not split; they are cut at half a million rows x heads (and never below the eight of a workgroup: at 256 sequences of 32
+    # not split; they are cut at half a million rows x heads (and never below the sixteen of a workgroup: at 256 sequences of 32
     # heads already, launches of fewer rows read the cache twice).
     splits = int(kwargs.get("num_splits", 0))
-    rows = 2000000 // splits // max(1, b * h) if splits > 1 else max(8 // (h // h_k), 524288 // max(1, b * h))
+    rows = 2000000 // splits // max(1, b * h) if splits > 1 else max(16 // (h // h_k), 524288 // max(1, b * h))
     per = max(1, min(4096, rows))
     if m > per or (out is not None and out.stride(3) != 1):
         res = out if out is not None else torch.empty_like(q)

@@ -19,7 +19,7 @@
 extern "C" {
 #endif
 
-#define BITDECODE_ABI_VERSION 6
+#define BITDECODE_ABI_VERSION 7
 
 enum {
     BITDECODE_OK = 0,
@@ -140,7 +140,8 @@ int bitdecode_fwd_static(const bitdecode_fwd_args* args, void* stream);
  * 358-368; its interface fixes is_causal = False, so every row attends every key).  In `fwd`: q and out are
  * [b, rows, h, 128], softmax_lse is [b, rows, h]; the workspace is sized, and zeroed for another shape, as for
  * rows * h heads: bitdecode_fwd_workspace_bytes(b, rows * h, num_splits).  The rows * (h / h_k) row and head pairs
- * of a kv head run in blocks of eight, one workgroup each: bitdecode_num_splits(_for) wants h_k * ceil(that / 8). */
+ * of a kv head run in blocks of eight or sixteen, one workgroup each: bitdecode_num_splits(_for) wants
+ * h_k * bitdecode_row_blocks(b, h_k, pairs, max_seqlen_k, num_cus (0: the current device's), bits).  num_splits = 0 chooses no more splits than the workspace holds. */
 typedef struct bitdecode_fwd_rows_args {
     bitdecode_fwd_args fwd;
     int32_t rows;              /* query rows per sequence, 1 to 4096                        */
@@ -149,6 +150,7 @@ typedef struct bitdecode_fwd_rows_args {
 } bitdecode_fwd_rows_args;
 
 int bitdecode_fwd_rows(const bitdecode_fwd_rows_args* args, void* stream);
+int bitdecode_row_blocks(int32_t b, int32_t h_k, int32_t pairs, int32_t max_seqlen_k, int32_t num_cus, int32_t bits);
 
 /* One decode step in one launch: attend the new token together with everything held, append it, and
  * quantize-pack the fp16 window when it fills.  This is the "residual kernel" the reference's figures

@@ -1,4 +1,4 @@
-"""Several query rows per sequence in one launch: the (row, head) pairs of a kv head run in blocks of eight."""
+"""Several query rows per sequence in one launch: the (row, head) pairs of a kv head run in blocks of eight or sixteen."""
 import math
 
 import pytest
@@ -111,3 +111,52 @@ def test_many_sequences_take_their_rows_in_one_launch(device):
     assert len(interface._plan_cache()) == 1
     for r in (0, 5, 7):
         assert torch.equal(out[:, r:r + 1], fwd_kvcache_int(q[:, r:r + 1].contiguous(), *cache, None, SCALE, "k-channel", 128, 4))
+
+
+@pytest.mark.parametrize("b,h,h_k,m,S,bits,gs,mode,dtype,ns", [
+    (8, 6, 2, 3, 128 * 130, 4, 128, "k-channel", "fp16", 5),      # 9 pairs: a block of sixteen with seven empty columns
+    (7, 8, 1, 4, 128 * 260, 2, 64, "k-channel", "bf16", 33),      # 32 pairs, more splits than a round of the merge takes
+    (9, 5, 5, 17, 128 * 36, 4, 32, "k-channel", "bf16", 1),       # 17 pairs: last block of one, one split
+    (16, 8, 2, 5, 128 * 65, 4, 64, "k-tensor", "fp16", 0),        # 20 pairs
+    (24, 16, 2, 4, 128 * 33, 2, 128, "k-channel", "fp16", 17),
+    (24, 16, 2, 2, 128 * 50, 2, 32, "k-channel", "fp16", 2),
+])
+def test_blocks_of_sixteen_equal_the_calls_for_each_row(device, b, h, h_k, m, S, bits, gs, mode, dtype, ns):
+    """As above, at sizes that run in blocks of sixteen: unequal lengths, windows, an empty sequence, outputs large enough for
+    the residual words in one sequence.  The LSE bound is that of the scores' fp32 sums, the output's the rounding of two
+    records and an output (2^-11 each of the sequence's values)."""
+    from bitladder_amd import _lib, fwd_kvcache_int, kvcache_pack_int
+    assert _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), S, 256, bits) == -(-m * (h // h_k) // 16)
+    R, tdt = 53, H.torch_dtype(dtype)
+    g = torch.Generator(device=device).manual_seed(m)
+    k, v = (torch.randn((b, S + R, h_k, 128), generator=g, device=device).to(tdt) for _ in range(2))
+    k[..., [5, 40, 99]] *= 6
+    v[1] *= 40                                              # residual words
+    q = torch.randn((b, h, m, 128), generator=g, device=device).to(tdt).transpose(1, 2)
+    cache = H.alloc_cache(b, S, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
+    kvcache_pack_int(k[:, :S], cache[0], cache[1], v[:, :S], cache[2], cache[3], None, None, S, mode, gs, bits)
+    lens = torch.full((b,), S, dtype=torch.int32, device=device)
+    res = torch.full((b,), R, dtype=torch.int32, device=device)
+    lens[2], lens[3], res[3], res[4] = 384, 0, 0, 1
+    kw = dict(seqlens_k=lens, k_residual=k[:, S:], v_residual=v[:, S:], residual_len=res, return_lse=True)
+    args = (*cache, None, SCALE, mode, gs, bits)
+    for flip in (1, -1, 1):                                 # launch after launch on one workspace, other queries in between
+        out, lse = fwd_kvcache_int(q * flip, *args, num_splits=ns, **kw)
+    assert torch.isinf(lse[3]).all() and not out[3].any()
+    scale_of = v.float().abs().amax((1, 2, 3)).reshape(b, 1, 1, 1) / 4
+    for r in sorted({0, 1, m // 2, m - 1}):
+        one, lse1 = fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args, num_splits=min(ns, 4), **kw)
+        err = (out[:, r:r + 1].float() - one.float()).abs()
+        bound = 1.5e-3 * scale_of + (2 ** -7 * one.float().abs() if dtype == "bf16" else 0)
+        assert (err <= bound).all(), (r, (err - bound).max().item())
+        ok = lens + res > 0
+        assert (lse[ok, r] - lse1[ok]).abs().max().item() < 5e-4, r
+
+
+def test_few_rows_stay_in_blocks_of_eight(device):
+    """Where eight pairs a workgroup are the faster choice the row blocks say so, whatever the sizes."""
+    from bitladder_amd import _lib
+    blocks = lambda *a: _lib.lib().bitdecode_row_blocks(*a)
+    assert [blocks(2, 8, p, 8192, 256, 4) for p in (1, 8, 9, 32)] == [1, 1, 2, 2]
+    assert blocks(1, 8, 32, 4096, 256, 4) == 4 and blocks(3, 8, 32, 4096, 256, 2) == 4 and blocks(4, 8, 64, 2048, 256, 2) == 4
+    assert blocks(1, 1, 64, 65536, 256, 4) == 8 and blocks(1, 1, 64, 131072, 256, 4) == 4 and blocks(1, 1, 64, 131072, 256, 2) == 8
