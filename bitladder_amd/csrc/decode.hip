@@ -499,33 +499,35 @@ struct UnitAddr {
     const uint8_t* kp;
     const uint8_t* vp;
 };
+// region: byte offset of the (batch, kv-head)'s codes in a contiguous cache (unit_region)
+__device__ __forceinline__ int64_t unit_region(const FwdParams& P, int bi, int hk) {
+    return (static_cast<int64_t>(bi) * P.hk + hk) * P.kpack_bh;
+}
 template <int BITS, int GS, bool KT = false>
-__device__ __forceinline__ UnitAddr<BITS, GS> unit_addr(const FwdParams& P, int bi, int hk, int u) {
+__device__ __forceinline__ UnitAddr<BITS, GS> unit_addr(const FwdParams& P, int64_t region, int bi, int hk, int u) {
     using C = UnitCfg<BITS, GS>;
-    const int uic = u % C::UPC;
-    // region and chunk inside it, as layout.h::chunk_place; a paged cache looks the page up in the block
-    // table with a scalar load written out here: a load the compiler tracks would be a vector load, and its
-    // wait would also drain the direct-to-LDS loads in flight
-    int ci = u / C::UPC;
-    int64_t bh = static_cast<int64_t>(bi) * P.hk + hk;
+    // Codes of K and V lie alike, so one byte offset serves both: units follow one another in the region.  A paged cache looks
+    // region and chunk up in the block table (layout.h::chunk_place) with a scalar load written out here: a load the compiler
+    // tracks would be a vector load, and its wait would also drain the direct-to-LDS loads in flight
+    int64_t off = region + static_cast<int64_t>(u) * 4096;
     if (P.block_table) {
-        const int slot = ci / P.chunks_per_page;
+        const int ci = u / C::UPC, slot = ci / P.chunks_per_page;
         int page;
         asm volatile("s_load_dword %0, %1, 0x0\n\ts_waitcnt lgkmcnt(0)"
                      : "=s"(page) : "s"(P.block_table + bi * P.bt_stride + slot) : "memory");
-        bh = static_cast<int64_t>(page) * P.hk + hk;
-        ci -= slot * P.chunks_per_page;
+        off = (static_cast<int64_t>(page) * P.hk + hk) * P.kpack_bh + static_cast<int64_t>(u - slot * P.chunks_per_page * C::UPC) * 4096;
     }
+    // Parameters take 512 / GS bytes a token, codes 16 * BITS: their offsets are the codes' shifted right.  (K parameters of
+    // a group wider than a unit: from the group's start.)  Four products of region strides per unit before, 50 of 80 scalar
+    // instructions per unit: 8 sequences of 1K-8K 13.5 -> 13.2 us, 6 paged ones of 10K at group 32 17.0 -> 16.7.
+    constexpr int kShift = __builtin_ctz(BITS * GS / 32);
+    static_assert((4096 >> kShift) == C::VPB && (KT ? C::KPB_T : C::KPB) == (KT || GS <= C::UT ? C::VPB : kKParamGroupBytes), "parameter offsets");
+    const int64_t par = off >> kShift;
     UnitAddr<BITS, GS> A;      // wave-uniform: everything here lives in SGPRs
-    A.kc = P.k_pack + bh * P.kpack_bh + static_cast<int64_t>(ci) * chunk_code_bytes(BITS) + uic * 4096;
-    A.vc = P.v_pack + bh * P.vpack_bh + static_cast<int64_t>(ci) * chunk_code_bytes(BITS) + uic * 4096;
-    if constexpr (KT) {      // per-token K parameters: [64-token half][channel group][tile][token] per chunk
-        A.kp = P.k_params + bh * P.kparams_bh + static_cast<int64_t>(ci) * v_param_chunk_bytes(GS) + uic * C::KPB_T;
-    } else {
-        A.kp = P.k_params + bh * P.kparams_bh +
-               (static_cast<int64_t>(ci) * (kChunk / GS) + (uic * C::UT) / GS) * kKParamGroupBytes;
-    }
-    A.vp = P.v_params + bh * P.vparams_bh + static_cast<int64_t>(ci) * v_param_chunk_bytes(GS) + uic * C::VPB;
+    A.kc = P.k_pack + off;
+    A.vc = P.v_pack + off;
+    A.kp = P.k_params + (KT || GS <= C::UT ? par : par & ~static_cast<int64_t>(kKParamGroupBytes - 1));
+    A.vp = P.v_params + par;
     return A;
 }
 // BYTES contiguous bytes (a multiple of 256) into LDS: whole 1 KB rows, the last one with only the
@@ -1671,13 +1673,10 @@ __device__ __forceinline__ void step_end(uint8_t* lds, int bi, int hk, int t) {
 // a launch is that of the unit whose two workgroups add up to the most.  The dispatcher fills the units
 // round-robin, so the workgroups at batch positions p and p + b/2 share a unit: position p takes the p-th
 // longest sequence and position ceil(b/2) + k the k-th shortest, which pairs the longest with the shortest.
-// A permutation of the batch index computed by every wave from the device-side lengths (lane j holds sequence
+// A permutation of the batch index computed by every wave from the device-side lengths (lane j < n holds that of sequence
 // j; equal lengths are ordered by index), so every workgroup arrives at the same one; the lengths are not
 // written during the launch.  Nothing else depends on it: results are indexed by the sequence.
-__device__ __forceinline__ int sequence_of_position(const FwdParams& P, int p, int lane) {
-    const int n = P.b;      // at most 64 (host)
-    int len = -1;
-    if (lane < n) len = min(max(P.seqlens[lane], 0), P.capacity);
+__device__ __forceinline__ int sequence_of_position(int len, int n, int p, int lane) {      // n at most 64 (host)
     int rank = 0;           // sequences that come before this lane's in descending order of length
     for (int j = 0; j < n; ++j) {
         const int lj = __builtin_amdgcn_readlane(len, j);
@@ -1736,7 +1735,8 @@ void fwd_splitkv_kernel(FwdParams P) {
     // Everything a workgroup needs before its first loads of the stream is asked for here, in the kernel's first
     // basic block (the fields are the head of the parameter block, kernels.h): left alone, the compiler fetches a
     // field behind the branch that first uses it, four or five rounds of scalar loads one after the other, half a
-    // microsecond in which the memory system has nothing to do.  The rest is read where it is used.
+    // microsecond in which the memory system has nothing to do.  The rest is read where it is used.  (Fields that are not used,
+    // the region strides behind kpack_bh, are named so that the loads stay few and wide: without them 0.1 us on every short call.)
     asm volatile("" : : "s"(P.nsplit), "s"(P.hk), "s"(P.g), "s"(P.b), "s"(P.nsplit_magic), "s"(P.hk_magic), "s"(P.seqlen),
                  "s"(P.reslen), "s"(P.capacity), "s"(P.res_cap), "s"(P.xcd_remap), "s"(P.seq_perm), "s"(P.seqlens),
                  "s"(P.reslens), "s"(P.q), "s"(P.q_sb), "s"(P.q_sh), "s"(P.k_pack), "s"(P.k_params), "s"(P.v_pack),
@@ -1793,8 +1793,25 @@ void fwd_splitkv_kernel(FwdParams P) {
     }
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave-uniform: unit addresses stay in SGPRs
+    int S, R, r_new = -1, step_len = 0;
     if constexpr (!APPEND) {
-        if (P.seq_perm) bi = sequence_of_position(P, bi, lane);
+        S = P.seqlen;
+        R = P.reslen;
+        if (P.seqlens || P.reslens) {
+            // Both lengths in one round trip, and where the sequences are dealt out by length out of the same loads (three dependent round
+            // trips before; 8 to 16 sequences of 1K-8K 0.1 us of 11 to 14, and as much for the calls that skip this: less code
+            // in front of their first load).  Values the host never saw: kept inside the cache and the window.
+            const int* const sl = P.seqlens ? P.seqlens : P.reslens;
+            const int* const rl = P.reslens ? P.reslens : P.seqlens;
+            const int j = P.seq_perm ? min(lane, P.b - 1) : bi;
+            int s_dev = sl[j], r_dev = rl[j];
+            s_dev = min(max(s_dev, 0), P.capacity);
+            r_dev = min(max(r_dev, 0), P.res_cap);
+            if (P.seq_perm) bi = sequence_of_position(s_dev, P.b, bi, lane);
+            const int src = P.seq_perm ? bi : 0;
+            if (P.seqlens) S = __builtin_amdgcn_readlane(s_dev, src);
+            if (P.reslens) R = __builtin_amdgcn_readlane(r_dev, src);
+        }
     }
     const int col = lane & 15, kg = lane >> 4;
     const int head = WIDE ? col : col & 7;          // query head inside the GQA group (ROWS: pair inside the block)
@@ -1803,16 +1820,11 @@ void fwd_splitkv_kernel(FwdParams P) {
     const int g = ROWS ? min(kCols, P.g * P.rows - kCols * blk) : P.g;
     const int h0 = ROWS ? hk * P.g * P.rows + kCols * blk : hk * P.g;
 
-    int S, R, r_new = -1, step_len = 0;
     if constexpr (APPEND) {
         step_len = step_length(P, bi);
         r_new = step_len & (kChunk - 1);
         S = min(step_len - r_new, P.capacity);     // a length beyond the capacity is the caller's error: stay inside
         R = r_new + 1;
-    } else {
-        // per-sequence values are device data the host never saw: keep them inside the cache and the window
-        S = P.seqlens ? min(max(P.seqlens[bi], 0), P.capacity) : P.seqlen;
-        R = P.reslens ? min(max(P.reslens[bi], 0), P.res_cap) : P.reslen;
     }
     const int nU = (S / kChunk) * C::UPC;
     const int ups = div_magic(nU + P.nsplit - 1, P.nsplit_magic);
@@ -1852,9 +1864,10 @@ void fwd_splitkv_kernel(FwdParams P) {
         }
     }
     PROF(13);
+    const int64_t region_off = unit_region(P, bi, hk);
     UnitAddr<BITS, GS> A;
     if (u < u1) {
-        A = unit_addr<BITS, GS, KT>(P, bi, hk, u);
+        A = unit_addr<BITS, GS, KT>(P, region_off, bi, hk, u);
         PROF(14);
         issue_first_rows<BITS, GS, KT, FEW>(A, lane * 16, region_lds);
         PROF(15);
@@ -1937,7 +1950,7 @@ void fwd_splitkv_kernel(FwdParams P) {
         }
         int kslot = 0;
         for (int un = u + NW; un < u1; un += NW) {        // units that have a successor: it is fetched from inside
-            const UnitAddr<BITS, GS> An = unit_addr<BITS, GS, KT>(P, bi, hk, un);
+            const UnitAddr<BITS, GS> An = unit_addr<BITS, GS, KT>(P, region_off, bi, hk, un);
             compute_unit<BITS, GS, BF16, true, KT, FEW, WIDE>(region, region_lds, kslot, A, An, Q, P, lane, lo_part, mg, st, KQp);
             A = An;
             kslot ^= 1;
