@@ -488,10 +488,12 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     // (the built-in scratch takes every call that leaves the count to the library: it chooses no more than fits)
     while (static_scratch && a->num_splits == 0 && nsplit > 1 && slots_bytes(a->b, n_h, nsplit) > kStaticScratchBytes - kStaticCounterBytes)
         --nsplit;
-    // (several query rows, count left to the library: no more splits than the caller's workspace holds, which it may have sized for
-    // a count of its own)
-    while (rows_args && a->num_splits == 0 && nsplit > 1 && bitdecode_fwd_workspace_bytes(a->b, n_h, nsplit) > (a->workspace ? a->workspace_bytes : 0))
-        --nsplit;
+    // (several query rows in blocks of sixteen, count left to the library: a workspace that holds the count of blocks of eight, which
+    // a caller may have asked for, is taken, with no more splits than it holds)
+    if (wide && a->num_splits == 0) {
+        const int least = choose_splits_for(a->b, a->h_k * row_blocks_of(rows * g, false), max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k != nullptr);
+        while (nsplit > least && bitdecode_fwd_workspace_bytes(a->b, n_h, nsplit) > (a->workspace ? a->workspace_bytes : 0)) --nsplit;
+    }
     if (nsplit > 1 && slots_bytes(a->b, n_h, nsplit) >= (size_t(1) << 31))
         return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d heads: partial outputs of 2 GiB or more", nsplit, a->b, n_h);
     // the kernel divides workgroup ids and unit counts by the split count and the head count with a
@@ -577,6 +579,7 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     uint8_t* ws = static_cast<uint8_t*>(a->workspace);
     if (step) {
         P.lengths = step->lengths;
+        P.seqlens = step->lengths;      // (decode.hip: step_length)
         P.step_tickets = reinterpret_cast<int*>(ws);
         ws += step_ticket_bytes(a->b);
         P.k_new = static_cast<const uint16_t*>(step->k_new);

@@ -30,9 +30,9 @@
 //  * The offset/zero biases and the softmax row sums are themselves computed on the MFMA pipe
 //    (A operand = the zero vector / the constant offsets / ones), which keeps the VALU for the
 //    code unpacking; this kernel is VALU-issue bound long before it is MFMA bound.
-//  * Online softmax in base 2 per head (softmax.h:250-310) in steps of 64 tokens: running max
+//  * Online softmax in base 2 per head (softmax.h:250-310) in steps of 64 tokens: maxima
 //    shared by the four lanes of a head through two lane-half swaps, accumulators rescaled only
-//    when some head's max actually moved.
+//    when some head's score exceeds its reference, which lies above the largest score so far (kHeadroom).
 //  * The waves of a workgroup merge through LDS, one wave per query head; splits merge in the
 //    same launch: that wave publishes the head's record (O / sum in fp16, max, sum) without waiting
 //    for the stores, an idle wave has meanwhile drawn a ticket from the head's counter, and the wave
@@ -1589,7 +1589,9 @@ __device__ __forceinline__ void wide_tail(const FwdParams& P, const uint8_t* lds
 // ---------------------------------------------------------------------------------------------
 // The length is stable for every workgroup that reads it: it is advanced only after all workgroups of
 // the sequence have drawn their tickets.
-__device__ __forceinline__ int step_length(const FwdParams& P, int bi) { return P.lengths[bi]; }
+// (read through `seqlens`, which holds the same pointer in a step: the field comes with the first kernel arguments, `lengths`
+// behind them cost a round of loads of its own, 0.2 us a step)
+__device__ __forceinline__ int step_length(const FwdParams& P, int bi) { return P.seqlens[bi]; }
 // A sequence whose window is about to fill while its cache has no room for another chunk cannot
 // take the token: it is attended, but neither stored nor counted.
 __device__ __forceinline__ bool step_overflows(int capacity, int t) {
@@ -1742,6 +1744,7 @@ void fwd_splitkv_kernel(FwdParams P) {
                  "s"(P.reslens), "s"(P.q), "s"(P.q_sb), "s"(P.q_sh), "s"(P.k_pack), "s"(P.k_params), "s"(P.v_pack),
                  "s"(P.v_params), "s"(P.block_table), "s"(P.kpack_bh), "s"(P.kparams_bh), "s"(P.vpack_bh), "s"(P.vparams_bh),
                  "s"(P.bt_stride), "s"(P.chunks_per_page), "s"(P.neg_scale), "s"(P.scale_log2));
+    if constexpr (ROWS) asm volatile("" : : "s"(P.rows), "s"(P.row_blocks), "s"(P.row_blocks_magic), "s"(P.g_magic), "s"(P.q_sr), "s"(P.out_sr));
     if constexpr (kLateArgs && !KT) asm volatile("" : : "s"(P.tickets), "s"(P.h));      // (for the slot words below)
     if constexpr (!kLateArgs) {
         asm volatile("" : : "s"(P.k_res), "s"(P.v_res), "s"(P.kres_sb), "s"(P.kres_st), "s"(P.kres_sh), "s"(P.vres_sb),

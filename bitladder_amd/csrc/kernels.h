@@ -111,7 +111,7 @@ struct FwdParams {
     // Decode step with append (lengths != nullptr): sequence i holds lengths[i] tokens, the last
     // lengths[i] % 128 of them in the fp16 window; its new token (k_new, v_new) is attended as the
     // window's next row, stored there, and a window that becomes full is packed behind the prefix.
-    // seqlens / reslens / seqlen / reslen are not used then.
+    // reslens / seqlen / reslen are not used then; seqlens holds the same pointer.
     int* lengths;               // [b], advanced by one by the last workgroup of each sequence
     int* step_tickets;          // [b] arrival counters, kTicketStride ints apart, zero between calls
     const uint16_t* k_new;

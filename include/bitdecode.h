@@ -141,7 +141,8 @@ int bitdecode_fwd_static(const bitdecode_fwd_args* args, void* stream);
  * [b, rows, h, 128], softmax_lse is [b, rows, h]; the workspace is sized, and zeroed for another shape, as for
  * rows * h heads: bitdecode_fwd_workspace_bytes(b, rows * h, num_splits).  The rows * (h / h_k) row and head pairs
  * of a kv head run in blocks of eight or sixteen, one workgroup each: bitdecode_num_splits(_for) wants
- * h_k * bitdecode_row_blocks(b, h_k, pairs, max_seqlen_k, num_cus (0: the current device's), bits).  num_splits = 0 chooses no more splits than the workspace holds. */
+ * h_k * bitdecode_row_blocks(b, h_k, pairs, max_seqlen_k, num_cus (0: the current device's), bits).  With
+ * num_splits = 0 a workspace sized for blocks of eight (h_k * ceil(pairs / 8)) is taken as well. */
 typedef struct bitdecode_fwd_rows_args {
     bitdecode_fwd_args fwd;
     int32_t rows;              /* query rows per sequence, 1 to 4096                        */

@@ -160,3 +160,30 @@ def test_few_rows_stay_in_blocks_of_eight(device):
     assert [blocks(2, 8, p, 8192, 256, 4) for p in (1, 8, 9, 32)] == [1, 1, 2, 2]
     assert blocks(1, 8, 32, 4096, 256, 4) == 4 and blocks(3, 8, 32, 4096, 256, 2) == 4 and blocks(4, 8, 64, 2048, 256, 2) == 4
     assert blocks(1, 1, 64, 65536, 256, 4) == 8 and blocks(1, 1, 64, 131072, 256, 4) == 4 and blocks(1, 1, 64, 131072, 256, 2) == 8
+
+
+def test_count_left_to_the_library_fits_a_workspace_sized_for_blocks_of_eight(device):
+    """The C entry with num_splits = 0: a workspace for the count of blocks of eight is taken, a smaller one refused."""
+    import ctypes
+
+    from bitladder_amd import _lib, fwd_kvcache_int, interface, kvcache_pack_int
+    g = torch.Generator(device=device).manual_seed(4)
+    k, v = (torch.randn((2, 8192, 8, 128), generator=g, device=device).half() for _ in range(2))
+    cache = H.alloc_cache(2, 8192, 8, 4, 128, device)
+    kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, 8192, "k-channel", 128, 4)
+    q = torch.randn((2, 8, 32, 128), generator=g, device=device).half()
+    want = fwd_kvcache_int(q, *cache, None, SCALE, "k-channel", 128, 4)
+    plan = interface.plan_fwd_kvcache_int(q, *cache, None, SCALE, "k-channel", 128, 4, _rows=True)
+    L, a = _lib.lib(), plan.args
+    n8 = L.bitdecode_num_splits_for(2, 8 * 4, 8192, 0, 0, 4, 128, 0)
+    assert plan.args.fwd.num_splits > n8 > 1
+    stream = torch.cuda.current_stream().cuda_stream
+    for splits, ok in ((n8, True), (n8 + 1, True), (n8 - 1, False)):
+        nbytes = L.bitdecode_fwd_workspace_bytes(2, 8 * 32, splits)
+        ws = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+        a.fwd.num_splits, a.fwd.workspace, a.fwd.workspace_bytes = 0, ws.data_ptr(), nbytes
+        plan.out.zero_()
+        assert (L.bitdecode_fwd_rows(ctypes.byref(a), stream) == 0) is ok
+        torch.cuda.synchronize()
+        if ok:      # (another split count: the rounding of the records)
+            assert (plan.out.float() - want.float()).abs().max() < 1e-3
