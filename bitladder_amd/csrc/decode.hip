@@ -2035,6 +2035,9 @@ void fwd_splitkv_kernel(FwdParams P) {
         sM[col * NW + wave] = col < g ? st.m * P.scale_log2 : -INFINITY;     // base-2 units
         sL[col * NW + wave] = col < g ? lsum : 0.0f;
     }
+    // The slot words (above) have to be in LDS before the other waves read them.  A wave with units or tiles has waited for all its loads by
+    // now, but in a split without any nothing has made wave 0 wait, and the barrier itself waits for LDS operations only.
+    wait_vm<0>();
     __syncthreads();
     PROF(4);
     if constexpr (APPEND) {

@@ -187,3 +187,38 @@ def test_count_left_to_the_library_fits_a_workspace_sized_for_blocks_of_eight(de
         torch.cuda.synchronize()
         if ok:      # (another split count: the rounding of the records)
             assert (plan.out.float() - want.float()).abs().max() < 1e-3
+
+
+@pytest.mark.parametrize("bits,gs,mode,dtype,ns", [(4, 128, "k-channel", "fp16", 5), (2, 64, "k-channel", "bf16", 9),
+                                                   (4, 64, "k-tensor", "fp16", 17)])
+def test_splits_without_work_have_some_in_the_next_launch(device, bits, gs, mode, dtype, ns):
+    """One workspace, lengths and windows that change from launch to launch: splits of a short or empty sequence have neither a unit nor a
+    tile, the same splits have both one launch later.  Bounds as for `test_blocks_of_sixteen_equal_the_calls_for_each_row`."""
+    from bitladder_amd import _lib, fwd_kvcache_int, kvcache_pack_int
+    from bitladder_amd.interface import plan_fwd_kvcache_int
+    b, h, h_k, m, S, R, tdt = 8, 16, 2, 5, 128 * 64, 128, H.torch_dtype(dtype)
+    assert _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), S, 256, bits) == 3      # blocks of sixteen
+    g = torch.Generator(device=device).manual_seed(ns)
+    k, v = (torch.randn((b, S + R, h_k, 128), generator=g, device=device).to(tdt) for _ in range(2))
+    q = torch.randn((b, m, h, 128), generator=g, device=device).to(tdt)
+    cache = H.alloc_cache(b, S, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
+    kvcache_pack_int(k[:, :S], cache[0], cache[1], v[:, :S], cache[2], cache[3], None, None, S, mode, gs, bits)
+    lens, res = (torch.zeros(b, dtype=torch.int32, device=device) for _ in range(2))
+    args = (q, *cache, None, SCALE, mode, gs, bits)
+    kw = dict(seqlens_k=lens, k_residual=k[:, S:], v_residual=v[:, S:], residual_len=res, return_lse=True)
+    plan = plan_fwd_kvcache_int(*args, num_splits=ns, _rows=True, **kw)
+    launches = [([0, 128, 256, S, 0, 128, 512, S - 128], [0, 0, 1, 0, 17, 128, 0, 3]),
+                ([S, S, S - 256, 0, 256, 0, 128, 128], [1, 0, 0, 0, 0, 16, 1, 0]),
+                ([128, 0, 0, 384, S, S, 0, 0], [0, 128, 0, 33, 0, 0, 0, 1])]
+    for _ in range(2):
+        for n_s, n_r in launches:
+            lens.copy_(torch.tensor(n_s, dtype=torch.int32))
+            res.copy_(torch.tensor(n_r, dtype=torch.int32))
+            out = plan.run()
+            for r in (0, m - 1):
+                one, lse1 = fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args[1:], num_splits=1, **kw)
+                err = (out[:, r:r + 1].float() - one.float()).abs()
+                assert (err <= 1.5e-3 + (2 ** -7 * one.float().abs() if dtype == "bf16" else 0)).all(), (n_s, r, err.max().item())
+                some = lens + res > 0
+                assert torch.isinf(plan.lse[~some]).all() and not out[~some].any()
+                assert (plan.lse[some, r] - lse1[some]).abs().max().item() < 5e-4
