@@ -30,9 +30,9 @@
 //  * The offset/zero biases and the softmax row sums are themselves computed on the MFMA pipe
 //    (A operand = the zero vector / the constant offsets / ones), which keeps the VALU for the
 //    code unpacking; this kernel is VALU-issue bound long before it is MFMA bound.
-//  * Online softmax in base 2 per head (softmax.h:250-310) in steps of 64 tokens: maxima
+//  * Online softmax in base 2 per head (softmax.h:250-310) in steps of 64 tokens: running max
 //    shared by the four lanes of a head through two lane-half swaps, accumulators rescaled only
-//    when some head's score exceeds its reference, which lies above the largest score so far (kHeadroom).
+//    when some head's max actually moved.
 //  * The waves of a workgroup merge through LDS, one wave per query head; splits merge in the
 //    same launch: that wave publishes the head's record (O / sum in fp16, max, sum) without waiting
 //    for the stores, an idle wave has meanwhile drawn a ticket from the head's counter, and the wave
@@ -91,7 +91,9 @@ __device__ unsigned long long* g_prof = nullptr;
 
 // Probabilities are kept as 2^shift * exp2(s - max) in fp16, and p * (V scale) must stay inside the fp16
 // range as well.  A 4-bit V scale is at most 131008 / 15 = 8734: p up to 4 is safe and keeps two more bits of
-// the small probabilities.  A 2-bit V scale reaches 131008 / 3 = 43669: p stays at 1 or below.
+// the small probabilities.  A 2-bit V scale reaches 131008 / 3 = 43669: p stays at 1 or below.  (Shifts of 2.75 and 0.5 still fit those
+// scales and halve the error of outputs of magnitude 0.01 and less, but bf16 values beyond the fp16 range, which the
+// quantizer takes as long as scale and zero are in range, would overflow earlier: 4 bits from a V scale of 9.7K on, not 16K.)
 constexpr float p_shift(int bits) { return bits == 4 ? 2.0f : 0.0f; }
 constexpr int kLdsRowHalves = 136;
 
@@ -99,8 +101,8 @@ __device__ __forceinline__ h2 pk_rtz(float a, float b) {
     return __builtin_bit_cast(h2, __builtin_amdgcn_cvt_pkrtz(a, b));
 }
 
-// rounded to nearest, one v_cvt_pk_f16_f32 (the bias of a truncation does not quite cancel between a sum of p * v and the sum of p:
-// see kHeadroom for what it makes of the error)
+// rounded to nearest, one v_cvt_pk_f16_f32.  (Scores of deviation 3 nats, 8K tokens, error against 64 bits: 4 bits g128 3.1e-4 of the norm
+// truncated, 2.5e-4 rounded; 2 bits 4.0e-4 and 3.5e-4.)
 __device__ __forceinline__ h2 pk_rne(float a, float b) {
     typedef float f2 __attribute__((ext_vector_type(2)));
     return __builtin_convertvector((f2{a, b}), h2);
@@ -224,8 +226,8 @@ __device__ __forceinline__ float colmax(float x) {
 
 template <int NCG>
 struct WaveState {
-    float m;          // reference of the exponentials (raw scores, q.k units) of this lane's head: no score so far is above it (kNoScore: none yet)
-    // (l and ob: an MFMA makes all four rows alike; only row 0 is kept in step with the reference and read)
+    float m;          // running max of the raw scores (q.k units) of this lane's head (kNoScore: none yet)
+    // (l and ob: an MFMA makes all four rows alike; only row 0 is kept in step with the maximum and read)
     f4 l;             // sum of p, accumulated by MFMA against a ones operand; both columns of a head hold it
     // Zero part of the V bias, one MFMA per 32 tokens for all channel groups: row m of its A operand has the zeros of group
     // m % NCG, so register c is group c's (with one MFMA per group six MFMAs and LDS reads more per 64 tokens at group 32).
@@ -235,29 +237,21 @@ struct WaveState {
     f4 o[8];          // O^T tiles: lane (head, q) holds channels 16*ct + 4*q + r
 };
 
-// The reference of a head without scores: below every sum of 128 products of fp16 values, and finite, so that differences with
-// it need no special case (p of a masked score, -inf, is zero whatever the reference).
+// The maximum of a head without scores: below every sum of 128 products of fp16 values, and finite, so that differences with
+// it need no special case (p of a masked score, -inf, is zero whatever the maximum).
 constexpr float kNoScore = -1e30f;
 
-// When a score exceeds the reference, the new reference is put this far above it (base-2 units), so that the next maxima do
-// not move it again: a move rescales all accumulators, 35 to 41 instructions, and with eight heads some maximum moves in most of a wave's
-// steps.  8 sequences of 64K at 2 bits 63.5 -> 61.4 us, 6 sequences of 10K at 4 bits g32 18.3 -> 17.8.  p stays at 2^pshift or
-// below (its product with the V scale has to stay in range) and is at least 2^(pshift - headroom) for the largest score.  An fp16 p keeps
-// its precision down to 2^-14, so the headroom costs only what lies 11 binades and more below the largest p; rounding p to
-// nearest (pk_rne) gains more: error against 64 bits, 4 bits g128 over 32K 4.9e-4 -> 3.9e-4 of the norm (3.8e-4 without headroom),
-// 2 bits g64 over 4K 4.6e-4 -> 3.9e-4 (3.8e-4).
-constexpr float kHeadroom = 3.0f;
-
 // Online-softmax step over N raw scores t (q.k units); on return t holds
-// p = 2^pshift * exp2(scale * (t - reference)).  Accumulators are rescaled only when the
-// reference of some head moved (wave-uniform branch).  mx: the largest new score of
+// p = 2^pshift * exp2(scale * (t - running max)).  Accumulators are rescaled only when the
+// running max of some head moved (wave-uniform branch).  mx: the largest new score of
 // the lane's head, the same in all its lanes.
-template <int N, int NCG>
-__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st, float mx, float pshift) {
+// (Headroom, a reference some binades above the maximum that moved it, saves most of the rescales, 1-3 % where a wave has many steps, but
+// takes as many bits from the small products p * (V scale): with three binades 4-bit g128 outputs at V of 0.003 and scores of deviation
+// 3 were off by 9.8e-3 of the norm instead of 1.3e-3.)
+template <int BITS, int N, int NCG>
+__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st, float mx) {
     if (__builtin_amdgcn_ballot_w64(mx > st.m) != 0) {
-        // (the headroom in raw score units; worked out here: as a kernel argument it took the short calls 0.1-0.2 us)
-        const float headroom = fminf(kHeadroom * __builtin_amdgcn_rcpf(scale), 1e30f);
-        const float m_new = mx > st.m ? mx + headroom : st.m;
+        const float m_new = fmaxf(st.m, mx);
         if (__builtin_amdgcn_ballot_w64(st.m != kNoScore) != 0) {
             // (not in a wave's first step, which has nothing to rescale: 512 to 8K tokens of one sequence, one unit per wave,
             // 0.12 us of 6.0 to 7.3)
@@ -272,16 +266,16 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
         }
         st.m = m_new;
     }
-    const float c0 = pshift - st.m * scale;
+    const float c0 = p_shift(BITS) - st.m * scale;
 #pragma unroll
     for (int i = 0; i < N; ++i) t[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[i], scale, c0));
 }
-template <int N, int NCG>
-__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st, float pshift) {
+template <int BITS, int N, int NCG>
+__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st) {
     float mx = t[0];
 #pragma unroll
     for (int i = 1; i < N; ++i) mx = fmaxf(mx, t[i]);
-    softmax_step<N, NCG>(t, scale, st, colmax(mx), pshift);
+    softmax_step<BITS, N, NCG>(t, scale, st, colmax(mx));
 }
 
 // Accumulators of the four S^T tiles of a 64-token step -> probabilities as operands of the second
@@ -322,7 +316,7 @@ __device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t h
                    "=&v"(mx), "=&v"(y)
                  : "v"(sc[2][0]), "v"(sc[2][1]), "v"(sc[2][2]), "v"(sc[2][3]), "v"(sc[3][0]), "v"(sc[3][1]),
                    "v"(sc[3][2]), "v"(sc[3][3]));
-    softmax_step<8, NCG>(t, scale, st, mx, p_shift(BITS));
+    softmax_step<BITS, 8, NCG>(t, scale, st, mx);
     u4 z0, m0, z1, m1;      // the hi columns hold sub-block 0, the lo columns sub-block 1
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -346,7 +340,7 @@ __device__ __forceinline__ void step_probabilities_wide(const f4 (&sc)[4], float
     float t[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) t[i] = sc[i / 4][i % 4];
-    softmax_step<16, NCG>(t, scale, st, p_shift(BITS));
+    softmax_step<BITS, 16, NCG>(t, scale, st);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
         u4 w;
@@ -1060,9 +1054,9 @@ __device__ __forceinline__ void load_fp16_tile(Fp16Tile& T, const WindowSrc& W, 
     }
 }
 
-template <bool BF16, int NCG, bool WIDE>
+template <int BITS, bool BF16, int NCG, bool WIDE>
 __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P, int n0, int R, int lane,
-                                          const QRows& Q, bool lo_part, WaveState<NCG>& st, uint16_t* lds, float pshift) {
+                                          const QRows& Q, bool lo_part, WaveState<NCG>& st, uint16_t* lds) {
     const int col = lane & 15, kg = lane >> 4;
 
     // V tile (16 tokens x 128 channels) goes through this wave's LDS slab to be read back
@@ -1090,7 +1084,7 @@ __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P,
             s[r] = tk < R ? tot : -INFINITY;
         }
     }
-    softmax_step<4, NCG>(s, P.scale_log2, st, pshift);
+    softmax_step<BITS, 4, NCG>(s, P.scale_log2, st);
     const h2 p01 = pk_rne(s[0], s[1]), p23 = pk_rne(s[2], s[3]);
     h4 pb = {p01[0], p01[1], p23[0], p23[1]};
     st.l = mfma16(h4{1, 1, 1, 1}, pb, st.l);
@@ -1978,7 +1972,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             while (true) {
                 const int tn = t + stride;
                 const bool more = tn < nT;
-                fp16_tile<BF16, NCG, WIDE>(T, P, t * 16, R, lane_w, Q, lo_part, st, slab, p_shift(BITS));
+                fp16_tile<BITS, BF16, NCG, WIDE>(T, P, t * 16, R, lane_w, Q, lo_part, st, slab);
                 if (!more) break;
                 load_fp16_tile<APPEND>(T, W, tn * 16, R, lane_w, r_new);
                 t = tn;
