@@ -224,7 +224,21 @@ __device__ __forceinline__ float colmax(float x) {
     return x;
 }
 
-template <int NCG>
+// The maximum of a head without scores: below every sum of 128 products of fp16 values, and finite, so that differences with
+// it need no special case (p of a masked score, -inf, is zero whatever the maximum).
+constexpr float kNoScore = -1e30f;
+
+// Blocks of sixteen pairs (WIDE) leave the lo parts of the split products no columns of their own, and run with 8 waves where 2-bit
+// blocks of eight have 16.  Every addition to sums that hold the code offsets rounds at their magnitude, so more of them per sum cost
+// accuracy.  At 4 bits the lo parts have sums of their own; at 2 bits the even and the odd steps of 64 tokens have a state each, as if of
+// two waves (their own maximum too: a wave's largest score decides what its small products keep).  Error against 64 bits of the
+// norm, one split of 8K tokens, blocks of eight | of sixteen with all in one set of sums | as it is: 4 bits g128 1.12e-3 | 1.17e-3 | 9.2e-4; 2 bits g64
+// 1.70e-3 | 2.39e-3 | 1.39e-3, g128 over 16K tokens 2.69e-3 | 4.94e-3 | 2.71e-3, g64 with V of 0.003 and scores of deviation 3 8.0e-4 | 1.07e-3 | 6.8e-4.  It takes 1-4 % (decode of 8 rows, 32 / 8
+// heads, 2 x 8K tokens at 4 bits 12.6 -> 13.0 us).
+constexpr bool lo_sums(int bits, bool wide) { return wide && bits == 4; }
+
+// LO: accumulators of their own for the lo parts where those have no columns of their own (WIDE, 4 bits)
+template <int NCG, bool LO>
 struct WaveState {
     float m;          // running max of the raw scores (q.k units) of this lane's head (kNoScore: none yet)
     // (l and ob: an MFMA makes all four rows alike; only row 0 is kept in step with the maximum and read)
@@ -235,11 +249,52 @@ struct WaveState {
     f4 zb;
     f4 ob[NCG];       // offset part of the V bias per channel group, hi and lo
     f4 o[8];          // O^T tiles: lane (head, q) holds channels 16*ct + 4*q + r
-};
+    f4 ob_lo[LO ? NCG : 1], o_lo[LO ? 8 : 1];
 
-// The maximum of a head without scores: below every sum of 128 products of fp16 values, and finite, so that differences with
-// it need no special case (p of a masked score, -inf, is zero whatever the maximum).
-constexpr float kNoScore = -1e30f;
+    __device__ __forceinline__ WaveState() {
+        m = kNoScore;
+        l = zb = f4{0, 0, 0, 0};
+#pragma unroll
+        for (int c = 0; c < NCG; ++c) ob[c] = f4{0, 0, 0, 0};
+#pragma unroll
+        for (int ct = 0; ct < 8; ++ct) o[ct] = f4{0, 0, 0, 0};
+        if constexpr (LO) {
+#pragma unroll
+            for (int c = 0; c < NCG; ++c) ob_lo[c] = f4{0, 0, 0, 0};
+#pragma unroll
+            for (int ct = 0; ct < 8; ++ct) o_lo[ct] = f4{0, 0, 0, 0};
+        }
+    }
+    // everything accumulated so far times alpha
+    __device__ __forceinline__ void rescale(float alpha) {
+        l[0] *= alpha;
+#pragma unroll
+        for (int c = 0; c < NCG; ++c) zb[c] *= alpha;
+#pragma unroll
+        for (int c = 0; c < NCG; ++c) ob[c][0] *= alpha;
+#pragma unroll
+        for (int ct = 0; ct < 8; ++ct) o[ct] *= alpha;
+        if constexpr (LO) {
+#pragma unroll
+            for (int c = 0; c < NCG; ++c) ob_lo[c][0] *= alpha;
+#pragma unroll
+            for (int ct = 0; ct < 8; ++ct) o_lo[ct] *= alpha;
+        }
+    }
+    // takes in what another state of the wave has accumulated
+    __device__ __forceinline__ void join(WaveState& x, float scale) {
+        const float m_new = fmaxf(m, x.m);
+        rescale(__builtin_amdgcn_exp2f((m - m_new) * scale));
+        x.rescale(__builtin_amdgcn_exp2f((x.m - m_new) * scale));
+        m = m_new;
+        l += x.l;
+        zb += x.zb;
+#pragma unroll
+        for (int c = 0; c < NCG; ++c) ob[c] += x.ob[c];
+#pragma unroll
+        for (int ct = 0; ct < 8; ++ct) o[ct] += x.o[ct];
+    }
+};
 
 // Online-softmax step over N raw scores t (q.k units); on return t holds
 // p = 2^pshift * exp2(scale * (t - running max)).  Accumulators are rescaled only when the
@@ -248,21 +303,14 @@ constexpr float kNoScore = -1e30f;
 // (Headroom, a reference some binades above the maximum that moved it, saves most of the rescales, 1-3 % where a wave has many steps, but
 // takes as many bits from the small products p * (V scale): with three binades 4-bit g128 outputs at V of 0.003 and scores of deviation
 // 3 were off by 9.8e-3 of the norm instead of 1.3e-3.)
-template <int BITS, int N, int NCG>
-__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st, float mx) {
+template <int BITS, int N, int NCG, bool LO>
+__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG, LO>& st, float mx) {
     if (__builtin_amdgcn_ballot_w64(mx > st.m) != 0) {
         const float m_new = fmaxf(st.m, mx);
         if (__builtin_amdgcn_ballot_w64(st.m != kNoScore) != 0) {
             // (not in a wave's first step, which has nothing to rescale: 512 to 8K tokens of one sequence, one unit per wave,
             // 0.12 us of 6.0 to 7.3)
-            const float alpha = __builtin_amdgcn_exp2f((st.m - m_new) * scale);
-            st.l[0] *= alpha;
-#pragma unroll
-            for (int c = 0; c < NCG; ++c) st.zb[c] *= alpha;
-#pragma unroll
-            for (int c = 0; c < NCG; ++c) st.ob[c][0] *= alpha;
-#pragma unroll
-            for (int ct = 0; ct < 8; ++ct) st.o[ct] *= alpha;
+            st.rescale(__builtin_amdgcn_exp2f((st.m - m_new) * scale));
         }
         st.m = m_new;
     }
@@ -270,12 +318,12 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
 #pragma unroll
     for (int i = 0; i < N; ++i) t[i] = __builtin_amdgcn_exp2f(__builtin_fmaf(t[i], scale, c0));
 }
-template <int BITS, int N, int NCG>
-__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG>& st) {
+template <int BITS, int N, int NCG, bool LO>
+__device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveState<NCG, LO>& st) {
     float mx = t[0];
 #pragma unroll
     for (int i = 1; i < N; ++i) mx = fmaxf(mx, t[i]);
-    softmax_step<BITS, N, NCG>(t, scale, st, colmax(mx));
+    softmax_step<BITS, N, NCG, LO>(t, scale, st, colmax(mx));
 }
 
 // Accumulators of the four S^T tiles of a 64-token step -> probabilities as operands of the second
@@ -292,7 +340,7 @@ __device__ __forceinline__ void softmax_step(float (&t)[N], float scale, WaveSta
 // ragged sequences of 1K-8K 18.4 against 18.1 us, 6 paged ones of 10K at group 32 19.4 against 18.9, 8 query rows over 2 x 8K
 // 15.4 against 15.0), equal with one 4-bit unit per wave.
 template <int BITS, int NCG>
-__device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t hi_cols, float scale, WaveState<NCG>& st,
+__device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t hi_cols, float scale, WaveState<NCG, false>& st,
                                                    h8 (&p16)[2], h8 (&pm)[2]) {
     float t[8];
 #pragma unroll
@@ -316,7 +364,7 @@ __device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t h
                    "=&v"(mx), "=&v"(y)
                  : "v"(sc[2][0]), "v"(sc[2][1]), "v"(sc[2][2]), "v"(sc[2][3]), "v"(sc[3][0]), "v"(sc[3][1]),
                    "v"(sc[3][2]), "v"(sc[3][3]));
-    softmax_step<BITS, 8, NCG>(t, scale, st, mx);
+    softmax_step<BITS, 8, NCG, false>(t, scale, st, mx);
     u4 z0, m0, z1, m1;      // the hi columns hold sub-block 0, the lo columns sub-block 1
 #pragma unroll
     for (int x = 0; x < 4; ++x) {
@@ -335,12 +383,12 @@ __device__ __forceinline__ void step_probabilities(const f4 (&sc)[4], uint32_t h
 
 // The same where every column is a pair of its own (sixteen query row and head pairs): the sums are whole scores, and a lane
 // exponentiates all sixteen of its column.
-template <int BITS, int NCG>
-__device__ __forceinline__ void step_probabilities_wide(const f4 (&sc)[4], float scale, WaveState<NCG>& st, h8 (&p16)[2]) {
+template <int BITS, int NCG, bool LO>
+__device__ __forceinline__ void step_probabilities_wide(const f4 (&sc)[4], float scale, WaveState<NCG, LO>& st, h8 (&p16)[2]) {
     float t[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) t[i] = sc[i / 4][i % 4];
-    softmax_step<BITS, 16, NCG>(t, scale, st);
+    softmax_step<BITS, 16, NCG, LO>(t, scale, st);
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
         u4 w;
@@ -764,7 +812,8 @@ template <int BITS, int GS, bool BF16, bool HAS_NEXT, bool KT, bool FEW, bool WI
 __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region_lds, int kslot,
                                              const UnitAddr<BITS, GS>& cur, const UnitAddr<BITS, GS>& next,
                                              const QRows& Q, const FwdParams& P, int lane, bool lo_part, const Magic& mg,
-                                             WaveState<kHeadDim / GS>& st, const TokenQ<kHeadDim / GS>* KQ = nullptr) {
+                                             WaveState<kHeadDim / GS, lo_sums(BITS, WIDE)>& st_even,
+                                             WaveState<kHeadDim / GS, lo_sums(BITS, WIDE)>& st_odd, const TokenQ<kHeadDim / GS>* KQ = nullptr) {
     using C = UnitCfg<BITS, GS>;
     constexpr int NCG = C::NCG, TPS = C::TPS, NKS = C::NKS, TPG = C::TPG, CTPG = GS / 16;
     constexpr int NSTEP = C::NSTEP, RPS = C::RPS, TPR = TPS / RPS;      // tiles per K row
@@ -774,6 +823,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
     const h8 ones = h8{1, 1, 1, 1, 1, 1, 1, 1};
     const uint32_t hi_cols = lo_part ? 0u : 0xffffffffu;
     const u4* kcode = reinterpret_cast<const u4*>(reg) + lane;             // row r: kcode[64 * r]
+    constexpr bool LO = lo_sums(BITS, WIDE);
     const u4* vcode = reinterpret_cast<const u4*>(reg + 4096) + lane;
     const uint8_t* kpar = reg + C::OFF_KP + kslot * C::KPB;
     const uint8_t* vpar = reg + C::OFF_VP + kg * 16;
@@ -791,6 +841,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
     if constexpr (!KT) start_group<BITS, WIDE>(G, kpar, Q, kg);
 #pragma unroll
     for (int step = 0; step < NSTEP; ++step) {
+        auto& st = WIDE && step % 2 ? st_odd : st_even;      // (lo_sums)
         f4 sc[TPS];
 #pragma unroll
         for (int tt = 0; tt < TPS; ++tt) {
@@ -859,7 +910,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
         static_assert(TPS == 4 && NKS == 2, "four tiles, two sub-blocks per step");
         h8 p16[NKS], pm[NKS];
         if constexpr (WIDE) {
-            step_probabilities_wide<BITS, NCG>(sc, P.scale_log2, st, p16);
+            step_probabilities_wide<BITS, NCG, lo_sums(BITS, WIDE)>(sc, P.scale_log2, st, p16);
         } else {
             step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pm);
         }
@@ -899,7 +950,10 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                             st.zb = mfma32(cvt_h8<false>(rz), p16[ks], st.zb);
                         }
                         st.ob[cg] = mfma32(noff, pp[cg][ks], st.ob[cg]);
-                        if constexpr (WIDE) st.ob[cg] = mfma32(noff, pp_lo[cg][ks], st.ob[cg]);
+                        if constexpr (WIDE) {
+                            f4& ob_lo = LO ? st.ob_lo[LO ? cg : 0] : st.ob[cg];
+                            ob_lo = mfma32(noff, pp_lo[cg][ks], ob_lo);
+                        }
                     }
                 }
             }
@@ -915,7 +969,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                 if constexpr (BITS == 4) {
                     const h8 a = dq4(w[x], mg);
                     st.o[ct] = mfma32(a, pp[cg][ksr], st.o[ct]);
-                    if constexpr (WIDE) st.o[ct] = mfma32(a, pp_lo[cg][ksr], st.o[ct]);
+                    if constexpr (WIDE) st.o_lo[ct] = mfma32(a, pp_lo[cg][ksr], st.o_lo[ct]);
                 } else {
                     h8 a0, a1;
                     dq2(w[x], a0, a1, mg);
@@ -1054,9 +1108,9 @@ __device__ __forceinline__ void load_fp16_tile(Fp16Tile& T, const WindowSrc& W, 
     }
 }
 
-template <int BITS, bool BF16, int NCG, bool WIDE>
+template <int BITS, bool BF16, int NCG, bool WIDE, bool LO>
 __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P, int n0, int R, int lane,
-                                          const QRows& Q, bool lo_part, WaveState<NCG>& st, uint16_t* lds) {
+                                          const QRows& Q, bool lo_part, WaveState<NCG, LO>& st, uint16_t* lds) {
     const int col = lane & 15, kg = lane >> 4;
 
     // V tile (16 tokens x 128 channels) goes through this wave's LDS slab to be read back
@@ -1084,7 +1138,7 @@ __device__ __forceinline__ void fp16_tile(const Fp16Tile& T, const FwdParams& P,
             s[r] = tk < R ? tot : -INFINITY;
         }
     }
-    softmax_step<BITS, 4, NCG>(s, P.scale_log2, st);
+    softmax_step<BITS, 4, NCG, LO>(s, P.scale_log2, st);
     const h2 p01 = pk_rne(s[0], s[1]), p23 = pk_rne(s[2], s[3]);
     h4 pb = {p01[0], p01[1], p23[0], p23[1]};
     st.l = mfma16(h4{1, 1, 1, 1}, pb, st.l);
@@ -1924,13 +1978,8 @@ void fwd_splitkv_kernel(FwdParams P) {
     const QRows Q = q_rows(sq, head, kg, lo_part);
     PROF(1);
 
-    WaveState<NCG> st;
-    st.m = kNoScore;
-    st.l = st.zb = f4{0, 0, 0, 0};
-#pragma unroll
-    for (int c = 0; c < NCG; ++c) st.ob[c] = f4{0, 0, 0, 0};
-#pragma unroll
-    for (int ct = 0; ct < 8; ++ct) st.o[ct] = f4{0, 0, 0, 0};
+    constexpr bool kLoSums = lo_sums(BITS, WIDE);
+    WaveState<NCG, kLoSums> st;
 
     // ---- packed units of this wave
     if (u < u1) {
@@ -1945,14 +1994,16 @@ void fwd_splitkv_kernel(FwdParams P) {
             KQ = token_q<BITS, NCG, WIDE>(Q);
             KQp = &KQ;
         }
+        [[maybe_unused]] WaveState<NCG, kLoSums> st_odd;      // (lo_sums)
         int kslot = 0;
         for (int un = u + NW; un < u1; un += NW) {        // units that have a successor: it is fetched from inside
             const UnitAddr<BITS, GS> An = unit_addr<BITS, GS, KT>(P, region_off, bi, hk, un);
-            compute_unit<BITS, GS, BF16, true, KT, FEW, WIDE>(region, region_lds, kslot, A, An, Q, P, lane, lo_part, mg, st, KQp);
+            compute_unit<BITS, GS, BF16, true, KT, FEW, WIDE>(region, region_lds, kslot, A, An, Q, P, lane, lo_part, mg, st, WIDE ? st_odd : st, KQp);
             A = An;
             kslot ^= 1;
         }
-        compute_unit<BITS, GS, BF16, false, KT, FEW, WIDE>(region, region_lds, kslot, A, A, Q, P, lane, lo_part, mg, st, KQp);
+        compute_unit<BITS, GS, BF16, false, KT, FEW, WIDE>(region, region_lds, kslot, A, A, Q, P, lane, lo_part, mg, st, WIDE ? st_odd : st, KQp);
+        if constexpr (WIDE && !kLoSums) st.join(st_odd, P.scale_log2);
     }
     PROF(3);
     // ---- fp16 window tiles of this wave (the region becomes the V-transpose slab)
@@ -1972,7 +2023,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             while (true) {
                 const int tn = t + stride;
                 const bool more = tn < nT;
-                fp16_tile<BITS, BF16, NCG, WIDE>(T, P, t * 16, R, lane_w, Q, lo_part, st, slab);
+                fp16_tile<BITS, BF16, NCG, WIDE, kLoSums>(T, P, t * 16, R, lane_w, Q, lo_part, st, slab);
                 if (!more) break;
                 load_fp16_tile<APPEND>(T, W, tn * 16, R, lane_w, r_new);
                 t = tn;
@@ -2014,7 +2065,8 @@ void fwd_splitkv_kernel(FwdParams P) {
     for (int ct = 0; ct < 8; ++ct) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float v = st.o[ct][r] + bias[ct / (GS / 16)];
+            float v = st.o[ct][r] + bias[ct / (GS / 16)];
+            if constexpr (kLoSums) v += st.o_lo[ct][r] + st.ob_lo[ct / (GS / 16)][0];
             st.o[ct][r] = WIDE ? v : v + partner(v);      // hi + lo
         }
     }

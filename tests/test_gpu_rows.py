@@ -222,3 +222,33 @@ def test_splits_without_work_have_some_in_the_next_launch(device, bits, gs, mode
                 some = lens + res > 0
                 assert torch.isinf(plan.lse[~some]).all() and not out[~some].any()
                 assert (plan.lse[some, r] - lse1[some]).abs().max().item() < 5e-4
+
+
+@pytest.mark.parametrize("bits,gs", [(4, 128), (4, 32), (2, 128), (2, 64)])
+@pytest.mark.parametrize("size,deviation", [(1.0, 1.0), (1.0, 3.0), (0.003, 3.0)])
+def test_blocks_of_sixteen_are_as_accurate_as_calls_for_each_row(device, bits, gs, size, deviation):
+    """Error against 64 bits over one split of 8K tokens, many fp32 additions per sum: no more than calls with one row have, whose
+    hi and lo parts are summed apart by 16 (2 bits) or 8 waves; 10 % for the order of the sums, over 64K outputs.  Where the roundings of
+    the sums make up the error (scores of deviation 1), 2 bits have sqrt(2) of it: sums as many, but the lo parts in them."""
+    from bitladder_amd import _lib, fwd_kvcache_int, kvcache_pack_int
+    from oracle import torch_oracle as T
+    b, h, h_k, m, S = 2, 32, 8, 8, 8192
+    assert _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), S, 256, bits) == 2
+    g = torch.Generator(device=device).manual_seed(bits + gs)
+    q = torch.randn((b, m, h, 128), generator=g, device=device).half()
+    k, v = (torch.randn((b, S, h_k, 128), generator=g, device=device) for _ in range(2))
+    k, v = k.half(), (v * size).half()
+    cache = H.alloc_cache(b, S, h_k, bits, gs, device)
+    kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, S, "k-channel", gs, bits)
+    z = T.quantize_kv(k.float(), v.float(), bits, gs, torch.float16)
+    kh = (z.k_codes.double().reshape(b, S // gs, gs, h_k, 128) * z.k_scale.double()[:, :, None] + z.k_zero.double()[:, :, None])
+    vh = (z.v_codes.double().reshape(b, S, h_k, 128 // gs, gs) * z.v_scale.double()[..., None] + z.v_zero.double()[..., None])
+    kh, vh = (t.reshape(b, S, h_k, 128).transpose(1, 2).contiguous() for t in (kh, vh))
+    scale = deviation * SCALE
+    qq = q.double().reshape(b, m, h_k, h // h_k, 128).permute(0, 2, 1, 3, 4).reshape(b, h_k, -1, 128)
+    ref = torch.softmax(qq @ kh.transpose(2, 3).contiguous() * scale, -1) @ vh
+    ref = ref.reshape(b, h_k, m, h // h_k, 128).transpose(1, 2).reshape(b, m, h, 128)
+    args = (*cache, None, scale, "k-channel", gs, bits)
+    ones = torch.cat([fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args, num_splits=1) for r in range(m)], 1)
+    err, one = ((t.double() - ref).norm().item() for t in (fwd_kvcache_int(q, *args, num_splits=1), ones))
+    assert err < 1.1 * (math.sqrt(2) if bits == 2 and deviation == 1.0 else 1.0) * one, (err / ref.norm().item(), one / ref.norm().item())
