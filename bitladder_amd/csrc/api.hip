@@ -555,7 +555,9 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
         P.out_sr = rows_args->out_stride_row;
     }
     // (decode.hip: kPartialLoFrom)
-    if (nsplit > 1 && static_cast<int64_t>(a->b) * a->h_k * row_blocks > cus) P.h |= INT32_MIN;
+    // (several query rows: counted in blocks of eight also where they run in blocks of sixteen, whose split counts are no reason to round more)
+    const int64_t blocks8 = rows > 1 ? row_blocks_of(rows * g, false) : 1;
+    if (nsplit > 1 && blocks8 * a->b * a->h_k > cus) P.h |= INT32_MIN;
     P.scale = a->softmax_scale;
     P.scale_log2 = fabsf(a->softmax_scale) * 1.4426950408889634f;   // decode_api.cpp:128-142
     P.neg_scale = a->softmax_scale < 0.0f;

@@ -89,3 +89,21 @@ def test_residual_words_in_the_step_and_with_several_rows(device):
         many, one = (c.step(q, *new, SCALE, num_splits=ns) for c, ns in zip(caches, (5, 1)))
         assert (many.float() - one.float()).abs().max() < 2e-3
         assert torch.equal(caches[0].k_res, caches[1].k_res) and torch.equal(caches[0].total, caches[1].total)
+
+
+@pytest.mark.parametrize("b,S,gs", [(18, 4096, 128), (17, 8192, 64)])
+def test_several_rows_lose_no_precision_to_the_split(device, b, S, gs):
+    """Sixteen (row, head) pairs of each of 144 or 136 (sequence, kv head) pairs: more blocks of eight than compute units, fewer of
+    sixteen.  The error of the library's own split count is that of one split or less, as with one row."""
+    from bitladder_amd import _lib, fwd_kvcache_int
+    q, k, v, cache = _setup(device, b, 8, S, 64, gs, b)
+    assert _lib.lib().bitdecode_row_blocks(b, 8, 16, S, 256, 4) == 1
+    rows = torch.cat([q.roll(j, 0) for j in range(8)], 1)
+    seqs = (0, b // 2, b - 1)
+    ref = torch.stack([torch.stack([_exact(rows[:, j:j + 1], k, v, S, gs, i) for j in range(8)]) for i in seqs])
+    err = []
+    for ns in (1, 0, 2, 3):
+        out = fwd_kvcache_int(rows, *cache, None, SCALE, "k-channel", gs, 4, k_residual=k[:, S:].contiguous(),
+                              v_residual=v[:, S:].contiguous(), num_splits=ns)[list(seqs)].double()
+        err.append(float((out - ref).norm() / ref.norm()))
+    assert max(err) == err[0], err
