@@ -10,7 +10,7 @@ import os
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libbitdecode.so")
 
-ABI_VERSION = 7
+ABI_VERSION = 8
 FP16, BF16 = 0, 1
 K_CHANNEL, K_TENSOR = 0, 1
 
@@ -98,7 +98,7 @@ class CacheArgs(ctypes.Structure):
 EXPORTS = ("bitdecode_abi_version", "bitdecode_last_error", "bitdecode_num_splits",
            "bitdecode_fwd_workspace_bytes", "bitdecode_num_splits_for", "bitdecode_qpack", "bitdecode_fwd",
            "bitdecode_fwd_append", "bitdecode_fwd_append_workspace_bytes", "bitdecode_fwd_static",
-           "bitdecode_fwd_rows", "bitdecode_row_blocks", "bitdecode_cache_prefill", "bitdecode_cache_append")
+           "bitdecode_fwd_rows", "bitdecode_row_blocks", "bitdecode_rows_splits", "bitdecode_cache_prefill", "bitdecode_cache_append")
 
 _lib = None
 
@@ -130,6 +130,8 @@ def lib():
         L.bitdecode_num_splits.argtypes = [_i32] * 7
         L.bitdecode_row_blocks.restype = ctypes.c_int
         L.bitdecode_row_blocks.argtypes = [_i32] * 6
+        L.bitdecode_rows_splits.restype = ctypes.c_int
+        L.bitdecode_rows_splits.argtypes = [_i32] * 11 + [ctypes.POINTER(_i32)]
         L.bitdecode_num_splits_for.restype = ctypes.c_int
         L.bitdecode_num_splits_for.argtypes = [_i32] * 8
         L.bitdecode_fwd_workspace_bytes.restype = ctypes.c_size_t

@@ -143,30 +143,6 @@ int choose_splits(int b, int hk, int max_seqlen_k, int max_res_len, int num_cus,
     return std::max(1, n);
 }
 
-// Several query rows per sequence: blocks of sixteen (query row, query head) pairs instead of eight?  A workgroup then unpacks the
-// codes for twice as many pairs, at half the vector instructions per pair, but a wave takes longer over a unit and over the merge.
-// So it pays with work: W = units of 64 tokens times blocks of eight pairs per compute unit.  us in blocks of eight | sixteen,
-// 32 / 8 heads unless said, 4 bits g128, 4 bits g32, 2 bits g128:
-//   1 x 4K, 8 rows            W  8:   8.6 |  9.9    9.4 | 10.5    9.2 | 10.3
-//   1 x 8K, 8 rows            W 16:  10.9 | 11.3   12.7 | 12.0   10.1 | 11.6       16 x 1K, 4 rows  W 16:  10.1 | 10.1   11.5 | 10.8   9.0 | 9.4
-//   1 x 12K, 8 rows           W 24:  12.9 | 11.9   14.8 | 12.8   11.9 | 12.2       3 x 4K, 8 rows   W 24:  14.7 | 12.3   17.2 | 13.7  13.1 | 10.9
-//   4 x 2K, 64 / 8, 8 rows    W 32:  16.9 | 12.4   20.1 | 13.9   13.4 | 11.5       32 x 2K, 8 / 8, 16 rows  W 64:  29.1 | 18.0   37.7 | 21.6  25.7 | 15.2
-// Where so few (sequence, kv head, block) triples are left that filling the machine takes more than 32 splits, the second round trip of
-// their merge outweighs it at 2 bits, and at 4 bits until W is larger:
-//   1 x 64K, 8 / 1, 8 rows    W 32:  17.7 | 18.6   21.0 | 19.9   16.7 | 17.9       1 x 128K, 8 / 1  W 64:  31.2 | 24.0   37.0 | 27.1  22.8 | 21.1 (g64 23.7 | 24.9)
-bool rows_wide(int b, int hk, int pairs, int max_s, int cus, int bits) {
-    if (pairs <= bitdecode::kMaxGroupHeads) return false;
-    const int64_t blocks8 = (pairs + bitdecode::kMaxGroupHeads - 1) / bitdecode::kMaxGroupHeads, blocks16 = (blocks8 + 1) / 2;
-    const bool many_splits = static_cast<int64_t>(b) * hk * blocks16 * 32 < cus;
-    if (many_splits && bits == 2) return false;
-    const int from = many_splits ? 48 : bits == 4 ? 20 : 28;
-    return static_cast<int64_t>(b) * hk * blocks8 * (max_s / 64) >= static_cast<int64_t>(from) * cus;
-}
-int row_blocks_of(int pairs, bool wide) {
-    const int block = wide ? bitdecode::kWidePairs : bitdecode::kMaxGroupHeads;
-    return (pairs + block - 1) / block;
-}
-
 // The 4-bit kernels also exist with 8 waves per workgroup (decode.hip: launch_fwd_tt), used whenever the packed
 // prefix is the bulk of the work.  With per-sequence lengths on the device the workgroups of the longest
 // sequences can be left streaming alone at the end, where 16 waves keep more bytes in flight per compute
@@ -222,6 +198,79 @@ int choose_splits_for(int b, int hk, int max_s, int max_r, int num_cus, int bits
     return n1;
 }
 
+// Several query rows per sequence, in blocks of eight or sixteen (query row, query head) pairs.  A workgroup of sixteen unpacks the
+// codes for twice as many pairs, at half the vector instructions per pair, but a wave takes longer over a unit and over the merge, and
+// a compute unit holds one such workgroup.
+struct RowsCall {
+    int b, hk, pairs, max_s, max_r, cus, bits, gs;
+    bool ragged;        // per-sequence lengths on the device
+    bool open;          // ... and no bound of theirs but the cache's capacity
+    int64_t blocks8() const { return (static_cast<int64_t>(pairs) + bitdecode::kMaxGroupHeads - 1) / bitdecode::kMaxGroupHeads; }
+    int64_t blocks16() const { return (blocks8() + 1) / 2; }
+    int64_t triples() const { return static_cast<int64_t>(b) * hk * blocks16(); }      // (sequence, kv head, block of sixteen)
+};
+
+// So sixteen pays with work: W = units of 64 tokens times blocks of eight pairs per compute unit.  us in blocks of eight | sixteen,
+// 32 / 8 heads unless said, 4 bits g128, 4 bits g32, 2 bits g128:
+//   1 x 4K, 8 rows            W  8:   8.6 |  9.9    9.4 | 10.5    9.2 | 10.3
+//   1 x 8K, 8 rows            W 16:  10.9 | 11.3   12.7 | 12.0   10.1 | 11.6       16 x 1K, 4 rows  W 16:  10.1 | 10.1   11.5 | 10.8   9.0 | 9.4
+//   1 x 12K, 8 rows           W 24:  12.9 | 11.9   14.8 | 12.8   11.9 | 12.2       3 x 4K, 8 rows   W 24:  14.7 | 12.3   17.2 | 13.7  13.1 | 10.9
+//   4 x 2K, 64 / 8, 8 rows    W 32:  16.9 | 12.4   20.1 | 13.9   13.4 | 11.5       32 x 2K, 8 / 8, 16 rows  W 64:  29.1 | 18.0   37.7 | 21.6  25.7 | 15.2
+// Where so few triples are left that filling the machine takes 32 splits and more, their merge outweighs it at 2 bits, and at 4 bits until
+// W is larger:
+//   1 x 64K, 8 / 1, 8 rows    W 32:  17.7 | 18.6   21.0 | 19.9   16.7 | 17.9       1 x 128K, 8 / 1  W 64:  31.2 | 24.0   37.0 | 27.1  22.8 | 21.1 (g64 23.7 | 24.9)
+//   2 x 25K, 12 / 4, 4 rows   W 25:  13.3 | 14.3 (31 splits)                          1 x 33K, 16 / 8, 8 rows  W 32, 2 bits: 14.3 | 14.9 (29)
+bool rows_work(const RowsCall& c) {
+    if (c.pairs <= bitdecode::kMaxGroupHeads) return false;
+    const bool many_splits = c.triples() * 32 <= c.cus;
+    if (many_splits && c.bits == 2) return false;
+    int from = many_splits ? 48 : c.bits == 4 ? 20 : 28;
+    // (lengths of an eighth to a quarter of the capacity, the only bound: W by the bound 60 9.4 | 11.8, 66 9.6 | 10.9, 83 12.5 | 11.7 and 15.8 | 19.9, 98
+    // 20.0 | 11.6, 115 17.1 | 11.4, 139 17.9 | 11.0)
+    if (c.open) from = std::max(from, 96);
+    return c.blocks8() * c.b * c.hk * (c.max_s / 64) >= static_cast<int64_t>(from) * c.cus;
+}
+
+// Whether a call of n splits runs in blocks of sixteen.  us in blocks of eight | sixteen over 1300 drawn calls, every bit width, group size, mode and element type among them:
+//  * Up to half the units' number of workgroups of sixteen, blocks of eight fit the machine side by side and take less time each, at
+//    every length (one split of 46K tokens, 21 triples, 2 bits: 128 | 174; 48 triples of 16K, 2 splits, 4 bits: 39.9 | 46.1; 128 triples 13.4 | 15.2), from
+//    160 on they do not (160: 29.3 | 18.0, 174: 43.3 | 27.7, 168: 28.9 | 18.7).  The library's own counts are above that.
+//  * A workgroup wants a unit of 64 tokens for each of its eight waves (5.5: 123 | 140).
+//  * Three or five blocks of eight make two or three of sixteen, a quarter or a sixth of whose columns is idle: only where the workgroups
+//    fill the machine (144 of 256 units: 15.5 | 18.1, 39.1 | 45.9; 176: 31.2 | 33.9; 1056 of 1280: 48.8 | 56.9; 240: 14.9 | 13.5, 53.8 | 35.6), and three blocks only
+//    with few splits to merge (4 bits, 21 splits: 13.9 | 16.5, 16: 31.9 | 28.3; 2 bits, 16: 20.4 | 21.1, 10: 15.4 | 17.3, 8: 23.7 | 21.3).
+//  * The 16-wave 4-bit kernel of blocks of eight (long sequences of unequal length, long windows) sums half as many tokens per wave: only
+//    where there are twice as many splits, so that no sum is longer than it would be.
+bool rows_wide(const RowsCall& c, int n) {
+    if (!rows_work(c)) return false;
+    const int64_t wgs = c.triples() * n;
+    if (2 * wgs <= c.cus || c.max_s / 64 < 8 * n) return false;
+    const int64_t slots = (wgs + c.cus - 1) / c.cus * c.cus;
+    if (c.blocks8() == 3 && (8 * wgs < 7 * slots || n > (c.bits == 4 ? 16 : 8))) return false;
+    if (c.blocks8() == 5 && 5 * wgs < 4 * slots) return false;
+    if (bitdecode::few_waves_variant(c.bits, c.gs) && !use_few_waves(c.bits, c.gs, c.max_s, c.max_r, n, c.ragged))
+        return n >= 2 * choose_splits_for(c.b, static_cast<int>(c.hk * c.blocks8()), c.max_s, c.max_r, c.cus, c.bits, c.gs, c.ragged);
+    return true;
+}
+
+struct RowsPlan { int splits; bool wide; };
+// Split count (num_splits, or the library's own if that is zero) and blocks of a call; no split count of its own whose workspace is
+// larger than `fits` says, if a smaller one can do.
+template <class Fits>
+RowsPlan plan_rows(const RowsCall& c, int num_splits, const Fits& fits) {
+    if (num_splits > 0) return {num_splits, rows_wide(c, num_splits)};
+    // (as for equal lengths: choose_splits_for's doubling counts on two workgroups per unit; 16 sequences of up to 2560 tokens in doubled and
+    // plain counts, blocks of eight: 17.6 and 12.6, 14.1; up to 896: 20.5 and 10.7, 12.7)
+    const int n16 = choose_splits(c.b, static_cast<int>(c.hk * c.blocks16()), c.max_s, c.max_r, c.cus, c.bits, c.gs);
+    if (rows_wide(c, n16) && fits(n16)) return {n16, true};
+    int n = choose_splits_for(c.b, static_cast<int>(c.hk * c.blocks8()), c.max_s, c.max_r, c.cus, c.bits, c.gs, c.ragged);
+    // a workspace sized by bitdecode_num_splits_for and bitdecode_row_blocks is taken
+    const int least = std::min(n, rows_work(c) ? choose_splits_for(c.b, static_cast<int>(c.hk * c.blocks16()), c.max_s, c.max_r, c.cus, c.bits, c.gs, c.ragged) : n);
+    while (n > least && !fits(n)) --n;
+    return {n, false};
+}
+int row_blocks_of(const RowsCall& c, bool wide) { return static_cast<int>(wide ? c.blocks16() : c.blocks8()); }
+
 }  // namespace
 
 extern "C" {
@@ -246,7 +295,22 @@ int bitdecode_num_splits_for(int32_t b, int32_t h_k, int32_t max_seqlen_k, int32
 
 int bitdecode_row_blocks(int32_t b, int32_t h_k, int32_t pairs, int32_t max_seqlen_k, int32_t num_cus, int32_t bits) {
     if (num_cus <= 0) num_cus = query_cus();
-    return row_blocks_of(std::max(1, pairs), rows_wide(b, h_k, pairs, max_seqlen_k, num_cus, bits));
+    if (check_quant(bits, 128, BITDECODE_FP16, bitdecode::kHeadDim)) return -1;
+    if (b <= 0 || h_k <= 0 || pairs <= 0) return fail(BITDECODE_EINVAL, "batch, head and pair counts must be positive"), -1;
+    const RowsCall c{b, h_k, pairs, max_seqlen_k, 0, num_cus, bits, 128, false, false};
+    return row_blocks_of(c, rows_work(c));
+}
+
+int bitdecode_rows_splits(int32_t b, int32_t h_k, int32_t pairs, int32_t max_seqlen_k, int32_t max_res_len, int32_t num_cus, int32_t bits,
+                          int32_t group_size, int32_t per_sequence_lengths, int32_t capacity, int32_t num_splits, int32_t* row_blocks) {
+    if (num_cus <= 0) num_cus = query_cus();
+    if (check_quant(bits, group_size, BITDECODE_FP16, bitdecode::kHeadDim)) return -1;
+    if (b <= 0 || h_k <= 0 || pairs <= 0 || num_splits < 0) return fail(BITDECODE_EINVAL, "batch, head, pair and split counts must be positive"), -1;
+    const RowsCall c{b, h_k, pairs, max_seqlen_k, max_res_len, num_cus, bits, group_size, per_sequence_lengths != 0,
+                     per_sequence_lengths != 0 && max_seqlen_k >= capacity};
+    const RowsPlan p = plan_rows(c, num_splits, [](int) { return true; });
+    if (row_blocks) *row_blocks = row_blocks_of(c, p.wide);
+    return p.splits;
 }
 
 // [tickets: one 256-byte block per (batch, query head)][o_part][ml_part]
@@ -455,8 +519,6 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     }
     if (max_s < 0 || max_r < 0) return fail(BITDECODE_EINVAL, "negative length");
     const int cus = query_cus();
-    const bool wide = rows > 1 && rows_wide(a->b, a->h_k, rows * g, max_s, cus, a->bits);
-    const int row_blocks = rows > 1 ? row_blocks_of(rows * g, wide) : 1;
     if (max_s % kChunk) return fail(BITDECODE_EINVAL, "packed length %d is not a multiple of 128", max_s);
     if (!a->block_table && max_s > a->cache_tokens)
         return fail(BITDECODE_EINVAL, "packed length %d exceeds cache capacity %d", max_s, a->cache_tokens);
@@ -483,17 +545,23 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     int nsplit = a->num_splits;
     if (nsplit < 0) return fail(BITDECODE_EINVAL, "num_splits %d is negative", nsplit);
     if (nsplit > 512) return fail(BITDECODE_EINVAL, "num_splits %d is above the limit of 512", nsplit);
-    if (nsplit == 0)
-        nsplit = choose_splits_for(a->b, a->h_k * row_blocks, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k && !step);
+    bool wide = false;
+    int row_blocks = 1, blocks8 = 1;
+    if (rows > 1) {
+        const int64_t cap = a->block_table ? static_cast<int64_t>(a->max_pages_per_seq) * a->cache_tokens : a->cache_tokens;
+        const RowsCall c{a->b, a->h_k, rows * g, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k != nullptr, a->seqlens_k && max_s >= cap};
+        const RowsPlan plan = plan_rows(c, nsplit, [&](int n) {
+            return n <= 1 || (a->workspace && bitdecode_fwd_workspace_bytes(a->b, n_h, n) <= a->workspace_bytes); });
+        nsplit = plan.splits;
+        wide = plan.wide;
+        row_blocks = row_blocks_of(c, wide);
+        blocks8 = row_blocks_of(c, false);
+    } else if (nsplit == 0) {
+        nsplit = choose_splits_for(a->b, a->h_k, max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k && !step);
+    }
     // (the built-in scratch takes every call that leaves the count to the library: it chooses no more than fits)
     while (static_scratch && a->num_splits == 0 && nsplit > 1 && slots_bytes(a->b, n_h, nsplit) > kStaticScratchBytes - kStaticCounterBytes)
         --nsplit;
-    // (several query rows in blocks of sixteen, count left to the library: a workspace that holds the count of blocks of eight, which
-    // a caller may have asked for, is taken, with no more splits than it holds)
-    if (wide && a->num_splits == 0) {
-        const int least = choose_splits_for(a->b, a->h_k * row_blocks_of(rows * g, false), max_s, max_r, cus, a->bits, a->group_size, a->seqlens_k != nullptr);
-        while (nsplit > least && bitdecode_fwd_workspace_bytes(a->b, n_h, nsplit) > (a->workspace ? a->workspace_bytes : 0)) --nsplit;
-    }
     if (nsplit > 1 && slots_bytes(a->b, n_h, nsplit) >= (size_t(1) << 31))
         return fail(BITDECODE_EUNSUPPORTED, "%d splits x %d x %d heads: partial outputs of 2 GiB or more", nsplit, a->b, n_h);
     // the kernel divides workgroup ids and unit counts by the split count and the head count with a
@@ -556,8 +624,7 @@ static int run_fwd(const bitdecode_fwd_args* a, const bitdecode_fwd_append_args*
     }
     // (decode.hip: kPartialLoFrom)
     // (several query rows: counted in blocks of eight also where they run in blocks of sixteen, whose split counts are no reason to round more)
-    const int64_t blocks8 = rows > 1 ? row_blocks_of(rows * g, false) : 1;
-    if (nsplit > 1 && blocks8 * a->b * a->h_k > cus) P.h |= INT32_MIN;
+    if (nsplit > 1 && static_cast<int64_t>(a->b) * a->h_k * blocks8 > cus) P.h |= INT32_MIN;
     P.scale = a->softmax_scale;
     P.scale_log2 = fabsf(a->softmax_scale) * 1.4426950408889634f;   // decode_api.cpp:128-142
     P.neg_scale = a->softmax_scale < 0.0f;

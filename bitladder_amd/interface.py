@@ -467,10 +467,12 @@ def plan_fwd_kvcache_int(q: torch.Tensor,
     a.quant_mode = mode
     a.softmax_scale = float(softmax_scale)
     with _on_device(device):
-        # (several query rows: a workgroup per block of row and head pairs of a kv head, workspace rows by pairs)
-        blocks = 1 if m == 1 else _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), a.max_seqlen_k, 0, num_bits)
-        ns, nbytes = _split_plan(device.index, b, h * m, h_k * blocks, a.max_seqlen_k, a.max_res_len,
-                                 seqlens_k is not None, num_bits, group_size, int(num_splits))
+        num_splits = int(num_splits)
+        if m > 1 and num_splits == 0:      # (workgroups by blocks of row and head pairs of a kv head, workspace rows by pairs)
+            num_splits = _lib.lib().bitdecode_rows_splits(b, h_k, m * (h // h_k), a.max_seqlen_k, a.max_res_len, 0, num_bits, group_size,
+                                                          seqlens_k is not None, capacity, 0, None)
+        ns, nbytes = _split_plan(device.index, b, h * m, h_k, a.max_seqlen_k, a.max_res_len,
+                                 seqlens_k is not None, num_bits, group_size, num_splits)
         a.num_splits = ns
         if nbytes:
             # zero-filled: the arrival counters at its head must be 0 before the first call

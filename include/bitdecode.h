@@ -19,7 +19,7 @@
 extern "C" {
 #endif
 
-#define BITDECODE_ABI_VERSION 7
+#define BITDECODE_ABI_VERSION 8
 
 enum {
     BITDECODE_OK = 0,
@@ -140,9 +140,10 @@ int bitdecode_fwd_static(const bitdecode_fwd_args* args, void* stream);
  * 358-368; its interface fixes is_causal = False, so every row attends every key).  In `fwd`: q and out are
  * [b, rows, h, 128], softmax_lse is [b, rows, h]; the workspace is sized, and zeroed for another shape, as for
  * rows * h heads: bitdecode_fwd_workspace_bytes(b, rows * h, num_splits).  The rows * (h / h_k) row and head pairs
- * of a kv head run in blocks of eight or sixteen, one workgroup each: bitdecode_num_splits(_for) wants
- * h_k * bitdecode_row_blocks(b, h_k, pairs, max_seqlen_k, num_cus (0: the current device's), bits).  With
- * num_splits = 0 a workspace sized for blocks of eight (h_k * ceil(pairs / 8)) is taken as well. */
+ * of a kv head run in blocks of eight or sixteen, one workgroup each.  bitdecode_rows_splits returns the split count that
+ * num_splits = 0 stands for.  With num_splits = 0 a workspace for fewer splits is taken as well, if it holds what
+ * bitdecode_num_splits_for chooses for h_k * ceil(pairs / 8), or for h_k * bitdecode_row_blocks(b, h_k, pairs, max_seqlen_k,
+ * num_cus, bits); the call then runs in blocks of eight. */
 typedef struct bitdecode_fwd_rows_args {
     bitdecode_fwd_args fwd;
     int32_t rows;              /* query rows per sequence, 1 to 4096                        */
@@ -151,6 +152,14 @@ typedef struct bitdecode_fwd_rows_args {
 } bitdecode_fwd_rows_args;
 
 int bitdecode_fwd_rows(const bitdecode_fwd_rows_args* args, void* stream);
+/* Split count of such a call, and through row_blocks (if not NULL) its number of blocks per kv head: the library's own count for
+ * num_splits = 0, otherwise num_splits.  pairs = rows * (h / h_k); per_sequence_lengths: seqlens_k is given; capacity: tokens a
+ * sequence can hold (cache_tokens, paged max_pages_per_seq * cache_tokens); num_cus = 0: the current device's.  -1 if
+ * the arguments are invalid. */
+int bitdecode_rows_splits(int32_t b, int32_t h_k, int32_t pairs, int32_t max_seqlen_k, int32_t max_res_len, int32_t num_cus,
+                          int32_t bits, int32_t group_size, int32_t per_sequence_lengths, int32_t capacity, int32_t num_splits,
+                          int32_t* row_blocks);
+/* Blocks per kv head by the amount of work alone (blocks of sixteen where there is enough of it); -1 if the arguments are invalid. */
 int bitdecode_row_blocks(int32_t b, int32_t h_k, int32_t pairs, int32_t max_seqlen_k, int32_t num_cus, int32_t bits);
 
 /* One decode step in one launch: attend the new token together with everything held, append it, and

@@ -12,6 +12,16 @@ pytestmark = pytest.mark.gpu
 SCALE = 1.0 / math.sqrt(128)
 
 
+def _blocks(b, h_k, pairs, max_s, max_r, bits, gs, ragged, capacity, ns):
+    """Blocks of row and head pairs per kv head that a call runs in."""
+    import ctypes
+
+    from bitladder_amd import _lib
+    n = ctypes.c_int32()
+    _lib.lib().bitdecode_rows_splits(b, h_k, pairs, max_s, max_r, 256, bits, gs, ragged, capacity, ns, ctypes.byref(n))
+    return n.value
+
+
 @pytest.mark.parametrize("h,h_k,m,bits,gs,mode,dtype,ns,paged", [
     (6, 2, 5, 4, 128, "k-channel", "fp16", 3, False),      # 15 pairs: a row is cut by the block boundary, last block of 7
     (3, 3, 9, 2, 64, "k-channel", "fp16", 2, False),       # 9 pairs: last block of 1
@@ -194,18 +204,18 @@ def test_count_left_to_the_library_fits_a_workspace_sized_for_blocks_of_eight(de
 def test_splits_without_work_have_some_in_the_next_launch(device, bits, gs, mode, dtype, ns):
     """One workspace, lengths and windows that change from launch to launch: splits of a short or empty sequence have neither a unit nor a
     tile, the same splits have both one launch later.  Bounds as for `test_blocks_of_sixteen_equal_the_calls_for_each_row`."""
-    from bitladder_amd import _lib, fwd_kvcache_int, kvcache_pack_int
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
     from bitladder_amd.interface import plan_fwd_kvcache_int
-    b, h, h_k, m, S, R, tdt = 8, 16, 2, 5, 128 * 64, 128, H.torch_dtype(dtype)
-    assert _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), S, 256, bits) == 3      # blocks of sixteen
+    b, h, h_k, m, S, R, tdt = 8, 16, 2, 6, 128 * 130, 128, H.torch_dtype(dtype)
+    assert _blocks(b, h_k, m * (h // h_k), S, R, bits, gs, True, S + 128, ns) == 3      # of sixteen
     g = torch.Generator(device=device).manual_seed(ns)
     k, v = (torch.randn((b, S + R, h_k, 128), generator=g, device=device).to(tdt) for _ in range(2))
     q = torch.randn((b, m, h, 128), generator=g, device=device).to(tdt)
-    cache = H.alloc_cache(b, S, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
+    cache = H.alloc_cache(b, S + 128, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
     kvcache_pack_int(k[:, :S], cache[0], cache[1], v[:, :S], cache[2], cache[3], None, None, S, mode, gs, bits)
     lens, res = (torch.zeros(b, dtype=torch.int32, device=device) for _ in range(2))
     args = (q, *cache, None, SCALE, mode, gs, bits)
-    kw = dict(seqlens_k=lens, k_residual=k[:, S:], v_residual=v[:, S:], residual_len=res, return_lse=True)
+    kw = dict(seqlens_k=lens, max_seqlen_k=S, k_residual=k[:, S:], v_residual=v[:, S:], residual_len=res, return_lse=True)
     plan = plan_fwd_kvcache_int(*args, num_splits=ns, _rows=True, **kw)
     launches = [([0, 128, 256, S, 0, 128, 512, S - 128], [0, 0, 1, 0, 17, 128, 0, 3]),
                 ([S, S, S - 256, 0, 256, 0, 128, 128], [1, 0, 0, 0, 0, 16, 1, 0]),
@@ -230,25 +240,63 @@ def test_blocks_of_sixteen_are_as_accurate_as_calls_for_each_row(device, bits, g
     """Error against 64 bits over one split of 8K tokens, many fp32 additions per sum: no more than calls with one row have, whose
     hi and lo parts are summed apart by 16 (2 bits) or 8 waves; 10 % for the order of the sums, over 64K outputs.  Where the roundings of
     the sums make up the error (scores of deviation 1), 2 bits have sqrt(2) of it: sums as many, but the lo parts in them."""
-    from bitladder_amd import _lib, fwd_kvcache_int, kvcache_pack_int
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
     from oracle import torch_oracle as T
-    b, h, h_k, m, S = 2, 32, 8, 8, 8192
-    assert _lib.lib().bitdecode_row_blocks(b, h_k, m * (h // h_k), S, 256, bits) == 2
+    b, h, h_k, m, S, n = 10, 32, 8, 8, 8192, 2
+    assert _blocks(b, h_k, m * (h // h_k), S, 0, bits, gs, False, S, 1) == 2      # of sixteen
     g = torch.Generator(device=device).manual_seed(bits + gs)
     q = torch.randn((b, m, h, 128), generator=g, device=device).half()
     k, v = (torch.randn((b, S, h_k, 128), generator=g, device=device) for _ in range(2))
     k, v = k.half(), (v * size).half()
     cache = H.alloc_cache(b, S, h_k, bits, gs, device)
     kvcache_pack_int(k, cache[0], cache[1], v, cache[2], cache[3], None, None, S, "k-channel", gs, bits)
-    z = T.quantize_kv(k.float(), v.float(), bits, gs, torch.float16)
-    kh = (z.k_codes.double().reshape(b, S // gs, gs, h_k, 128) * z.k_scale.double()[:, :, None] + z.k_zero.double()[:, :, None])
-    vh = (z.v_codes.double().reshape(b, S, h_k, 128 // gs, gs) * z.v_scale.double()[..., None] + z.v_zero.double()[..., None])
-    kh, vh = (t.reshape(b, S, h_k, 128).transpose(1, 2).contiguous() for t in (kh, vh))
+    z = T.quantize_kv(k[:n].float(), v[:n].float(), bits, gs, torch.float16)      # (of the first n sequences)
+    kh = (z.k_codes.double().reshape(n, S // gs, gs, h_k, 128) * z.k_scale.double()[:, :, None] + z.k_zero.double()[:, :, None])
+    vh = (z.v_codes.double().reshape(n, S, h_k, 128 // gs, gs) * z.v_scale.double()[..., None] + z.v_zero.double()[..., None])
+    kh, vh = (t.reshape(n, S, h_k, 128).transpose(1, 2).contiguous() for t in (kh, vh))
     scale = deviation * SCALE
-    qq = q.double().reshape(b, m, h_k, h // h_k, 128).permute(0, 2, 1, 3, 4).reshape(b, h_k, -1, 128)
+    qq = q[:n].double().reshape(n, m, h_k, h // h_k, 128).permute(0, 2, 1, 3, 4).reshape(n, h_k, -1, 128)
     ref = torch.softmax(qq @ kh.transpose(2, 3).contiguous() * scale, -1) @ vh
-    ref = ref.reshape(b, h_k, m, h // h_k, 128).transpose(1, 2).reshape(b, m, h, 128)
+    ref = ref.reshape(n, h_k, m, h // h_k, 128).transpose(1, 2).reshape(n, m, h, 128)
     args = (*cache, None, scale, "k-channel", gs, bits)
     ones = torch.cat([fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args, num_splits=1) for r in range(m)], 1)
-    err, one = ((t.double() - ref).norm().item() for t in (fwd_kvcache_int(q, *args, num_splits=1), ones))
+    err, one = ((t[:n].double() - ref).norm().item() for t in (fwd_kvcache_int(q, *args, num_splits=1), ones))
     assert err < 1.1 * (math.sqrt(2) if bits == 2 and deviation == 1.0 else 1.0) * one, (err / ref.norm().item(), one / ref.norm().item())
+
+
+@pytest.mark.parametrize("b,h,h_k,m,S,bits,gs,mode,dtype,ns", [
+    (8, 6, 2, 3, 128 * 130, 4, 128, "k-channel", "fp16", 9),      # 9 pairs: a block of sixteen with seven empty columns
+    (7, 8, 1, 4, 128 * 260, 2, 64, "k-channel", "bf16", 33),      # more splits than a round of the merge takes
+    (16, 5, 5, 32, 128 * 16, 4, 32, "k-channel", "bf16", 1),      # one split
+    (16, 8, 2, 5, 128 * 64, 4, 64, "k-tensor", "fp16", 0),        # 20 pairs
+    (24, 16, 2, 4, 128 * 72, 2, 128, "k-channel", "fp16", 17),
+    (70, 16, 2, 2, 128 * 50, 2, 32, "k-channel", "fp16", 1),      # more sequences than are dealt out by length
+    (9, 16, 2, 7, 128 * 64, 2, 128, "k-channel", "fp16", 0),      # 56 pairs: a last block of eight
+])
+def test_blocks_of_sixteen_with_unequal_lengths(device, b, h, h_k, m, S, bits, gs, mode, dtype, ns):
+    """Calls that do run in blocks of sixteen, each row against a call of its own; bounds as for `test_blocks_of_sixteen_equal_the_calls_for_each_row`."""
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
+    R, tdt, pairs = 53, H.torch_dtype(dtype), m * (h // h_k)
+    assert _blocks(b, h_k, pairs, S, R, bits, gs, True, S + 128, ns) == -(-pairs // 16) < -(-pairs // 8)
+    g = torch.Generator(device=device).manual_seed(m)
+    k, v = (torch.randn((b, S + R, h_k, 128), generator=g, device=device, dtype=tdt) for _ in range(2))
+    k[..., [5, 40, 99]] *= 6
+    v[1] *= 40                                              # residual words
+    q = torch.randn((b, h, m, 128), generator=g, device=device).to(tdt).transpose(1, 2)
+    cache = H.alloc_cache(b, S + 128, h_k, bits, gs, device, k_tensor=mode == "k-tensor")
+    kvcache_pack_int(k[:, :S], cache[0], cache[1], v[:, :S], cache[2], cache[3], None, None, S, mode, gs, bits)
+    lens = torch.tensor([S - 128 * ((5 * i) % 9) for i in range(b)], dtype=torch.int32, device=device)
+    res = torch.full((b,), R, dtype=torch.int32, device=device)
+    lens[2], lens[3], res[3], res[4] = 384, 0, 0, 1
+    args = (*cache, None, SCALE, mode, gs, bits)
+    kw = dict(seqlens_k=lens, max_seqlen_k=S, k_residual=k[:, S:], v_residual=v[:, S:], residual_len=res, return_lse=True)
+    for flip in (1, -1, 1):                                 # launch after launch on one workspace, other queries in between
+        out, lse = fwd_kvcache_int(q * flip, *args, num_splits=ns, **kw)
+    assert torch.isinf(lse[3]).all() and not out[3].any()
+    scale_of = v[:8].float().abs().amax((1, 2, 3)).reshape(-1, 1, 1, 1) / 4
+    for r in sorted({0, 1, m // 2, m - 1}):
+        one, lse1 = fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args, num_splits=min(ns, 4), **kw)
+        err = (out[:8, r:r + 1].float() - one[:8].float()).abs()
+        assert (err <= 1.5e-3 * scale_of[:b] + (2 ** -7 * one[:8].float().abs() if dtype == "bf16" else 0)).all(), (r, err.max().item())
+        ok = lens + res > 0
+        assert (lse[ok, r] - lse1[ok]).abs().max().item() < 5e-4, r

@@ -73,9 +73,10 @@ def test_small_values_keep_their_bits(device, bits, gs, size, rows):
     Bound: a product's pair is off by 2^-24 / sqrt(12), times the code (rms below 9 of 15, 2.2 of 3), p by as much or 2^-12 of itself, over
     the sum L of the p; fp16 rounding of the output; four times the relative error at V of 1 (7e-4 of the norm for p and the
     fp32 sums) covers neither."""
-    from bitladder_amd import _lib, fwd_kvcache_int, kvcache_pack_int
+    from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
+    from tests.test_gpu_rows import _blocks
     S, h_k, g = 128 * 64, 2, 8 // rows
-    b = 1 if rows == 1 else 48
+    b = 1 if rows == 1 else 72
     gen = torch.Generator(device=device).manual_seed(bits + gs)
     q = torch.randn((1, 1, h_k * g, 128), generator=gen, device=device).half()
     k = torch.randn((1, S, h_k, 128), generator=gen, device=device)
@@ -93,7 +94,7 @@ def test_small_values_keep_their_bits(device, bits, gs, size, rows):
         args = (q, *cache)
     else:       # the same sequence often enough for blocks of sixteen pairs, with as many equal rows
         args = (q.expand(b, 2 * rows, -1, -1).contiguous(), *(t.expand(b, *t.shape[1:]).contiguous() for t in cache))
-        assert _lib.lib().bitdecode_row_blocks(b, h_k, 2 * rows * g, S, 256, bits) == 1
+        assert _blocks(b, h_k, 2 * rows * g, S, 0, bits, gs, False, S, 1) == 1      # of sixteen
     out = fwd_kvcache_int(*args, None, scale, "k-channel", gs, bits, num_splits=1)
     rms_code = 9 if bits == 4 else 2.2
     slip = 2 ** -24 / math.sqrt(12) * math.sqrt(S) / p.sum(-1).reshape(-1, 1) * (rms_code + 2 * size)

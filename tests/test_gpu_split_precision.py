@@ -95,9 +95,10 @@ def test_residual_words_in_the_step_and_with_several_rows(device):
 def test_several_rows_lose_no_precision_to_the_split(device, b, S, gs):
     """Sixteen (row, head) pairs of each of 144 or 136 (sequence, kv head) pairs: more blocks of eight than compute units, fewer of
     sixteen.  The error of the library's own split count is that of one split or less, as with one row."""
-    from bitladder_amd import _lib, fwd_kvcache_int
+    from bitladder_amd import fwd_kvcache_int
+    from tests.test_gpu_rows import _blocks
     q, k, v, cache = _setup(device, b, 8, S, 64, gs, b)
-    assert _lib.lib().bitdecode_row_blocks(b, 8, 16, S, 256, 4) == 1
+    assert {_blocks(b, 8, 16, S, 64, 4, gs, False, S, ns) for ns in (0, 1, 2, 3)} == {1}      # of sixteen
     rows = torch.cat([q.roll(j, 0) for j in range(8)], 1)
     seqs = (0, b // 2, b - 1)
     ref = torch.stack([torch.stack([_exact(rows[:, j:j + 1], k, v, S, gs, i) for j in range(8)]) for i in seqs])

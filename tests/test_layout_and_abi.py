@@ -446,3 +446,34 @@ def test_cache_entries_reject_bad_arguments_without_launching():
                                  (lib.bitdecode_cache_prefill, args(d=64), 2, "head_dim")):
         assert entry(ctypes.byref(a), None) == code, (text, lib.bitdecode_last_error())
         assert text in lib.bitdecode_last_error().decode()
+
+
+def _rows(b, h_k, pairs, max_s, bits=4, gs=128, ragged=False, capacity=1 << 20, ns=0, max_r=64):
+    """(split count, blocks per kv head) of a call for several query rows on 256 compute units."""
+    blocks = ctypes.c_int32()
+    n = _lib.lib().bitdecode_rows_splits(b, h_k, pairs, max_s, max_r, 256, bits, gs, ragged, capacity, ns, ctypes.byref(blocks))
+    return n, blocks.value
+
+
+def test_blocks_of_several_query_rows():
+    """Blocks of sixteen pairs where there is work enough for them and workgroups enough to need them."""
+    assert _rows(2, 8, 32, 8192) == (8, 2)
+    assert _rows(2, 8, 8, 8192)[1] == 1 and _rows(1, 8, 32, 4096) == (8, 4)
+    # a caller's split count: up to half the units the workgroups of eight fit the machine side by side
+    assert [_rows(2, 8, 32, 8192, ns=n) for n in (1, 4, 5, 16, 17)] == [(1, 4), (4, 4), (5, 2), (16, 2), (17, 4)]
+    assert _rows(8, 4, 64, 16384, 2, ns=1) == (1, 8) and _rows(8, 4, 64, 16384, 2, ns=2) == (2, 4)
+    # lengths on the device: no doubled split count (one workgroup per unit), not more than 32 units per workgroup without twice as
+    # many splits as blocks of eight have, and more work where the capacity is the only bound
+    assert _rows(16, 8, 16, 4096, ragged=True) == (2, 1) and _lib.lib().bitdecode_num_splits_for(16, 8, 4096, 64, 256, 4, 128, 1) == 4
+    assert _rows(9, 8, 48, 896, ragged=True) == (1, 3)
+    assert _rows(16, 8, 16, 16384, ragged=True) == (2, 1) and _rows(16, 8, 16, 16384, ragged=True, ns=1) == (1, 2) == _rows(16, 8, 16, 16384, ns=1, max_r=513)
+    assert _rows(16, 8, 16, 16384, 2, ragged=True) == (2, 1)
+    assert _rows(2, 8, 32, 8192, ragged=True, capacity=8192)[1] == 4 and _rows(2, 8, 32, 24576, 2, ragged=True, capacity=24576) == (8, 2)
+    # three and five blocks of eight: only where the workgroups fill the units
+    assert _rows(9, 8, 24, 2560, ragged=True) == (2, 3) and _rows(6, 8, 40, 9728, 2) == (1, 5) and _rows(5, 16, 40, 5376) == (1, 3)
+    assert _rows(30, 1, 24, 4864) == (4, 2) and _rows(3, 2, 20, 20608, gs=64) == (14, 3)
+    # never more than a launch's split limit, one split where there is nothing to split, and invalid arguments
+    assert _rows(1, 8, 64, 0) == (1, 8)
+    L = _lib.lib()
+    assert _rows(0, 8, 32, 8192)[0] == _rows(1, 0, 32, 8192)[0] == _rows(1, 8, 0, 8192)[0] == _rows(1, 8, 32, 8192, 3)[0] == _rows(1, 8, 32, 8192, ns=-1)[0] == -1
+    assert L.bitdecode_row_blocks(0, 8, 32, 8192, 256, 4) == L.bitdecode_row_blocks(1, 8, -1, 8192, 256, 4) == L.bitdecode_row_blocks(1, 8, 32, 8192, 256, 3) == -1
