@@ -1726,14 +1726,16 @@ __device__ __forceinline__ void step_end(uint8_t* lds, int bi, int hk, int t) {
 // A permutation of the batch index computed by every wave from the device-side lengths (lane j < n holds that of sequence
 // j; equal lengths are ordered by index), so every workgroup arrives at the same one; the lengths are not
 // written during the launch.  Nothing else depends on it: results are indexed by the sequence.
-__device__ __forceinline__ int sequence_of_position(int len, int n, int p, int lane) {      // n at most 64 (host)
+// (descending: longest first throughout, for the kernels of which a unit holds one workgroup: a unit that is done takes the next.  Blocks of sixteen, 20 to 31
+// sequences in one to three splits 3-8 % over the pairing above; nothing where all workgroups start at once.)
+__device__ __forceinline__ int sequence_of_position(int len, int n, int p, int lane, bool descending) {      // n at most 64 (host)
     int rank = 0;           // sequences that come before this lane's in descending order of length
     for (int j = 0; j < n; ++j) {
         const int lj = __builtin_amdgcn_readlane(len, j);
         rank += (lj > len || (lj == len && j < lane)) ? 1 : 0;
     }
     const int half = (n + 1) >> 1;
-    const int pos = rank < half ? rank : half + (n - 1 - rank);
+    const int pos = descending || rank < half ? rank : half + (n - 1 - rank);
     const unsigned long long hit = __ballot(lane < n && pos == p);
     // (pos is a permutation of 0 .. n-1, so exactly one lane answers; p itself if that were ever not so)
     return __builtin_amdgcn_readfirstlane(hit ? static_cast<int>(__builtin_ctzll(hit)) : p);
@@ -1858,7 +1860,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             int s_dev = sl[j], r_dev = rl[j];
             s_dev = min(max(s_dev, 0), P.capacity);
             r_dev = min(max(r_dev, 0), P.res_cap);
-            if (P.seq_perm) bi = sequence_of_position(s_dev, P.b, bi, lane);
+            if (P.seq_perm) bi = sequence_of_position(s_dev, P.b, bi, lane, WIDE);
             const int src = P.seq_perm ? bi : 0;
             if (P.seqlens) S = __builtin_amdgcn_readlane(s_dev, src);
             if (P.reslens) R = __builtin_amdgcn_readlane(r_dev, src);
