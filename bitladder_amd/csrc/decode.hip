@@ -1749,9 +1749,10 @@ __device__ __forceinline__ int sequence_of_position(int len, int n, int p, int l
 // the wave that draws the last ticket merges all partials of the head
 // (flash_fwd_kernel.h:1217-1298 formula) and resets the ticket.
 //
-// Dynamic LDS: [NW wave regions of UnitCfg::REGION bytes][q: 8 head rows, 288 B apart][zeros]
-// [sM, sL: per-wave max and sum, 8 heads x NW floats each][append flag][tickets and slots of the 8 heads].  A wave's region is reused as its
-// V-transpose slab for fp16 tiles and as its slot of the cross-wave merge buffer (g x 128 floats <= 4 KB).
+// Dynamic LDS, for the C = 8 heads (or pairs) of a workgroup, 16 pairs where WIDE:
+// [NW wave regions of UnitCfg::REGION bytes][q: C rows, 288 B apart][zeros; not where WIDE]
+// [sM, sL: per-wave max and sum, C x NW floats each][append flag][tickets and slots, C each].  A wave's region is reused as its
+// V-transpose slab for fp16 tiles and as its slot of the cross-wave merge buffer (g x 128 floats: up to 4 KB, WIDE 8 KB).
 // ---------------------------------------------------------------------------------------------
 template <int BITS, int GS, bool FEW, bool WIDE>
 constexpr int fwd_lds_bytes() {
@@ -1778,7 +1779,7 @@ __global__ __launch_bounds__((UnitCfg<BITS, GS, FEW>::NW * 64), (FEW && !(KT && 
 void fwd_splitkv_kernel(FwdParams P) {
     constexpr bool ROWS = ROWS_KIND != kRowsNone, WIDE = ROWS_KIND == kRowsWide;
     constexpr int kCols = WIDE ? kWidePairs : kMaxGroupHeads;      // heads or pairs of a workgroup
-    static_assert(!WIDE || (FEW && !APPEND && kWidePairs * kHeadDim * 4 <= 8192), "8 waves; a wave's slot of the merge in its region");
+    static_assert(!WIDE || (FEW && !APPEND), "blocks of sixteen: 8 waves, no step with append");
     static_assert(!KT || BITS == 4, "per-token K parameters: 4 bits");
     // The decode step with append has more parameter fields than scalar registers, and the per-token-K kernels
     // have no vector register to spare for scalar spills: they fetch what only the window and the tail need from
@@ -1805,6 +1806,8 @@ void fwd_splitkv_kernel(FwdParams P) {
     constexpr int NCG = C::NCG, NW = C::NW, REGION = C::REGION;
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     static_assert(sizeof(qp::PackLds<GS>) <= NW * REGION, "the pack tile reuses the wave regions");
+    static_assert(kCols * kHeadDim * 4 <= REGION, "a wave's slot of the merge is its region");
+    static_assert(16 * kLdsRowHalves * 2 <= REGION, "and so is its V-transpose slab");
     uint8_t* const sq = lds + NW * REGION;                                   // [8][128] 16-bit q, zeros
     float* const sM = reinterpret_cast<float*>(sq + q_bytes(WIDE));   // [kCols][NW]
     float* const sL = sM + NW * kCols;
