@@ -220,11 +220,14 @@ struct RowsCall {
 // W is larger:
 //   1 x 64K, 8 / 1, 8 rows    W 32:  17.7 | 18.6   21.0 | 19.9   16.7 | 17.9       1 x 128K, 8 / 1  W 64:  31.2 | 24.0   37.0 | 27.1  22.8 | 21.1 (g64 23.7 | 24.9)
 //   2 x 25K, 12 / 4, 4 rows   W 25:  13.3 | 14.3 (31 splits)                          1 x 33K, 16 / 8, 8 rows  W 32, 2 bits: 14.3 | 14.9 (29)
+// (2 bits g128 before its blocks of sixteen summed the lo parts apart, 5-9 % of their time, decode.hip: lo_sums.  Since then, with 16 splits
+// and more: 1 x 14K, 8 rows W 28 13.0 | 13.7, 1 x 16K W 32 and 1 x 18K W 36 13.2 | 13.2 and 14.2 | 14.2, 1 x 20K W 40 14.7 | 14.3; with fewer: 7 x 4K and 16 x 1.75K, 4
+// rows W 28 13.2 | 12.3 and 13.6 | 12.2, 2 x 8K, 8 rows W 32 13.0 | 13.0.)
 bool rows_work(const RowsCall& c) {
     if (c.pairs <= bitdecode::kMaxGroupHeads) return false;
     const bool many_splits = c.triples() * 32 <= c.cus;
     if (many_splits && c.bits == 2) return false;
-    int from = many_splits ? 48 : c.bits == 4 ? 20 : 28;
+    int from = many_splits ? 48 : c.bits == 4 ? 20 : c.gs == 128 && c.triples() * 16 <= c.cus ? 32 : 28;
     // (lengths of an eighth to a quarter of the capacity, the only bound: W by the bound 60 9.4 | 11.8, 66 9.6 | 10.9, 83 12.5 | 11.7 and 15.8 | 19.9, 98
     // 20.0 | 11.6, 115 17.1 | 11.4, 139 17.9 | 11.0)
     if (c.open) from = std::max(from, 96);

@@ -230,14 +230,15 @@ constexpr float kNoScore = -1e30f;
 
 // Blocks of sixteen pairs (WIDE) leave the lo parts of the split products no columns of their own, and run with 8 waves where 2-bit
 // blocks of eight have 16.  Every addition to sums that hold the code offsets rounds at their magnitude, so more of them per sum cost
-// accuracy.  At 4 bits the lo parts have sums of their own; at 2 bits the even and the odd steps of 64 tokens have a state each, as if of
-// two waves (their own maximum too: a wave's largest score decides what its small products keep).  Error against 64 bits of the
-// norm, one split of 8K tokens, blocks of eight | of sixteen with all in one set of sums | as it is: 4 bits g128 1.12e-3 | 1.17e-3 | 9.2e-4; 2 bits g64
-// 1.70e-3 | 2.39e-3 | 1.39e-3, g128 over 16K tokens 2.69e-3 | 4.94e-3 | 2.71e-3, g64 with V of 0.003 and scores of deviation 3 8.0e-4 | 1.07e-3 | 6.8e-4.  It takes 1-4 % (decode of 8 rows, 32 / 8
-// heads, 2 x 8K tokens at 4 bits 12.6 -> 13.0 us).
-constexpr bool lo_sums(int bits, bool wide) { return wide && bits == 4; }
+// accuracy.  The lo parts have sums of their own, but for 2 bits at g64 and g32, whose blocks of eight have 12 and 8 waves.  At 2 bits the even and
+// the odd steps of 64 tokens have a state each, as if of two waves (their own maximum too: a wave's largest score decides what its small
+// products keep).  Error against 64 bits of the norm, blocks of eight | of sixteen with all in one set of sums | as it is, one split: 8K tokens
+// 4 bits g128 1.15e-3 | 1.17e-3 | 9.4e-4, 2 bits g64 1.74e-3 | 2.39e-3 | 1.43e-3, g128 1.43e-3 | - | 1.10e-3 (two states without sums for the lo
+// parts 1.48e-3, over 2K tokens 4.5e-4 | - | 3.7e-4 and 5.4e-4).  It takes 1-4 % (8 rows of 32 / 8 heads over 2 x 8K tokens at 4 bits 12.6 -> 13.0 us), at
+// 2 bits g128 5-9 % more (10 x 8K 37.2 -> 39.2 us, blocks of eight 60.6).
+constexpr bool lo_sums(int bits, int gs, bool wide) { return wide && (bits == 4 || gs == 128); }
 
-// LO: accumulators of their own for the lo parts where those have no columns of their own (WIDE, 4 bits)
+// LO: accumulators of their own for the lo parts (lo_sums)
 template <int NCG, bool LO>
 struct WaveState {
     float m;          // running max of the raw scores (q.k units) of this lane's head (kNoScore: none yet)
@@ -249,7 +250,10 @@ struct WaveState {
     f4 zb;
     f4 ob[NCG];       // offset part of the V bias per channel group, hi and lo
     f4 o[8];          // O^T tiles: lane (head, q) holds channels 16*ct + 4*q + r
-    f4 ob_lo[LO ? NCG : 1], o_lo[LO ? 8 : 1];
+    // (the lo parts' offset bias goes into zb where that is one group's: sums of the size of the signal, unlike those in ob.  An array
+    // of its own cost the 2-bit kernels, two states at 255 registers, spills.)
+    static constexpr bool kOwnLoBias = LO && NCG > 1;
+    f4 ob_lo[kOwnLoBias ? NCG : 1], o_lo[LO ? 8 : 1];
 
     __device__ __forceinline__ WaveState() {
         m = kNoScore;
@@ -258,9 +262,11 @@ struct WaveState {
         for (int c = 0; c < NCG; ++c) ob[c] = f4{0, 0, 0, 0};
 #pragma unroll
         for (int ct = 0; ct < 8; ++ct) o[ct] = f4{0, 0, 0, 0};
-        if constexpr (LO) {
+        if constexpr (kOwnLoBias) {
 #pragma unroll
             for (int c = 0; c < NCG; ++c) ob_lo[c] = f4{0, 0, 0, 0};
+        }
+        if constexpr (LO) {
 #pragma unroll
             for (int ct = 0; ct < 8; ++ct) o_lo[ct] = f4{0, 0, 0, 0};
         }
@@ -274,25 +280,35 @@ struct WaveState {
         for (int c = 0; c < NCG; ++c) ob[c][0] *= alpha;
 #pragma unroll
         for (int ct = 0; ct < 8; ++ct) o[ct] *= alpha;
-        if constexpr (LO) {
+        if constexpr (kOwnLoBias) {
 #pragma unroll
             for (int c = 0; c < NCG; ++c) ob_lo[c][0] *= alpha;
+        }
+        if constexpr (LO) {
 #pragma unroll
             for (int ct = 0; ct < 8; ++ct) o_lo[ct] *= alpha;
         }
     }
-    // takes in what another state of the wave has accumulated
+    // takes in what another state of the wave has accumulated.  With sums of the lo parts' own the V biases are added to the outputs
+    // first: the rescale and the addition round at the size of what they are given, which few steps per state do not hide.
     __device__ __forceinline__ void join(WaveState& x, float scale) {
-        const float m_new = fmaxf(m, x.m);
-        rescale(__builtin_amdgcn_exp2f((m - m_new) * scale));
-        x.rescale(__builtin_amdgcn_exp2f((x.m - m_new) * scale));
+        static_assert(!kOwnLoBias, "lo biases in zb or ob");
+        const float m_new = fmaxf(m, x.m), a = __builtin_amdgcn_exp2f((m - m_new) * scale), b = __builtin_amdgcn_exp2f((x.m - m_new) * scale);
         m = m_new;
-        l += x.l;
-        zb += x.zb;
+        if constexpr (LO) {
+            l = l * a + x.l * b;
 #pragma unroll
-        for (int c = 0; c < NCG; ++c) ob[c] += x.ob[c];
+            for (int ct = 0; ct < 8; ++ct) o[ct] = (o[ct] + ob[0][0] + (o_lo[ct] + zb[0])) * a + (x.o[ct] + x.ob[0][0] + (x.o_lo[ct] + x.zb[0])) * b;
+        } else {
+            rescale(a);
+            x.rescale(b);
+            l += x.l;
+            zb += x.zb;
 #pragma unroll
-        for (int ct = 0; ct < 8; ++ct) o[ct] += x.o[ct];
+            for (int c = 0; c < NCG; ++c) ob[c] += x.ob[c];
+#pragma unroll
+            for (int ct = 0; ct < 8; ++ct) o[ct] += x.o[ct];
+        }
     }
 };
 
@@ -812,8 +828,8 @@ template <int BITS, int GS, bool BF16, bool HAS_NEXT, bool KT, bool FEW, bool WI
 __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region_lds, int kslot,
                                              const UnitAddr<BITS, GS>& cur, const UnitAddr<BITS, GS>& next,
                                              const QRows& Q, const FwdParams& P, int lane, bool lo_part, const Magic& mg,
-                                             WaveState<kHeadDim / GS, lo_sums(BITS, WIDE)>& st_even,
-                                             WaveState<kHeadDim / GS, lo_sums(BITS, WIDE)>& st_odd, const TokenQ<kHeadDim / GS>* KQ = nullptr) {
+                                             WaveState<kHeadDim / GS, lo_sums(BITS, GS, WIDE)>& st_even,
+                                             WaveState<kHeadDim / GS, lo_sums(BITS, GS, WIDE)>& st_odd, const TokenQ<kHeadDim / GS>* KQ = nullptr) {
     using C = UnitCfg<BITS, GS>;
     constexpr int NCG = C::NCG, TPS = C::TPS, NKS = C::NKS, TPG = C::TPG, CTPG = GS / 16;
     constexpr int NSTEP = C::NSTEP, RPS = C::RPS, TPR = TPS / RPS;      // tiles per K row
@@ -823,7 +839,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
     const h8 ones = h8{1, 1, 1, 1, 1, 1, 1, 1};
     const uint32_t hi_cols = lo_part ? 0u : 0xffffffffu;
     const u4* kcode = reinterpret_cast<const u4*>(reg) + lane;             // row r: kcode[64 * r]
-    constexpr bool LO = lo_sums(BITS, WIDE);
+    constexpr bool LO = lo_sums(BITS, GS, WIDE);
     const u4* vcode = reinterpret_cast<const u4*>(reg + 4096) + lane;
     const uint8_t* kpar = reg + C::OFF_KP + kslot * C::KPB;
     const uint8_t* vpar = reg + C::OFF_VP + kg * 16;
@@ -910,7 +926,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
         static_assert(TPS == 4 && NKS == 2, "four tiles, two sub-blocks per step");
         h8 p16[NKS], pm[NKS];
         if constexpr (WIDE) {
-            step_probabilities_wide<BITS, NCG, lo_sums(BITS, WIDE)>(sc, P.scale_log2, st, p16);
+            step_probabilities_wide<BITS, NCG, lo_sums(BITS, GS, WIDE)>(sc, P.scale_log2, st, p16);
         } else {
             step_probabilities<BITS, NCG>(sc, hi_cols, P.scale_log2, st, p16, pm);
         }
@@ -951,7 +967,7 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                         }
                         st.ob[cg] = mfma32(noff, pp[cg][ks], st.ob[cg]);
                         if constexpr (WIDE) {
-                            f4& ob_lo = LO ? st.ob_lo[LO ? cg : 0] : st.ob[cg];
+                            f4& ob_lo = st.kOwnLoBias ? st.ob_lo[st.kOwnLoBias ? cg : 0] : LO ? st.zb : st.ob[cg];
                             ob_lo = mfma32(noff, pp_lo[cg][ks], ob_lo);
                         }
                     }
@@ -976,8 +992,9 @@ __device__ __forceinline__ void compute_unit(const uint8_t* reg, uint32_t region
                     st.o[ct] = mfma32(a0, pp[cg][0], st.o[ct]);
                     st.o[ct] = mfma32(a1, pp[cg][1], st.o[ct]);
                     if constexpr (WIDE) {
-                        st.o[ct] = mfma32(a0, pp_lo[cg][0], st.o[ct]);
-                        st.o[ct] = mfma32(a1, pp_lo[cg][1], st.o[ct]);
+                        f4& o_lo = LO ? st.o_lo[LO ? ct : 0] : st.o[ct];
+                        o_lo = mfma32(a0, pp_lo[cg][0], o_lo);
+                        o_lo = mfma32(a1, pp_lo[cg][1], o_lo);
                     }
                 }
             }
@@ -1983,7 +2000,7 @@ void fwd_splitkv_kernel(FwdParams P) {
     const QRows Q = q_rows(sq, head, kg, lo_part);
     PROF(1);
 
-    constexpr bool kLoSums = lo_sums(BITS, WIDE);
+    constexpr bool kLoSums = lo_sums(BITS, GS, WIDE), kTwoStates = WIDE && BITS == 2;
     WaveState<NCG, kLoSums> st;
 
     // ---- packed units of this wave
@@ -2008,7 +2025,7 @@ void fwd_splitkv_kernel(FwdParams P) {
             kslot ^= 1;
         }
         compute_unit<BITS, GS, BF16, false, KT, FEW, WIDE>(region, region_lds, kslot, A, A, Q, P, lane, lo_part, mg, st, WIDE ? st_odd : st, KQp);
-        if constexpr (WIDE && !kLoSums) st.join(st_odd, P.scale_log2);
+        if constexpr (kTwoStates) st.join(st_odd, P.scale_log2);
     }
     PROF(3);
     // ---- fp16 window tiles of this wave (the region becomes the V-transpose slab)
@@ -2070,8 +2087,9 @@ void fwd_splitkv_kernel(FwdParams P) {
     for (int ct = 0; ct < 8; ++ct) {
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            float v = st.o[ct][r] + bias[ct / (GS / 16)];
-            if constexpr (kLoSums) v += st.o_lo[ct][r] + st.ob_lo[ct / (GS / 16)][0];
+            float v = st.o[ct][r];
+            if constexpr (!(kTwoStates && kLoSums)) v += bias[ct / (GS / 16)];      // (added when they were joined)
+            if constexpr (!kTwoStates && kLoSums) v += st.o_lo[ct][r] + (st.kOwnLoBias ? st.ob_lo[st.kOwnLoBias ? ct / (GS / 16) : 0][0] : 0.0f);
             st.o[ct][r] = WIDE ? v : v + partner(v);      // hi + lo
         }
     }

@@ -234,16 +234,16 @@ def test_splits_without_work_have_some_in_the_next_launch(device, bits, gs, mode
                 assert (plan.lse[some, r] - lse1[some]).abs().max().item() < 5e-4
 
 
+@pytest.mark.parametrize("b,h,m,S", [(10, 32, 8, 8192), (32, 8, 16, 2048)])
 @pytest.mark.parametrize("bits,gs", [(4, 128), (4, 32), (2, 128), (2, 64)])
 @pytest.mark.parametrize("size,deviation", [(1.0, 1.0), (1.0, 3.0), (0.003, 3.0)])
-def test_blocks_of_sixteen_are_as_accurate_as_calls_for_each_row(device, bits, gs, size, deviation):
-    """Error against 64 bits over one split of 8K tokens, many fp32 additions per sum: no more than calls with one row have, whose
-    hi and lo parts are summed apart by 16 (2 bits) or 8 waves; 10 % for the order of the sums, over 64K outputs.  Where the roundings of
-    the sums make up the error (scores of deviation 1), 2 bits have sqrt(2) of it: sums as many, but the lo parts in them."""
+def test_blocks_of_sixteen_are_as_accurate_as_calls_for_each_row(device, bits, gs, size, deviation, b, h, m, S):
+    """Error against 64 bits over one split, many fp32 additions per sum: no more than calls with one row have, whose
+    hi and lo parts are summed apart by 16 (2 bits; 12 at group 64) or 8 waves; 10 % for the order of the sums, over 32K outputs and more."""
     from bitladder_amd import fwd_kvcache_int, kvcache_pack_int
     from oracle import torch_oracle as T
-    b, h, h_k, m, S, n = 10, 32, 8, 8, 8192, 2
-    assert _blocks(b, h_k, m * (h // h_k), S, 0, bits, gs, False, S, 1) == 2      # of sixteen
+    h_k, n = 8, 2
+    assert _blocks(b, h_k, m * (h // h_k), S, 0, bits, gs, False, S, 1) == m * (h // h_k) // 16      # of sixteen
     g = torch.Generator(device=device).manual_seed(bits + gs)
     q = torch.randn((b, m, h, 128), generator=g, device=device).half()
     k, v = (torch.randn((b, S, h_k, 128), generator=g, device=device) for _ in range(2))
@@ -261,7 +261,7 @@ def test_blocks_of_sixteen_are_as_accurate_as_calls_for_each_row(device, bits, g
     args = (*cache, None, scale, "k-channel", gs, bits)
     ones = torch.cat([fwd_kvcache_int(q[:, r:r + 1].contiguous(), *args, num_splits=1) for r in range(m)], 1)
     err, one = ((t[:n].double() - ref).norm().item() for t in (fwd_kvcache_int(q, *args, num_splits=1), ones))
-    assert err < 1.1 * (math.sqrt(2) if bits == 2 and deviation == 1.0 else 1.0) * one, (err / ref.norm().item(), one / ref.norm().item())
+    assert err < 1.1 * one, (err / ref.norm().item(), one / ref.norm().item())
 
 
 @pytest.mark.parametrize("b,h,h_k,m,S,bits,gs,mode,dtype,ns", [

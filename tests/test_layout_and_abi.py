@@ -472,6 +472,9 @@ def test_blocks_of_several_query_rows():
     # three and five blocks of eight: only where the workgroups fill the units
     assert _rows(9, 8, 24, 2560, ragged=True) == (2, 3) and _rows(6, 8, 40, 9728, 2) == (1, 5) and _rows(5, 16, 40, 5376) == (1, 3)
     assert _rows(30, 1, 24, 4864) == (4, 2) and _rows(3, 2, 20, 20608, gs=64) == (14, 3)
+    # 2 bits at group 128, whose blocks of sixteen take longer: where 16 splits are needed, with more work
+    assert _rows(1, 8, 32, 14336, 2) == (8, 4) and _rows(1, 8, 32, 14336, 2, 64)[1] == 2 and _rows(1, 8, 32, 16384, 2) == (16, 2)
+    assert _rows(16, 8, 16, 1792, 2) == (2, 1) and _rows(7, 8, 16, 4096, 2)[1] == 1
     # never more than a launch's split limit, one split where there is nothing to split, and invalid arguments
     assert _rows(1, 8, 64, 0) == (1, 8)
     L = _lib.lib()
