@@ -1655,7 +1655,7 @@ __device__ __forceinline__ void wide_tail(const FwdParams& P, const uint8_t* lds
 // The length is stable for every workgroup that reads it: it is advanced only after all workgroups of
 // the sequence have drawn their tickets.
 // (read through `seqlens`, which holds the same pointer in a step: the field comes with the first kernel arguments, `lengths`
-// behind them cost a round of loads of its own, 0.2 us a step)
+// behind them cost a round of loads of its own)
 __device__ __forceinline__ int step_length(const FwdParams& P, int bi) { return P.seqlens[bi]; }
 // A sequence whose window is about to fill while its cache has no room for another chunk cannot
 // take the token: it is attended, but neither stored nor counted.
@@ -1787,7 +1787,7 @@ constexpr int fwd_lds_bytes() {
 // rows, tickets and the merge go by the pair's number.  The workgroups of a kv head's blocks read the same codes; where the
 // grid is remapped (several splits, a multiple of eight pairs) they are neighbours on one XCD, and all but the first find them in
 // its L2; otherwise they are dealt to all XCDs.  Eight rows of 32 / 8 heads over 2 x 8K tokens: 112 us with the rows
-// folded into the head dimension on the host (four launches), 14.5 in blocks of eight, 11.9 in blocks of sixteen.
+// folded into the head dimension on the host (four launches), 15.3 in blocks of eight, 12.8 in blocks of sixteen.
 template <int BITS, int GS, bool BF16, bool APPEND, bool KT, bool FEW, int ROWS_KIND>
 // (second bound: waves per SIMD the register count has to leave room for.  Two workgroups of the 8-wave kernels share
 // a compute unit when sequences differ in length, 4 waves per SIMD like the 16-wave kernels: 128 registers.  The
